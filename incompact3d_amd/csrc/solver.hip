@@ -315,14 +315,14 @@ int gradp_correct(const Context &c, x3d_solver *S, T *const u[3], T *const W[5],
   return X3D_OK;
 }
 
-// The six y/z momentum sweeps of step_once (no SGS force), nrep times, into
-// the work buffer W[0]; *bytes = algorithmic bytes per launch on average.
+// The six y/z momentum sweeps of step_once (no SGS force; one launch per
+// direction), nrep times, into the work buffers W[0..2]; *bytes = algorithmic
+// bytes per sweep on average.
 template <typename T>
 int momentum_yz(Context &c, x3d_solver *S, int nrep, double *bytes) {
   const int nx = S->nx, ny = S->ny, nz = S->nz;
   const T *cu[3];
   for (int i = 0; i < 3; ++i) cu[i] = sizeof(T) == 8 ? (const T *)S->u64[i] : (const T *)S->u32[i];
-  T *W0 = (T *)S->w[0];
   double fields = 0;
   for (int comp = 0; comp < 3; ++comp) {
     fields += (comp == 2 ? 1 : 2) + 1;        // z: u_z (and u_c), out
@@ -330,13 +330,15 @@ int momentum_yz(Context &c, x3d_solver *S, int nrep, double *bytes) {
   }
   *bytes = fields / 6.0 * (double)S->n * sizeof(T);
   S->have_pressure = false;   // the probe writes W[0]
+  MomIO<T> z, y;
+  for (int i = 0; i < 3; ++i) {
+    z.u[i] = y.u[i] = cu[i];
+    z.out[i] = y.out[i] = (T *)S->w[i];
+    y.acc[i] = (const T *)S->w[i];
+  }
   for (int r = 0; r < nrep; ++r) {
-    for (int comp = 0; comp < 3; ++comp) {
-      X3D_TRY(launch_momentum<T>(c, 2, comp, cu, nullptr, W0, nullptr, nullptr, nullptr, nullptr, nullptr, 0, 0, 0,
-                                 0, nx, ny, nz, c.stream));
-      X3D_TRY(launch_momentum<T>(c, 1, comp, cu, W0, W0, nullptr, nullptr, nullptr, nullptr, nullptr, 0, 0, 0, 0,
-                                 nx, ny, nz, c.stream));
-    }
+    X3D_TRY(launch_momentum<T>(c, 2, z, nx, ny, nz, c.stream));
+    X3D_TRY(launch_momentum<T>(c, 1, y, nx, ny, nz, c.stream));
   }
   return X3D_OK;
 }
@@ -465,23 +467,28 @@ int step_once(Context &c, x3d_solver *S) {
     X3D_TRY(compute_sgs<T>(c, S, cu, sgs));
   }
   if (S->fused) {
-    for (int comp = 0; comp < 3; ++comp) {
-      T *f1 = (T *)S->hist[comp][S->slot[0]];
-      const T *f2 = (T *)S->hist[comp][S->slot[1]];
-      const T *f3 = (T *)S->hist[comp][S->slot[2]];
-      X3D_TRY(launch_momentum<T>(c, 2, comp, cu, sgs[comp], W[0], nullptr, nullptr, nullptr, nullptr, nullptr, 0, 0,
-                                 0, 0, nx, ny, nz, c.stream));
-      X3D_TRY(launch_momentum<T>(c, 1, comp, cu, W[0], W[0], nullptr, nullptr, nullptr, nullptr, nullptr, 0, 0, 0,
-                                 0, nx, ny, nz, c.stream));
+    MomIO<T> z, y, x;
+    for (int i = 0; i < 3; ++i) {
+      z.u[i] = y.u[i] = x.u[i] = cu[i];
+      z.acc[i] = sgs[i];
+      z.out[i] = y.out[i] = W[i];
+      y.acc[i] = x.acc[i] = W[i];
+      x.out[i] = (T *)S->hist[i][S->slot[0]];
+      x.f2[i] = (const T *)S->hist[i][S->slot[1]];
+      x.f3[i] = (const T *)S->hist[i][S->slot[2]];
       // FP64: the new velocity into u64b; FP32: the increment into u64b (as
       // FP32) and the new FP32 velocity into u32b, u64 updated by GRAD_X
-      if constexpr (sizeof(T) == 8)
-        X3D_TRY(launch_momentum<T>(c, 0, comp, cu, W[0], f1, f2, f3, S->u64b[comp], nullptr, nullptr, a, b, cc,
-                                   nterms, nx, ny, nz, c.stream));
-      else
-        X3D_TRY(launch_momentum<T>(c, 0, comp, cu, W[0], f1, f2, f3, nullptr, (float *)S->u64b[comp],
-                                   S->u32b[comp], a, b, cc, nterms, nx, ny, nz, c.stream));
+      if constexpr (sizeof(T) == 8) {
+        x.u_new[i] = S->u64b[i];
+      } else {
+        x.delta[i] = (float *)S->u64b[i];
+        x.shadow[i] = S->u32b[i];
+      }
     }
+    x.ca = a; x.cb = b; x.cc = cc; x.nterms = nterms;
+    X3D_TRY(launch_momentum<T>(c, 2, z, nx, ny, nz, c.stream));
+    X3D_TRY(launch_momentum<T>(c, 1, y, nx, ny, nz, c.stream));
+    X3D_TRY(launch_momentum<T>(c, 0, x, nx, ny, nz, c.stream));
     for (int i = 0; i < 3; ++i) {
       if (sizeof(T) == 8) std::swap(S->u64[i], S->u64b[i]);
       else std::swap(S->u32[i], S->u32b[i]);

@@ -191,16 +191,25 @@ constexpr size_t POISSON_SCRATCH_BYTES = (size_t)160 << 20;
 void *poisson_scratch(int device);
 
 // ---------------------------------------------------------------- fused sweeps
-// momentum.hip: the transeq right-hand side of component comp along dir
-// (out = acc + ...); the x sweep also applies AB3 (nterms > 0): FP64 compute
-// writes the new velocity to u_new; FP32 compute writes the FP32 increment
-// to delta and the new FP32 velocity to shadow, and the FP64 velocity takes
-// the increment in the gradient correction.
+// momentum.hip: the transeq right-hand side of all three components along
+// dir (out = acc + ...); the x sweep also applies AB3 (nterms > 0): FP64
+// compute writes the new velocity to u_new; FP32 compute writes the FP32
+// increment to delta and the new FP32 velocity to shadow, and the FP64
+// velocity takes the increment in the gradient correction.  acc[i] may be
+// out[i] or null.
+template <typename T>
+struct MomIO {
+  const T *u[3] = {}, *acc[3] = {};
+  T *out[3] = {};
+  const T *f2[3] = {}, *f3[3] = {};
+  double *u_new[3] = {};
+  float *delta[3] = {}, *shadow[3] = {};
+  double ca = 0, cb = 0, cc = 0;
+  int nterms = 0;
+};
 bool momentum_fusable(const Context &c);
 template <typename T>
-int launch_momentum(const Context &c, int dir, int comp, const T *const u[3], const T *acc, T *out,
-                    const T *f2, const T *f3, double *u_new, float *delta, float *shadow, double ca,
-                    double cb, double cc, int nterms, int nx, int ny, int nz, hipStream_t st);
+int launch_momentum(const Context &c, int dir, const MomIO<T> &io, int nx, int ny, int nz, hipStream_t st);
 
 // projection.hip: divergence (x, y, z) and gradient + cor_vel (z, y, x)
 enum { SW_DIV_X = 0, SW_DIV_Y, SW_DIV_Z, SW_GRAD_Z, SW_GRAD_Y, SW_GRAD_X };
