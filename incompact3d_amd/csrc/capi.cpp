@@ -263,8 +263,10 @@ int x3d_init(const x3d_params *p) {
   X3D_TRY(build_schemes(*c));
   X3D_TRY(upload_sets(*c));
   {
-    int r = build_stretching(*c);
+    int r = bounded_setup(*c);
+    if (r == X3D_OK) r = build_stretching(*c);
     if (r != X3D_OK) {
+      bounded_free(*c);
       free_stretching(*c);
       free_sets(*c);
       return r;
@@ -276,6 +278,7 @@ int x3d_init(const x3d_params *p) {
   {
     int r = poisson_setup(*c);
     if (r != X3D_OK && r != X3D_ERR_UNSUPPORTED) {
+      bounded_free(*c);
       free_stretching(*c);
       free_sets(*c);
       return r;
@@ -290,6 +293,7 @@ int x3d_finalize(void) {
   if (!g_ctx) return X3D_OK;
   (void)hipDeviceSynchronize();
   poisson_free(*g_ctx);
+  bounded_free(*g_ctx);
   free_stretching(*g_ctx);
   free_sets(*g_ctx);
   for (TriSet &f : g_foreign) {

@@ -66,7 +66,7 @@ template <> struct Halo<OP_INTERPV> { static constexpr int L = 4, R = 3; };
 // (the direct four-term form needs fewer registers where a kernel is at its
 // register budget).
 template <int OP, typename T, int W, bool D2S = true>
-__device__ __forceinline__ T interior_row(const T (&v)[W], const int k, const Sten<T> &s) {
+__host__ __device__ __forceinline__ T interior_row(const T (&v)[W], const int k, const Sten<T> &s) {
   if constexpr (OP == OP_DER1) {
     // derive.f90:34-36
     return s.afi * (v[k + 1] - v[k - 1]) + s.bfi * (v[k + 2] - v[k - 2]);
@@ -106,7 +106,7 @@ __device__ __forceinline__ T interior_row(const T (&v)[W], const int k, const St
 
 // Rows of a non-periodic line that use a boundary closure (<= 4 per end).
 template <int OP>
-__device__ __forceinline__ bool is_boundary_row(int i, int n_out) {
+__host__ __device__ __forceinline__ bool is_boundary_row(int i, int n_out) {
   if constexpr (OP == OP_DER1) return i < 2 || i >= n_out - 2;
   else if constexpr (OP == OP_DER2) return i < 4 || i >= n_out - 4;
   else if constexpr (OP == OP_DERVP) return i == 0 || i == n_out - 1;
@@ -116,13 +116,13 @@ __device__ __forceinline__ bool is_boundary_row(int i, int n_out) {
 }
 
 template <typename T>
-__device__ __forceinline__ T d2t(T a, T up, T u0, T um) {
+__host__ __device__ __forceinline__ T d2t(T a, T up, T u0, T um) {
   return a * (up - u0 - u0 + um);
 }
 
 // Boundary closures, written row by row after the reference.
 template <int OP, typename T, typename LD>
-__device__ T boundary_row(int i, int n_in, int n_out, const Sten<T> &s, int bc1, int bcn, int npaire,
+__host__ __device__ T boundary_row(int i, int n_in, int n_out, const Sten<T> &s, int bc1, int bcn, int npaire,
                           LD U) {
   if constexpr (OP == OP_DER1) {
     // derx_11 derive.f90:88-130, derx_12 :161-200, derx_21 :231-270, derx_22 :299-306

@@ -1,4 +1,5 @@
-// Fused momentum right-hand side of transeq.f90:73-470 for a periodic box.
+// Fused momentum right-hand side of transeq.f90:73-470 along periodic
+// directions (bounded.hip holds the sweeps along bounded ones).
 //
 // One launch per sweep direction d computes for each velocity component c
 // the three compact solves the reference does for that pair
@@ -21,7 +22,7 @@
 #include <cmath>
 #include <vector>
 
-#include "lines_impl.h"
+#include "bounded_impl.h"
 
 namespace x3d {
 
@@ -49,6 +50,7 @@ struct MomArgs {
   float *shadow[3];
   double ca, cb, cc;
   int nterms;                   // 0: no AB3
+  MomUpdate<T> up;              // x sweep of the general step
 };
 
 // ---------------------------------------------------------------- y / z sweeps
@@ -190,7 +192,8 @@ __device__ __forceinline__ void mom_line(const MomArgs<T> &A, const LineCoef<T, 
 }
 
 // ---------------------------------------------------------------- x sweep (one wavefront per line)
-template <typename T, int V>
+// GEN: the general velocity update (RK3, bounded y or z) in place of plain AB3.
+template <typename T, int V, bool GEN>
 __global__ void __launch_bounds__(256) mom_x_kernel(const MomArgs<T> A, int nlines) {
   const int lane = threadIdx.x & 63;
   const int wave = (blockIdx.x * blockDim.x + threadIdx.x) >> 6;
@@ -223,6 +226,32 @@ __global__ void __launch_bounds__(256) mom_x_kernel(const MomArgs<T> A, int nlin
     // every epilogue input is read before the first store (the compiler
     // cannot move loads above stores to possibly aliasing arrays)
     T acc[V], f2[V], f3[V];
+    if constexpr (GEN) {
+      const MomUpdate<T> &U = A.up;
+      T rot[V];
+      double un[V];
+      load_run<T, V>(acc_in + base, acc);
+      if (U.nterms >= 2) load_run<T, V>(U.f2[comp] + base, f2);
+      if (U.nterms >= 3) load_run<T, V>(U.f3[comp] + base, f3);
+      if (U.rot[comp]) load_run<T, V>(U.rot[comp] + base, rot);
+      if constexpr (sizeof(T) == 4) load_run<double, V>(U.u64[comp] + base, un);
+      const int lu = __builtin_amdgcn_readfirstlane(ln), k = lu / U.ny, j = lu - k * U.ny;
+#pragma unroll
+      for (int m = 0; m < V; ++m) {
+        r[m] = mom_forced(U, comp, acc[m] + r[m], rot[m]);
+        const double uo = sizeof(T) == 8 ? (double)uc[m] : un[m];
+        un[m] = pre_correc_point(U, comp, e0 + m, j, k, mom_increment(U, r[m], f2[m], f3[m]) + uo);
+      }
+      store_run<T, V>(A.out[comp] + base, r);
+      store_run<double, V>(U.u64[comp] + base, un);
+      if constexpr (sizeof(T) == 4) {
+        float sh[V];
+#pragma unroll
+        for (int m = 0; m < V; ++m) sh[m] = (float)un[m];
+        store_run<float, V>(U.u32[comp] + base, sh);
+      }
+      continue;
+    }
     if (acc_in) load_run<T, V>(acc_in + base, acc);
     if (A.nterms >= 2) load_run<T, V>(f2_in + base, f2);
     if (A.nterms >= 3) load_run<T, V>(f3_in + base, f3);
@@ -262,7 +291,8 @@ __global__ void __launch_bounds__(256) mom_x_kernel(const MomArgs<T> A, int nlin
 
 // ---------------------------------------------------------------- host side
 
-// The fused sweeps cover periodic lines with nx = 64, 128, 256 or 512 (one
+// The fused sweeps cover bounded lines that have tables (bounded.hip) and
+// periodic lines with nx = 64, 128, 256 or 512 (one
 // wavefront per x line, 1..8 points per lane) and ny, nz that YzShape can
 // plan (a multiple of 16 whose block fits; 16..512 for both precisions).  The product derivative
 // uses the set of parity d==c (transeq.f90:125) and the velocity derivative
@@ -273,6 +303,10 @@ __global__ void __launch_bounds__(256) mom_x_kernel(const MomArgs<T> A, int nlin
 bool momentum_fusable(const Context &c) {
   for (int d = 0; d < 3; ++d) {
     const DirCoef &D = c.dir[d];
+    if (D.bc1 != 0 && D.bcn != 0) {
+      if (!bounded_momentum_ok<double>(c, d) || !bounded_momentum_ok<float>(c, d)) return false;
+      continue;
+    }
     if (D.bc1 != 0 || D.bcn != 0) return false;
     if (!same_set(c.sets[D.set_d1_even], c.sets[D.set_d1_odd])) return false;
     if (!same_set(c.sets[D.set_d2_even], c.sets[D.set_d2_odd])) return false;
@@ -286,6 +320,16 @@ bool momentum_fusable(const Context &c) {
   return true;
 }
 
+template <typename T, bool GEN>
+static void launch_mom_x(const MomArgs<T> &A, int V, int nlines, dim3 grid, dim3 block, hipStream_t st) {
+  switch (V) {
+    case 1: hipLaunchKernelGGL((mom_x_kernel<T, 1, GEN>), grid, block, 0, st, A, nlines); break;
+    case 2: hipLaunchKernelGGL((mom_x_kernel<T, 2, GEN>), grid, block, 0, st, A, nlines); break;
+    case 4: hipLaunchKernelGGL((mom_x_kernel<T, 4, GEN>), grid, block, 0, st, A, nlines); break;
+    default: hipLaunchKernelGGL((mom_x_kernel<T, 8, GEN>), grid, block, 0, st, A, nlines); break;
+  }
+}
+
 // One sweep of all three components (blockIdx.z): 3 launches a step instead
 // of 9.  Small grids gain: a one-component sweep of 64^3 leaves most of the
 // chip idle (128 to 256 blocks), three at once fill it (ten 64^3 FP32 steps
@@ -294,7 +338,7 @@ bool momentum_fusable(const Context &c) {
 template <typename T>
 int launch_momentum(const Context &c, int dir, const MomIO<T> &io, int nx, int ny, int nz, hipStream_t st) {
   const DirCoef &D = c.dir[dir];
-  if (D.bc1 != 0) return fail(X3D_ERR_UNSUPPORTED, "fused momentum sweep: periodic lines only");
+  if (D.bc1 != 0) return launch_bounded_momentum<T>(c, dir, io, st);
   if (!same_set(c.sets[D.set_d1_even], c.sets[D.set_d1_odd]) || !same_set(c.sets[D.set_d2_even], c.sets[D.set_d2_odd]))
     return fail(X3D_ERR_UNSUPPORTED, "fused momentum sweep: product and velocity sets differ");
   const TriSet &s1 = c.sets[D.set_d1_even];
@@ -326,17 +370,19 @@ int launch_momentum(const Context &c, int dir, const MomIO<T> &io, int nx, int n
     const int V = n / 64;
     if (n % 64 != 0 || !(V == 1 || V == 2 || V == 4 || V == 8))
       return fail(X3D_ERR_UNSUPPORTED, "fused x sweep needs nx = 64, 128, 256 or 512");
-    for (int i = 0; i < 3; ++i)
+    for (int i = 0; i < 3 && !io.general; ++i)
       if (io.nterms && (sizeof(T) == 8 ? !io.u_new[i] : (!io.delta[i] || !io.shadow[i])))
         return fail(X3D_ERR_ARG, "momentum: AB3 output buffers missing");
     const int nlines = ny * nz;
     const int waves = nlines < 8192 ? nlines : 8192;
     const dim3 grid((waves + 3) / 4, 1, 3), block(256);
-    switch (V) {
-      case 1: hipLaunchKernelGGL((mom_x_kernel<T, 1>), grid, block, 0, st, A, nlines); break;
-      case 2: hipLaunchKernelGGL((mom_x_kernel<T, 2>), grid, block, 0, st, A, nlines); break;
-      case 4: hipLaunchKernelGGL((mom_x_kernel<T, 4>), grid, block, 0, st, A, nlines); break;
-      default: hipLaunchKernelGGL((mom_x_kernel<T, 8>), grid, block, 0, st, A, nlines); break;
+    if (io.general) {
+      X3D_TRY(fill_update<T>(c, io, &A.up));
+      for (int i = 0; i < 3; ++i)
+        if (!io.acc[i]) return fail(X3D_ERR_ARG, "momentum: the x sweep comes last");
+      launch_mom_x<T, true>(A, V, nlines, grid, block, st);
+    } else {
+      launch_mom_x<T, false>(A, V, nlines, grid, block, st);
     }
   } else {
     if (io.nterms) return fail(X3D_ERR_ARG, "AB3 is fused into the x sweep only");

@@ -1,4 +1,5 @@
-// Fused pressure projection sweeps for a periodic box.
+// Fused pressure projection sweeps along periodic directions (bounded.hip
+// holds those along bounded ones).
 //
 //   divergence        navier.f90:257-372   x, y, z sweeps (velocity grid ->
 //                                          pressure grid, staggered "vp" ops)
@@ -17,51 +18,10 @@
 #include <cmath>
 #include <vector>
 
-#include "lines_impl.h"
+#include "bounded_impl.h"
 #include "state64.h"
 
 namespace x3d {
-
-// Inputs of each sweep and the solve they feed: I0/I1 interpolations, D0 the
-// derivative (-1: absent).
-//   DIV_X   out0 = Dvp(u), out1 = Ivp(v), out2 = Ivp(w)        navier.f90:297,313-314
-//   DIV_Y   out0 = Ivp(in0) + Dvp(in1), out1 = Ivp(in2)         navier.f90:321-327
-//   DIV_Z   out0 = Ivp(in0) + Dvp(in1)                          navier.f90:333-339
-//   GRAD_Z  out0 = Ipv(in0), out1 = Dpv(in0)                    navier.f90:400-403
-//   GRAD_Y  out0 = Ipv(in0), out1 = Dpv(in0), out2 = Ipv(in1)   navier.f90:414-419
-//   GRAD_X  u -= Dpv(in0), v -= Ipv(in1), w -= Ipv(in2)         navier.f90:426-431, cor_vel 206-249
-template <int SW>
-struct Recipe;
-template <>
-struct Recipe<SW_DIV_X> {
-  static constexpr bool PV = false;
-  static constexpr int NIN = 3, NI = 2, I0 = 1, I1 = 2, D0 = 0;
-};
-template <>
-struct Recipe<SW_DIV_Y> {
-  static constexpr bool PV = false;
-  static constexpr int NIN = 3, NI = 2, I0 = 0, I1 = 2, D0 = 1;
-};
-template <>
-struct Recipe<SW_DIV_Z> {
-  static constexpr bool PV = false;
-  static constexpr int NIN = 2, NI = 1, I0 = 0, I1 = -1, D0 = 1;
-};
-template <>
-struct Recipe<SW_GRAD_Z> {
-  static constexpr bool PV = true;
-  static constexpr int NIN = 1, NI = 1, I0 = 0, I1 = -1, D0 = 0;
-};
-template <>
-struct Recipe<SW_GRAD_Y> {
-  static constexpr bool PV = true;
-  static constexpr int NIN = 2, NI = 2, I0 = 0, I1 = 1, D0 = 0;
-};
-template <>
-struct Recipe<SW_GRAD_X> {
-  static constexpr bool PV = true;
-  static constexpr int NIN = 3, NI = 2, I0 = 1, I1 = 2, D0 = 0;
-};
 
 template <typename T>
 struct ProjArgs {
@@ -84,6 +44,7 @@ struct ProjArgs {
   const float *hold[3];
   int32_t *res[3];
   double *divp;                 // DIV_Z: per-block max and sum |div u*| (null: none)
+  CorVel cv;                    // GRAD_X of the general step
 };
 
 // ---------------------------------------------------------------- y / z sweeps
@@ -174,28 +135,7 @@ __global__ void __launch_bounds__(1024) proj_yz_kernel(const ProjArgs<T> A) {
           sm += fabs(v);
         }
       }
-#pragma unroll
-      for (int off = 32; off > 0; off >>= 1) {
-        const double om = __shfl_xor(mx, off), os = __shfl_xor(sm, off);
-        mx = om > mx ? om : mx;
-        sm += os;
-      }
-      __shared__ double rmx[16], rsm[16];
-      if ((tid & 63) == 0) {
-        rmx[tid >> 6] = mx;
-        rsm[tid >> 6] = sm;
-      }
-      __syncthreads();
-      if (tid == 0) {
-        double bm = rmx[0], bs = rsm[0];
-        for (int i = 1; i < (nthr + 63) / 64; ++i) {
-          bm = rmx[i] > bm ? rmx[i] : bm;
-          bs += rsm[i];
-        }
-        const unsigned nblk = gridDim.x * gridDim.y, blk = blockIdx.y * gridDim.x + blockIdx.x;
-        A.divp[blk] = bm;
-        A.divp[nblk + blk] = bs;
-      }
+      block_max_sum(mx, sm, tid, nthr, A.divp);
     }
   }
 }
@@ -248,12 +188,33 @@ __device__ __forceinline__ void correct(const ProjArgs<T> &A, const int c, const
   }
 }
 
+// The same in the general step (no split state, no increment), with the wall
+// planes stored; base is the first of V points of line (j, k).
+template <int V, typename T>
+__device__ __forceinline__ void correct_general(const CorVel &A, const int c, const long long base, const int i0,
+                                                const int j, const int k, const T (&g)[V]) {
+#pragma unroll
+  for (int m = 0; m < V; ++m) store_wall(A, c, i0 + m, j, k, g[m]);
+  if (!A.apply) return;
+  double u[V];
+  load_run<double, V>(A.u64[c] + base, u);
+#pragma unroll
+  for (int m = 0; m < V; ++m) u[m] = u[m] - (double)g[m];
+  store_run<double, V>(A.u64[c] + base, u);
+  if constexpr (sizeof(T) == 4) {
+    float f[V];
+#pragma unroll
+    for (int m = 0; m < V; ++m) f[m] = (float)u[m];
+    store_run<float, V>(A.u32[c] + base, f);
+  }
+}
+
 // FP32 gradient sweep over 256-point lines: held to 128 VGPRs (4 waves per
 // SIMD instead of 3), which it fits without spilling
 template <typename T, int V, int SW>
 constexpr int projx_wpe() { return (sizeof(T) == 4 && V == 4 && SW == SW_GRAD_X) ? 4 : 1; }
 
-template <typename T, int V, int SW>
+template <typename T, int V, int SW, bool GEN>
 __global__ void __launch_bounds__(256, (projx_wpe<T, V, SW>())) proj_x_kernel(const ProjArgs<T> A, int nlines) {
   using R = Recipe<SW>;
   constexpr int OPI = R::PV ? OP_INTERPV : OP_INTERVP;
@@ -314,6 +275,11 @@ __global__ void __launch_bounds__(256, (projx_wpe<T, V, SW>())) proj_x_kernel(co
       store_run<T, V>(A.out[0] + base, wD);
       store_run<T, V>(A.out[1] + base, wI[0]);
       store_run<T, V>(A.out[2] + base, wI[1]);
+    } else if constexpr (GEN) {
+      const int lu = __builtin_amdgcn_readfirstlane(ln), k = lu / A.cv.ny, j = lu - k * A.cv.ny;
+      correct_general<V>(A.cv, 0, base, e0, j, k, wD);
+      correct_general<V>(A.cv, 1, base, e0, j, k, wI[0]);
+      correct_general<V>(A.cv, 2, base, e0, j, k, wI[1]);
     } else {   // SW_GRAD_X: u_c -= grad_c p with the FP64 velocity (cor_vel)
       correct<V>(A, 0, base, wD);
       correct<V>(A, 1, base, wI[0]);
@@ -324,10 +290,15 @@ __global__ void __launch_bounds__(256, (projx_wpe<T, V, SW>())) proj_x_kernel(co
 
 // ---------------------------------------------------------------- host side
 // The fused projection covers the grids of the fused momentum sweeps: periodic
-// lines, nx = 64..512 (x wavefronts) and ny, nz planned by YzShape.
+// lines with nx = 64..512 (x wavefronts) and ny, nz planned by YzShape, and
+// bounded lines that have tables (bounded.hip).
 bool projection_fusable(const Context &c) {
   for (int d = 0; d < 3; ++d) {
     const DirCoef &D = c.dir[d];
+    if (D.bc1 != 0 && D.bcn != 0) {
+      if (!bounded_projection_ok<double>(c, d) || !bounded_projection_ok<float>(c, d)) return false;
+      continue;
+    }
     if (D.bc1 != 0 || D.bcn != 0 || D.nm != D.n) return false;
     if (d == 0) {
       const int V = D.n / 64;
@@ -345,40 +316,38 @@ static void launch_yz(const ProjArgs<T> &A, const YzShape<T> &Y, hipStream_t st)
   hipLaunchKernelGGL((proj_yz_kernel<T, YzShape<T>::L, SW>), grid, block, Y.shmem, st, A);
 }
 
-template <typename T, int SW>
+template <typename T, int SW, bool GEN>
 static void launch_x(const ProjArgs<T> &A, int V, int nlines, hipStream_t st) {
   const int waves = nlines < 8192 ? nlines : 8192;
   const dim3 grid((waves + 3) / 4), block(256);
   switch (V) {
-    case 1: hipLaunchKernelGGL((proj_x_kernel<T, 1, SW>), grid, block, 0, st, A, nlines); break;
-    case 2: hipLaunchKernelGGL((proj_x_kernel<T, 2, SW>), grid, block, 0, st, A, nlines); break;
-    case 4: hipLaunchKernelGGL((proj_x_kernel<T, 4, SW>), grid, block, 0, st, A, nlines); break;
-    default: hipLaunchKernelGGL((proj_x_kernel<T, 8, SW>), grid, block, 0, st, A, nlines); break;
+    case 1: hipLaunchKernelGGL((proj_x_kernel<T, 1, SW, GEN>), grid, block, 0, st, A, nlines); break;
+    case 2: hipLaunchKernelGGL((proj_x_kernel<T, 2, SW, GEN>), grid, block, 0, st, A, nlines); break;
+    case 4: hipLaunchKernelGGL((proj_x_kernel<T, 4, SW, GEN>), grid, block, 0, st, A, nlines); break;
+    default: hipLaunchKernelGGL((proj_x_kernel<T, 8, SW, GEN>), grid, block, 0, st, A, nlines); break;
   }
 }
 
-// One projection sweep.  in/out follow the recipes above; u64/u32 are used
-// by SW_GRAD_X only (u32 null for FP64 compute).
+// One projection sweep; in/out follow the recipes.
 template <typename T>
-int launch_projection(const Context &c, int sw, const T *const in[3], T *const out[3], double *const u64[3],
-                      float *const u32[3], const float *const du[3], int nx, int ny, int nz, hipStream_t st,
-                      double *divp, int *divp_blocks, const float *const hold[3], int32_t *const res[3]) {
+int launch_projection(const Context &c, int sw, const ProjIO<T> &io, hipStream_t st) {
   if (sw < SW_DIV_X || sw > SW_GRAD_X) return fail(X3D_ERR_ARG, "projection: unknown sweep");
   const int dir = (sw == SW_DIV_X || sw == SW_GRAD_X) ? 0 : (sw == SW_DIV_Y || sw == SW_GRAD_Y) ? 1 : 2;
   const bool pv = sw >= SW_GRAD_Z;
   const DirCoef &D = c.dir[dir];
-  if (D.bc1 != 0 || D.nm != D.n) return fail(X3D_ERR_UNSUPPORTED, "fused projection: periodic lines only");
+  if (D.bc1 != 0) return launch_bounded_projection<T>(c, sw, io, st);
+  if (D.nm != D.n) return fail(X3D_ERR_UNSUPPORTED, "fused projection: periodic lines only");
   const TriSet &sI = c.sets[pv ? D.set_ci6 : D.set_ci6p];
   const TriSet &sD = c.sets[D.set_c6];
   ProjArgs<T> A{};
   for (int i = 0; i < 3; ++i) {
-    A.in[i] = in[i];
-    A.out[i] = out ? out[i] : nullptr;
-    A.u64[i] = u64 ? u64[i] : nullptr;
-    A.u32[i] = u32 ? u32[i] : nullptr;
-    A.du[i] = du ? du[i] : nullptr;
-    A.hold[i] = hold ? hold[i] : nullptr;
-    A.res[i] = res ? res[i] : nullptr;
+    A.in[i] = io.in[i];
+    A.out[i] = io.out[i];
+    A.u64[i] = io.u64[i];
+    A.u32[i] = io.u32[i];
+    A.du[i] = io.du[i];
+    A.hold[i] = io.hold[i];
+    A.res[i] = io.res[i];
   }
   TriDev<T> tI, tD;
   if constexpr (sizeof(T) == 8) { tI = sI.dev64(); tD = sD.dev64(); }
@@ -388,36 +357,42 @@ int launch_projection(const Context &c, int sw, const T *const in[3], T *const o
   A.rdenI = tI.rden; A.rdenD = tD.rden;
   A.s = cast_sten<T>(D.s);
   A.n = D.n;
-  const int n = D.n;
+  const int n = D.n, ny = c.p.ny, nz = c.p.nz;
   if (dir == 0) {
     const int V = n / 64;
     if (n % 64 != 0 || !(V == 1 || V == 2 || V == 4 || V == 8))
       return fail(X3D_ERR_UNSUPPORTED, "fused x sweep needs nx = 64, 128, 256 or 512");
-    if (sw == SW_GRAD_X) {
+    const int nlines = ny * nz;
+    if (sw == SW_DIV_X) {
+      launch_x<T, SW_DIV_X, false>(A, V, nlines, st);
+    } else if (io.general) {
+      X3D_TRY(fill_corvel<T>(c, io, &A.cv));
+      launch_x<T, SW_GRAD_X, true>(A, V, nlines, st);
+    } else {
       bool ok = true;
       for (int i = 0; i < 3; ++i) {
-        if (res && sizeof(T) == 4) ok = ok && hold && hold[i] && res[i] && u32 && u32[i] && du && du[i];
-        else ok = ok && u64 && u64[i];
+        if (io.res[i] && sizeof(T) == 4) ok = ok && io.hold[i] && io.u32[i] && io.du[i];
+        else ok = ok && io.u64[i];
       }
       if (!ok) return fail(X3D_ERR_ARG, "projection: GRAD_X needs the FP64 velocity (plain or split)");
+      launch_x<T, SW_GRAD_X, false>(A, V, nlines, st);
     }
-    const int nlines = ny * nz;
-    if (sw == SW_DIV_X) launch_x<T, SW_DIV_X>(A, V, nlines, st);
-    else launch_x<T, SW_GRAD_X>(A, V, nlines, st);
   } else {
+    // x is on the pressure grid in every y and z pass, y in every z pass
+    const int nx = c.nxm, nym = c.nym;
     if (dir == 1) {
-      A.na = nx; A.nb = nz; A.sa = 1; A.sb = (long long)nx * ny; A.se = nx;
+      A.na = nx; A.nb = nz; A.sa = 1; A.sb = (long long)nx * n; A.se = nx;
     } else {
-      A.na = nx; A.nb = ny; A.sa = 1; A.sb = nx; A.se = (long long)nx * ny;
+      A.na = nx; A.nb = nym; A.sa = 1; A.sb = nx; A.se = (long long)nx * nym;
     }
     YzShape<T> Y;
     if (!Y.plan(n, 2, 3)) return fail(X3D_ERR_UNSUPPORTED, "fused y/z sweep: line length not supported");
-    if ((size_t)nx * ny * nz * sizeof(T) >= ((size_t)1 << 32))
+    if ((size_t)A.na * A.nb * n * sizeof(T) >= ((size_t)1 << 32))
       return fail(X3D_ERR_UNSUPPORTED, "fused y/z sweep: field larger than 4 GiB");
     A.kdepth = std::max(tI.kdepth, tD.kdepth);
-    if (sw == SW_DIV_Z && divp) {
-      A.divp = divp;
-      if (divp_blocks) *divp_blocks = ((A.na + Y.TL - 1) / Y.TL) * A.nb;
+    if (sw == SW_DIV_Z && io.divp) {
+      A.divp = io.divp;
+      if (io.divp_blocks) *io.divp_blocks = ((A.na + Y.TL - 1) / Y.TL) * A.nb;
     }
     switch (sw) {
       case SW_DIV_Y: launch_yz<T, SW_DIV_Y>(A, Y, st); break;
@@ -431,11 +406,7 @@ int launch_projection(const Context &c, int sw, const T *const in[3], T *const o
   return X3D_OK;
 }
 
-template int launch_projection<double>(const Context &, int, const double *const[3], double *const[3],
-                                       double *const[3], float *const[3], const float *const[3], int, int, int,
-                                       hipStream_t, double *, int *, const float *const[3], int32_t *const[3]);
-template int launch_projection<float>(const Context &, int, const float *const[3], float *const[3],
-                                      double *const[3], float *const[3], const float *const[3], int, int, int,
-                                      hipStream_t, double *, int *, const float *const[3], int32_t *const[3]);
+template int launch_projection<double>(const Context &, int, const ProjIO<double> &, hipStream_t);
+template int launch_projection<float>(const Context &, int, const ProjIO<float> &, hipStream_t);
 
 }  // namespace x3d

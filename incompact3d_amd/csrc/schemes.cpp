@@ -299,6 +299,11 @@ int chain_depth(const TriSet &s, int L, double tol) {
     gfw[e / L] *= std::fabs(s.fs[e]);
     gbw[e / L] *= std::fabs(s.ff[e] * s.fw[e]);
   }
+  return chain_depth(gfw, gbw, tol);
+}
+
+int chain_depth(const std::vector<double> &gfw, const std::vector<double> &gbw, double tol) {
+  const int P = (int)gfw.size();
   double rho = 0;
   for (int p = 0; p < P; ++p) rho = std::max(rho, std::max(gfw[p], gbw[p]));
   if (rho >= 1.0) return P;

@@ -74,7 +74,8 @@ int launch_wall_store(const T *g, double *dst, double gdt, int nx, int ny, int n
 struct x3d_solver {
   int precision = 0;
   int itime = 0;
-  bool fused = false;          // the fused sweeps (momentum.hip, projection.hip) cover this grid
+  bool fused = false;          // the fused sweeps (momentum.hip, projection.hip, bounded.hip) cover this grid
+  bool plain = false;          // ... and the step is AB3 on a periodic box
   size_t n = 0;
   int nx = 0, ny = 0, nz = 0;
   double *u64[3] = {nullptr, nullptr, nullptr};   // current velocity (FP64)
@@ -389,6 +390,106 @@ int channel_forcing(const Context &c, x3d_solver *S, int comp, T *f1, const T *c
   return X3D_OK;
 }
 
+// gradp and cor_vel by the fused sweeps of the general step, pressure in
+// W[0], which is kept.  The buffer set the velocity left in the x momentum
+// sweep is free by now; the third field of the y pass goes there (a bounded
+// y's lines grow in that pass, so it cannot overwrite its input).
+template <typename T>
+int fused_gradp(const Context &c, x3d_solver *S, T *const W[5], double gdt, bool apply) {
+  T *const spare = sizeof(T) == 8 ? (T *)S->u64b[0] : (T *)S->u32b[0];
+  ProjIO<T> gz, gy, gx;
+  gz.in[0] = W[0];
+  gz.out[0] = W[1];
+  gz.out[1] = W[2];
+  X3D_TRY(launch_projection<T>(c, SW_GRAD_Z, gz, c.stream));
+  gy.in[0] = W[1];
+  gy.in[1] = W[2];
+  gy.out[0] = W[3];
+  gy.out[1] = W[4];
+  gy.out[2] = spare;
+  X3D_TRY(launch_projection<T>(c, SW_GRAD_Y, gy, c.stream));
+  gx.in[0] = W[3];
+  gx.in[1] = W[4];
+  gx.in[2] = spare;
+  for (int i = 0; i < 3; ++i) {
+    gx.u64[i] = S->u64[i];
+    gx.u32[i] = sizeof(T) == 8 ? nullptr : S->u32[i];
+  }
+  gx.general = true;
+  gx.apply = apply;
+  gx.wall1 = S->wall1;
+  gx.walln = S->walln;
+  gx.wallg = S->wallg;
+  gx.gdt = gdt;
+  return launch_projection<T>(c, SW_GRAD_X, gx, c.stream);
+}
+
+// One sub-step of the general fused path (RK3, or AB3 with bounded
+// directions): three momentum sweeps, the last of which adds the forcing and
+// updates the velocity ca f1 + cb f2 + cc f3 with pre_correc, divergence,
+// pressure, correction.  slot: hist slots of f1, f2, f3.
+template <typename T>
+int fused_substep(Context &c, x3d_solver *S, double ca, double cb, double cc, int nterms, const int slot[3],
+                  double gdt) {
+  const int nx = S->nx, ny = S->ny, nz = S->nz;
+  T *W[5] = {(T *)S->w[0], (T *)S->w[1], (T *)S->w[2], (T *)S->w[3], (T *)S->w[4]};
+  const T *u[3];
+  for (int i = 0; i < 3; ++i) u[i] = sizeof(T) == 8 ? (const T *)S->u64[i] : (const T *)S->u32[i];
+  X3D_TRY(channel_cfr(c, S));
+  MomIO<T> z, y, x;
+  if (S->les) {
+    T *sgs[3];
+    for (int i = 0; i < 3; ++i) z.acc[i] = sgs[i] = (T *)S->lesw + (17 + i) * S->n;
+    X3D_TRY(compute_sgs<T>(c, S, u, sgs));
+  }
+  for (int i = 0; i < 3; ++i) {
+    z.u[i] = y.u[i] = x.u[i] = u[i];
+    z.out[i] = y.out[i] = W[i];
+    y.acc[i] = x.acc[i] = W[i];
+    x.out[i] = (T *)S->hist[i][slot[0]];
+    x.f2[i] = (const T *)S->hist[i][slot[1]];
+    x.f3[i] = (const T *)S->hist[i][slot[2]];
+    x.u_new[i] = sizeof(T) == 8 ? S->u64b[i] : S->u64[i];
+    x.shadow[i] = sizeof(T) == 8 ? nullptr : S->u32b[i];
+  }
+  x.general = true;
+  x.ca = ca; x.cb = cb; x.cc = cc; x.nterms = nterms;
+  // momentum_forcing_channel (Case-Channel.f90:396-420)
+  if (S->forcing == 2) x.addc = S->fvalue;
+  if (S->itime < S->spinup_time) {
+    x.rot[0] = u[1];
+    x.rotc[0] = (T)-S->wrotation;
+    x.rot[1] = u[0];
+    x.rotc[1] = (T)S->wrotation;
+  }
+  x.wall1 = S->wall1; x.walln = S->walln; x.wallg = S->wallg; x.gdt = gdt;
+  X3D_TRY(launch_momentum<T>(c, 2, z, nx, ny, nz, c.stream));
+  X3D_TRY(launch_momentum<T>(c, 1, y, nx, ny, nz, c.stream));
+  X3D_TRY(launch_momentum<T>(c, 0, x, nx, ny, nz, c.stream));
+  for (int i = 0; i < 3; ++i) {
+    if (sizeof(T) == 8) std::swap(S->u64[i], S->u64b[i]);
+    else std::swap(S->u32[i], S->u32b[i]);
+  }
+  ProjIO<T> dx, dy, dz;
+  for (int i = 0; i < 3; ++i) {
+    dx.in[i] = sizeof(T) == 8 ? (const T *)S->u64[i] : (const T *)S->u32[i];
+    dx.out[i] = W[i];
+    dy.in[i] = W[i];
+  }
+  X3D_TRY(launch_projection<T>(c, SW_DIV_X, dx, c.stream));
+  dy.out[0] = W[3];
+  dy.out[1] = W[4];
+  X3D_TRY(launch_projection<T>(c, SW_DIV_Y, dy, c.stream));
+  dz.in[0] = W[3];
+  dz.in[1] = W[4];
+  dz.out[0] = W[0];
+  dz.divp = S->divp;
+  dz.divp_blocks = &S->divp_n;
+  X3D_TRY(launch_projection<T>(c, SW_DIV_Z, dz, c.stream));
+  X3D_TRY(poisson_solve<T>(c, W[0], c.stream));
+  return fused_gradp<T>(c, S, W, gdt, true);
+}
+
 // One RK3 step (itimescheme=5, xcompact3d.f90:46-87): three sub-steps of
 // transeq RHS, the low-storage update of time_integrators.f90:151-157 with
 // the coefficients of variables.f90:1388-1399 (FP64 accumulation),
@@ -407,6 +508,11 @@ int step_rk3(Context &c, x3d_solver *S) {
   const double gdt[3] = {adt[0], adt[1] + bdt[1], adt[2] + bdt[2]};
   const T *cu[3] = {u[0], u[1], u[2]};
   for (int itr = 0; itr < 3; ++itr) {
+    if (S->fused) {
+      X3D_TRY(fused_substep<T>(c, S, adt[itr], bdt[itr], 0.0, itr == 0 ? 1 : 2, S->slot, gdt[itr]));
+      std::swap(S->slot[0], S->slot[1]);   // f2 <- f1
+      continue;
+    }
     X3D_TRY(channel_cfr(c, S));
     T *sgs[3] = {nullptr, nullptr, nullptr};
     if (S->les) {
@@ -456,6 +562,14 @@ int step_once(Context &c, x3d_solver *S) {
   }
   // gdt(1) of variables.f90:1368-1372, the same at every step
   const double gdt = (23.0 / 12.0) * dt + (-(16.0 / 12.0) * dt) + (5.0 / 12.0) * dt;
+  if (S->fused && !S->plain) {
+    X3D_TRY(fused_substep<T>(c, S, a, b, cc, nterms, S->slot, gdt));
+    const int s1 = S->slot[0], s2 = S->slot[1], s3 = S->slot[2];
+    S->slot[0] = s3;
+    S->slot[1] = s1;
+    S->slot[2] = s2;
+    return X3D_OK;
+  }
   X3D_TRY(channel_cfr(c, S));
   // transeq (z, y, x sweeps per component) with AB3 fused into the x sweep;
   // the new velocity goes to the second buffer set
@@ -517,38 +631,49 @@ int step_once(Context &c, x3d_solver *S) {
   S->slot[2] = s2;
   // projection
   if (S->fused) {
-    T *const onone[3] = {nullptr, nullptr, nullptr};
-    const T *const dx_in[3] = {cu[0], cu[1], cu[2]};
-    T *const dx_out[3] = {W[0], W[1], W[2]};
-    X3D_TRY(launch_projection<T>(c, SW_DIV_X, dx_in, dx_out, nullptr, nullptr, nullptr, nx, ny, nz, c.stream));
-    const T *const dy_in[3] = {W[0], W[1], W[2]};
-    T *const dy_out[3] = {W[3], W[1], nullptr};
-    X3D_TRY(launch_projection<T>(c, SW_DIV_Y, dy_in, dy_out, nullptr, nullptr, nullptr, nx, ny, nz, c.stream));
-    const T *const dz_in[3] = {W[3], W[1], nullptr};
-    T *const dz_out[3] = {W[0], nullptr, nullptr};
-    X3D_TRY(launch_projection<T>(c, SW_DIV_Z, dz_in, dz_out, nullptr, nullptr, nullptr, nx, ny, nz, c.stream,
-                                 S->divp, &S->divp_n));
-    X3D_TRY(poisson_solve<T>(c, W[0], c.stream));
-    const T *const gz_in[3] = {W[0], nullptr, nullptr};
-    T *const gz_out[3] = {W[1], W[2], nullptr};
-    X3D_TRY(launch_projection<T>(c, SW_GRAD_Z, gz_in, gz_out, nullptr, nullptr, nullptr, nx, ny, nz, c.stream));
-    const T *const gy_in[3] = {W[1], W[2], nullptr};
-    T *const gy_out[3] = {W[3], W[4], W[1]};   // W[0] keeps the pressure
-    X3D_TRY(launch_projection<T>(c, SW_GRAD_Y, gy_in, gy_out, nullptr, nullptr, nullptr, nx, ny, nz, c.stream));
-    const T *const gx_in[3] = {W[3], W[4], W[1]};
-    double *const u64[3] = {S->u64[0], S->u64[1], S->u64[2]};
-    float *const u32[3] = {S->u32[0], S->u32[1], S->u32[2]};
-    const float *const du[3] = {(const float *)S->u64b[0], (const float *)S->u64b[1], (const float *)S->u64b[2]};
-    if (S->split) {
-      // after the swap u32b holds the rounding of the velocity before the step
-      const float *const hold[3] = {S->u32b[0], S->u32b[1], S->u32b[2]};
-      X3D_TRY(launch_projection<T>(c, SW_GRAD_X, gx_in, onone, nullptr, u32, du, nx, ny, nz, c.stream, nullptr,
-                                   nullptr, hold, S->res));
-      S->u64_stale = true;
-    } else {
-      X3D_TRY(launch_projection<T>(c, SW_GRAD_X, gx_in, onone, u64, sizeof(T) == 8 ? nullptr : u32,
-                                   sizeof(T) == 8 ? nullptr : du, nx, ny, nz, c.stream));
+    ProjIO<T> dx, dy, dz, gz, gy, gx;
+    for (int i = 0; i < 3; ++i) {
+      dx.in[i] = cu[i];
+      dx.out[i] = W[i];
+      dy.in[i] = W[i];
     }
+    X3D_TRY(launch_projection<T>(c, SW_DIV_X, dx, c.stream));
+    dy.out[0] = W[3];
+    dy.out[1] = W[1];
+    X3D_TRY(launch_projection<T>(c, SW_DIV_Y, dy, c.stream));
+    dz.in[0] = W[3];
+    dz.in[1] = W[1];
+    dz.out[0] = W[0];
+    dz.divp = S->divp;
+    dz.divp_blocks = &S->divp_n;
+    X3D_TRY(launch_projection<T>(c, SW_DIV_Z, dz, c.stream));
+    X3D_TRY(poisson_solve<T>(c, W[0], c.stream));
+    gz.in[0] = W[0];
+    gz.out[0] = W[1];
+    gz.out[1] = W[2];
+    X3D_TRY(launch_projection<T>(c, SW_GRAD_Z, gz, c.stream));
+    gy.in[0] = W[1];
+    gy.in[1] = W[2];
+    gy.out[0] = W[3];   // W[0] keeps the pressure
+    gy.out[1] = W[4];
+    gy.out[2] = W[1];
+    X3D_TRY(launch_projection<T>(c, SW_GRAD_Y, gy, c.stream));
+    gx.in[0] = W[3];
+    gx.in[1] = W[4];
+    gx.in[2] = W[1];
+    for (int i = 0; i < 3; ++i) {
+      if (S->split) {
+        // after the swap u32b holds the rounding of the velocity before the step
+        gx.u32[i] = S->u32[i];
+        gx.du[i] = (const float *)S->u64b[i];
+        gx.hold[i] = S->u32b[i];
+        gx.res[i] = S->res[i];
+      } else {
+        gx.u64[i] = S->u64[i];
+      }
+    }
+    X3D_TRY(launch_projection<T>(c, SW_GRAD_X, gx, c.stream));
+    if (S->split) S->u64_stale = true;
   } else {
     X3D_TRY(pre_correc(c, S, gdt));
     X3D_TRY(divergence<T>(c, cu, W, nx, ny, nz));
@@ -606,7 +731,8 @@ int alloc_solver(Context &c, x3d_solver *S) {
     X3D_HIP(hipMalloc(&S->u64[i], n * 8));
     if (S->precision == 1) X3D_HIP(hipMalloc(&S->u32[i], n * 4));
     if (S->fused) {
-      X3D_HIP(hipMalloc(&S->u64b[i], n * 8));
+      // (the general FP32 step updates u64 in place)
+      if (S->precision == 0 || S->plain) X3D_HIP(hipMalloc(&S->u64b[i], n * 8));
       if (S->precision == 1) X3D_HIP(hipMalloc(&S->u32b[i], n * 4));
     }
     if (S->split) X3D_HIP(hipMalloc(&S->res[i], n * 4));
@@ -721,9 +847,9 @@ int x3d_solver_create(int precision, x3d_solver **out) {
   S->n = (size_t)S->nx * S->ny * S->nz;
   S->wall1 = c->dir[1].bc1 == 2;
   S->walln = c->dir[1].bcn == 2;
-  S->fused = c->p.itimescheme == 3 && c->p.istret == 0 && momentum_fusable(*c) && projection_fusable(*c) &&
-             getenv("X3D_UNFUSED_MOMENTUM") == nullptr;
-  S->split = S->fused && precision == 1;
+  S->fused = momentum_fusable(*c) && projection_fusable(*c) && getenv("X3D_UNFUSED_MOMENTUM") == nullptr;
+  S->plain = S->fused && c->p.itimescheme == 3 && c->dir[0].bc1 == 0 && c->dir[1].bc1 == 0 && c->dir[2].bc1 == 0;
+  S->split = S->plain && precision == 1;
   int r = alloc_solver(*c, S);
   if (r != X3D_OK) {
     free_solver(S);
@@ -900,7 +1026,7 @@ int x3d_solver_momentum_yz(x3d_solver *S, int nrep, double *bytes_per_launch) {
   Context *c;
   X3D_TRY(require_ctx(&c));
   if (!S || nrep < 0 || !bytes_per_launch) return fail(X3D_ERR_ARG, "bad arguments");
-  if (!S->fused) return fail(X3D_ERR_UNSUPPORTED, "momentum sweeps: the solver does not use the fused path");
+  if (!S->plain) return fail(X3D_ERR_UNSUPPORTED, "momentum sweeps: the solver does not use the fused path");
   if (S->precision == 0) return momentum_yz<double>(*c, S, nrep, bytes_per_launch);
   return momentum_yz<float>(*c, S, nrep, bytes_per_launch);
 }
@@ -939,7 +1065,7 @@ int x3d_solver_set_rotation(x3d_solver *S, double wrotation, int spinup_time) {
   X3D_TRY(require_ctx(&c));
   if (!S) return fail(X3D_ERR_ARG, "null solver");
   if (!std::isfinite(wrotation) || spinup_time < 0) return fail(X3D_ERR_ARG, "bad rotation arguments");
-  if (S->fused && spinup_time > 0)
+  if (S->plain && spinup_time > 0)
     return fail(X3D_ERR_UNSUPPORTED, "the spin-up rotation runs on the per-operator step (bounded y, or RK3)");
   S->wrotation = wrotation;
   S->spinup_time = spinup_time;
@@ -1142,11 +1268,13 @@ int x3d_solver_restart(x3d_solver *S, const char *rundir, double *t) {
     if (S->precision == 0) {
       double *u[3] = {S->u64[0], S->u64[1], S->u64[2]};
       double *W[5] = {(double *)S->w[0], (double *)S->w[1], (double *)S->w[2], (double *)S->w[3], (double *)S->w[4]};
-      X3D_TRY(gradp_correct<double>(*c, S, u, W, gdt, false));
+      if (S->fused) X3D_TRY(fused_gradp<double>(*c, S, W, gdt, false));
+      else X3D_TRY(gradp_correct<double>(*c, S, u, W, gdt, false));
     } else {
       float *u[3] = {S->u32[0], S->u32[1], S->u32[2]};
       float *W[5] = {(float *)S->w[0], (float *)S->w[1], (float *)S->w[2], (float *)S->w[3], (float *)S->w[4]};
-      X3D_TRY(gradp_correct<float>(*c, S, u, W, gdt, false));
+      if (S->fused) X3D_TRY(fused_gradp<float>(*c, S, W, gdt, false));
+      else X3D_TRY(gradp_correct<float>(*c, S, u, W, gdt, false));
     }
   }
   X3D_HIP(hipStreamSynchronize(c->stream));

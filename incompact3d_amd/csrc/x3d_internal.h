@@ -81,8 +81,10 @@ constexpr int SEG_L64 = 8, SEG_L32 = 16;
 int upload_set(TriSet &s);
 // Same coefficients (ff, fs, fw, sm, alfa, denominator).
 bool same_set(const TriSet &a, const TriSet &b);
-// Segment carry-chain depth for L-point segments at tolerance tol.
+// Segment carry-chain depth for L-point segments at tolerance tol; of given
+// attenuations per segment, forward and backward.
 int chain_depth(const TriSet &s, int L, double tol);
+int chain_depth(const std::vector<double> &gfw, const std::vector<double> &gbw, double tol);
 
 struct DirCoef {
   int n = 0, nm = 0, bc1 = 0, bcn = 0;
@@ -96,12 +98,22 @@ struct DirCoef {
   int set_c6 = -1, set_ci6p = -1, set_ci6 = -1, set_cip6 = -1, set_ciip6 = -1;
 };
 
+// Tables of one operator on the bounded lines of a direction (bounded_impl.h):
+// padded packed factors and closure weights, FP64 and FP32 copies, segments
+// and chain depth of each precision.
+struct BoundTab {
+  double *d64 = nullptr;
+  float *d32 = nullptr;
+  int P64 = 0, P32 = 0, K64 = 0, K32 = 0;
+};
+
 struct Context {
   x3d_params p{};
   int nxm = 0, nym = 0, nzm = 0;
   double xnu = 0;
   DirCoef dir[3];
   std::vector<TriSet> sets;
+  BoundTab btab[3][6][2];       // [direction][LineOpKind][parity]
   hipStream_t stream = nullptr;
   int device = 0;
   // stretched y mesh (istret != 0): the metrics of stretching.f90 on the
@@ -123,6 +135,10 @@ struct Context {
 
 Context *ctx();                 // nullptr if x3d_init not called
 int require_ctx(Context **c);
+
+// bounded.hip: the tables of the bounded directions
+int bounded_setup(Context &c);
+void bounded_free(Context &c);
 
 // schemes.cpp
 int build_schemes(Context &c);
@@ -191,12 +207,17 @@ constexpr size_t POISSON_SCRATCH_BYTES = (size_t)160 << 20;
 void *poisson_scratch(int device);
 
 // ---------------------------------------------------------------- fused sweeps
-// momentum.hip: the transeq right-hand side of all three components along
-// dir (out = acc + ...); the x sweep also applies AB3 (nterms > 0): FP64
-// compute writes the new velocity to u_new; FP32 compute writes the FP32
-// increment to delta and the new FP32 velocity to shadow, and the FP64
-// velocity takes the increment in the gradient correction.  acc[i] may be
-// out[i] or null.
+// momentum.hip (periodic lines), bounded.hip (free-slip and no-slip ends): the
+// transeq right-hand side of all three components along dir (out = acc +
+// ...; acc[i] may be out[i] or null).  The x sweep also updates the velocity
+// (nterms > 0 terms of AB3 or RK3), in one of two ways:
+//   plain (periodic AB3): FP64 compute writes the new velocity to u_new; FP32
+//     compute writes the FP32 increment to delta and the new FP32 velocity to
+//     shadow, and the FP64 velocity takes the increment in the gradient
+//     correction;
+//   general: forcing and pre_correc as well; FP64 compute writes the new
+//     velocity to u_new, FP32 compute updates the FP64 velocity u_new in place
+//     and writes its rounding to shadow.
 template <typename T>
 struct MomIO {
   const T *u[3] = {}, *acc[3] = {};
@@ -206,19 +227,53 @@ struct MomIO {
   float *delta[3] = {}, *shadow[3] = {};
   double ca = 0, cb = 0, cc = 0;
   int nterms = 0;
+  // general update
+  bool general = false;
+  double addc = 0;              // constant pressure gradient
+  const T *rot[3] = {};         // spin-up rotation: velocity and factor
+  T rotc[3] = {};
+  bool wall1 = false, walln = false;
+  const double *wallg = nullptr;
+  double gdt = 0;
 };
 bool momentum_fusable(const Context &c);
 template <typename T>
 int launch_momentum(const Context &c, int dir, const MomIO<T> &io, int nx, int ny, int nz, hipStream_t st);
+template <typename T>
+bool bounded_momentum_ok(const Context &c, int dir);
+template <typename T>
+int launch_bounded_momentum(const Context &c, int dir, const MomIO<T> &io, hipStream_t st);
 
-// projection.hip: divergence (x, y, z) and gradient + cor_vel (z, y, x)
+// projection.hip, bounded.hip: divergence (x, y, z) and gradient + cor_vel (z,
+// y, x).  Where a direction is bounded its input and output lines differ in
+// length and outputs must not be inputs.
 enum { SW_DIV_X = 0, SW_DIV_Y, SW_DIV_Z, SW_GRAD_Z, SW_GRAD_Y, SW_GRAD_X };
+template <typename T>
+struct ProjIO {
+  const T *in[3] = {};
+  T *out[3] = {};
+  // DIV_Z: per-block max and sum of |div u*|, and the number of blocks
+  double *divp = nullptr;
+  int *divp_blocks = nullptr;
+  // GRAD_X: the FP64 velocity and, with FP32 compute, its rounding; plain
+  // periodic FP32 steps: the AB3 increment du and the split state (hold, res)
+  double *u64[3] = {};
+  float *u32[3] = {};
+  const float *du[3] = {}, *hold[3] = {};
+  int32_t *res[3] = {};
+  // general step: the wall planes over gdt are stored, the velocity is
+  // corrected if apply is set
+  bool general = false, apply = true, wall1 = false, walln = false;
+  double *wallg = nullptr;
+  double gdt = 0;
+};
 bool projection_fusable(const Context &c);
 template <typename T>
-int launch_projection(const Context &c, int sw, const T *const in[3], T *const out[3], double *const u64[3],
-                      float *const u32[3], const float *const du[3], int nx, int ny, int nz, hipStream_t st,
-                      double *divp = nullptr, int *divp_blocks = nullptr, const float *const hold[3] = nullptr,
-                      int32_t *const res[3] = nullptr);
+int launch_projection(const Context &c, int sw, const ProjIO<T> &io, hipStream_t st);
+template <typename T>
+bool bounded_projection_ok(const Context &c, int dir);
+template <typename T>
+int launch_bounded_projection(const Context &c, int sw, const ProjIO<T> &io, hipStream_t st);
 
 // ---------------------------------------------------------------- closure network (mlp.hip)
 struct MlpDev;
