@@ -31,8 +31,9 @@ double row_of(int i, int n_in, int n_out, const Sten<double> &s, int bc1, int bc
 template <int OP>
 void edge_weights(int n_in, int n_out, const Sten<double> &s, int bc1, int bcn, int par, double *W) {
   using F = EdgeForm<OP>;
+  std::fill(W, W + EDGE_WORDS, 0.0);
   for (int end = 0; end < 2; ++end)
-    for (int q = 0; q < 4; ++q) {
+    for (int q = 0; q < F::NR; ++q) {
       const int i = end == 0 ? q : n_out - 1 - q;
       double w[8] = {};
       // the row's value on the function of the distance from this end that
@@ -40,7 +41,7 @@ void edge_weights(int n_in, int n_out, const Sten<double> &s, int bc1, int bcn, 
       auto on = [&](auto f) {
         return row_of<OP>(i, n_in, n_out, s, bc1, bcn, par, [&](int j) { return f(end == 0 ? j : n_in - 1 - j); });
       };
-      for (int j = 0; j < F::NE; ++j) {
+      for (int j = 0; j < F::NE(q); ++j) {
         if (F::KIND == 0) w[j] = on([&](int d) { return d == j ? 1.0 : 0.0; });
         else if (j == 0) w[j] = on([](int) { return 1.0; });
         else if (F::KIND == 1) w[j] = on([&](int d) { return d >= j ? 1.0 : 0.0; });
@@ -162,6 +163,23 @@ struct BMomArgs {
   MomUpdate<T> up;              // x sweep
 };
 
+// The rows of a segment to memory; NT: streaming stores.
+template <typename T, int L, bool NT>
+__device__ __forceinline__ void store_rows(T *p, const unsigned off, const unsigned step, const T (&v)[L],
+                                           const int rows) {
+  if (rows == L) {
+#pragma unroll
+    for (int m = 0; m < L; ++m) {
+      if constexpr (NT) st_nt(p, off + (unsigned)m * step, v[m]);
+      else at(p, off + (unsigned)m * step) = v[m];
+    }
+  } else {
+#pragma unroll
+    for (int m = 0; m < L; ++m)
+      if (m < rows) at(p, off + (unsigned)m * step) = v[m];
+  }
+}
+
 // -1/2 D1(u_d u_c) - 1/2 u_d D1(u_c) + nu D2(u_c) of the rows of a segment:
 // the right-hand sides from the windows.
 template <typename T, int L>
@@ -221,21 +239,30 @@ __global__ void __launch_bounds__(1024) bmom_yz_kernel(const BMomArgs<T> A) {
     for (int m = 0; m < L; ++m) dd[m] = wd[m + 2];
     bmom_rhs<T, L>(A, wc, wd, w, along, seg, rows);
   }
+  // (a block has at least n threads)
+  T mt[3];
+  if (A.m1 && tid < n) {
+    mt[0] = A.m1[tid];
+    mt[1] = A.m2[tid];
+    mt[2] = A.m4[tid];
+  }
   tc.store(cs, src, tid, nthr, CW);
-  if (A.m1) {
-    for (int i = tid; i < n; i += nthr) {
-      met[i] = A.m1[i];
-      met[n + i] = A.m2[i];
-      met[2 * n + i] = A.m4[i];
-    }
+  if (A.m1 && tid < n) {
+    met[tid] = mt[0];
+    met[n + tid] = mt[1];
+    met[2 * n + tid] = mt[2];
   }
   __syncthreads();
   bound_solve<T, L, 3, NT>(w, cs, cf, cb, gf, gb, line, seg, TL, P, A.K);
   if (!active) return;
+  // the row offsets are worked out again rather than held through the solve
+  // (they spilled)
+  int e1 = e0;
+  asm volatile("" : "+v"(e1));
   if (A.m1) {
 #pragma unroll
     for (int m = 0; m < L; ++m) {
-      const int e = e0 + m < n ? e0 + m : n - 1;
+      const int e = e1 + m < n ? e1 + m : n - 1;
       const T p1 = met[e], p2 = met[n + e], p4 = met[2 * n + e];
       w[0][m] = T(-0.5) * (p1 * w[0][m]) + T(-0.5) * (dd[m] * (p1 * w[1][m])) +
                 A.xnu * (p2 * w[2][m]) - A.xnu * (p4 * w[1][m]);
@@ -244,20 +271,17 @@ __global__ void __launch_bounds__(1024) bmom_yz_kernel(const BMomArgs<T> A) {
 #pragma unroll
     for (int m = 0; m < L; ++m) w[0][m] = T(-0.5) * w[0][m] + T(-0.5) * (dd[m] * w[1][m]) + A.xnu * w[2][m];
   }
-  const unsigned ob = base + (unsigned)e0 * step;
+  // loads of rows past the segment's repeat its last one, without branches
+  const unsigned ob = base + (unsigned)e1 * step;
   if (acc) {
     // acc may be out: this thread's points are all read before any is written
     T ac[L];
 #pragma unroll
-    for (int m = 0; m < L; ++m) ac[m] = m < rows ? at(acc, ob + (unsigned)m * step) : T(0);
+    for (int m = 0; m < L; ++m) ac[m] = at(acc, ob + (unsigned)(m < rows ? m : rows - 1) * step);
 #pragma unroll
-    for (int m = 0; m < L; ++m)
-      if (m < rows) at(out, ob + (unsigned)m * step) = ac[m] + w[0][m];
-  } else {
-#pragma unroll
-    for (int m = 0; m < L; ++m)
-      if (m < rows) at(out, ob + (unsigned)m * step) = w[0][m];
+    for (int m = 0; m < L; ++m) w[0][m] = ac[m] + w[0][m];
   }
+  store_rows<T, L, false>(out, ob, step, w[0], rows);
 }
 
 // x lines: TL whole lines are one contiguous piece of memory, staged in LDS
@@ -482,22 +506,15 @@ __global__ void __launch_bounds__(1024) bproj_yz_kernel(const BProjArgs<T> A) {
     for (int m = 0; m < L; ++m) w[N - 1][m] *= A.met[e0 + m < n_out ? e0 + m : n_out - 1];
   }
   const unsigned ob = ((unsigned)al + (unsigned)b * (unsigned)A.sb_out) * (unsigned)sizeof(T) + (unsigned)e0 * step;
-  if (active) {
+  if constexpr (SW == SW_DIV_Y || SW == SW_DIV_Z) {
 #pragma unroll
-    for (int m = 0; m < L; ++m) {
-      if (m >= rows) continue;
-      const unsigned o = ob + (unsigned)m * step;
-      if constexpr (SW == SW_DIV_Y) {
-        at(A.out[0], o) = w[0][m] + w[N - 1][m];
-        at(A.out[1], o) = w[1][m];
-      } else if constexpr (SW == SW_DIV_Z) {
-        at(A.out[0], o) = w[0][m] + w[N - 1][m];
-      } else {
-        at(A.out[0], o) = w[0][m];
-        at(A.out[1], o) = w[N - 1][m];
-        if constexpr (SW == SW_GRAD_Y) at(A.out[2], o) = w[1][m];
-      }
-    }
+    for (int m = 0; m < L; ++m) w[0][m] += w[N - 1][m];
+  }
+  if (active) {
+    store_rows<T, L, R::PV>(A.out[0], ob, step, w[0], rows);
+    if constexpr (SW == SW_DIV_Y) store_rows<T, L, false>(A.out[1], ob, step, w[1], rows);
+    if constexpr (R::PV) store_rows<T, L, true>(A.out[1], ob, step, w[N - 1], rows);
+    if constexpr (SW == SW_GRAD_Y) store_rows<T, L, true>(A.out[2], ob, step, w[1], rows);
   }
   if constexpr (SW == SW_DIV_Z) {
     if (A.divp) {
@@ -506,7 +523,7 @@ __global__ void __launch_bounds__(1024) bproj_yz_kernel(const BProjArgs<T> A) {
 #pragma unroll
         for (int m = 0; m < L; ++m) {
           if (m >= rows) continue;
-          const double v = (double)(w[0][m] + w[N - 1][m]);
+          const double v = (double)w[0][m];
           mx = v > mx ? v : mx;
           sm += fabs(v);
         }

@@ -23,31 +23,47 @@ namespace x3d {
 // [end][row from the end][8].
 constexpr int EDGE_WORDS = 2 * 4 * 8;
 
-// How many of an end's points a closure row reads, and what its weights
-// multiply: 0 the points, 1 U0 and first differences, 2 U0, U1 - U0 and second
-// differences.
+// Closure rows at each end (NR), the points row q reads (its first NE(q)), and
+// what its weights multiply (KIND): 0 the points, 1 U0 and first differences,
+// 2 U0, U1 - U0 and second differences.
 template <int OP>
 struct EdgeForm {
-  static constexpr int NE = OP == OP_DER2 || OP == OP_INTERVP || OP == OP_INTERPV ? 8 : 6;
+  static constexpr int NR = OP == OP_DER1 || OP == OP_DERPV ? 2 : (OP == OP_DERVP ? 1 : (OP == OP_INTERVP ? 3 : 4));
   static constexpr int KIND = OP == OP_DER2 ? 2 : (OP == OP_INTERVP || OP == OP_INTERPV ? 0 : 1);
+  static constexpr int NE(int q) {
+    return OP == OP_DER1 ? 4 : (OP == OP_DER2 ? q + 5 : (OP == OP_INTERVP ? q + 5 : (OP == OP_INTERPV ? q + 4 : 3)));
+  }
 };
 
+// Constant memory as the scalar unit reads it: the weights are the same for
+// every lane, and as ordinary loads they cost each end's thread a chain of
+// vector-memory latencies (the channel's y momentum sweep took 183 us with
+// those; the weights now come in through scalar loads).
+template <typename T>
+using CPtr = const __attribute__((address_space(4))) T *;
+template <typename T>
+__device__ __forceinline__ CPtr<T> uniform_ptr(const T *p) {
+  return (CPtr<T>)p;
+}
+
 template <int OP, typename T>
-__device__ __forceinline__ void edge_rows(const T (&U)[8], const T *__restrict__ W, T (&r)[4]) {
+__device__ __forceinline__ void edge_rows(const T (&U)[8], CPtr<T> W, T (&r)[4]) {
   using F = EdgeForm<OP>;
+  constexpr int NB = F::NE(F::NR - 1);
   T b[8];
 #pragma unroll
-  for (int j = 0; j < F::NE; ++j) {
+  for (int j = 0; j < NB; ++j) {
     if constexpr (F::KIND == 0) b[j] = U[j];
     else if (j == 0) b[j] = U[0];
     else if (F::KIND == 1 || j == 1) b[j] = U[j] - U[j - 1];
     else b[j] = (U[j] - U[j - 1]) - (U[j - 1] - U[j - 2]);
   }
 #pragma unroll
-  for (int q = 0; q < 4; ++q) {
+  for (int q = 0; q < F::NR; ++q) {
     T a = W[8 * q] * b[0];
 #pragma unroll
-    for (int j = 1; j < F::NE; ++j) a += W[8 * q + j] * b[j];
+    for (int j = 1; j < NB; ++j)
+      if (j < F::NE(q)) a += W[8 * q + j] * b[j];
     r[q] = a;
   }
 }
@@ -63,10 +79,12 @@ __device__ __forceinline__ int bound_rows(int seg, int P, int n_out) {
 }
 
 // Right-hand sides of a segment from its window U(e0-HW .. e0+L+HW-1), e0 its
-// first row; W the closure weights, rows how many rows the segment has.
+// first row; edge the closure weights, rows how many rows the segment has.
 template <int OP, typename T, int L, int HW>
 __device__ __forceinline__ void bound_rhs(const T (&win)[L + 2 * HW], T (&w)[L], const Sten<T> &s,
-                                          const T *__restrict__ W, const int seg, const int P, const int rows) {
+                                          const T *edge, const int seg, const int P, const int rows) {
+  using F = EdgeForm<OP>;
+  const CPtr<T> W = uniform_ptr(edge);
   // window index of the line's last point, seen from the last segment
   constexpr int FAR = L + HW - 1 + (OP == OP_DERVP || OP == OP_INTERVP) - (OP == OP_DERPV || OP == OP_INTERPV);
 #pragma unroll
@@ -77,14 +95,14 @@ __device__ __forceinline__ void bound_rhs(const T (&win)[L + 2 * HW], T (&w)[L],
     for (int j = 0; j < 8; ++j) U[j] = win[HW + j];
     edge_rows<OP, T>(U, W, r);
 #pragma unroll
-    for (int q = 0; q < 4; ++q) w[q] = r[q];
+    for (int q = 0; q < F::NR; ++q) w[q] = r[q];
   } else if (seg == P - 1) {
     T U[8], r[4];
 #pragma unroll
     for (int j = 0; j < 8; ++j) U[j] = win[FAR - j];
     edge_rows<OP, T>(U, W + 32, r);
 #pragma unroll
-    for (int q = 0; q < 4; ++q) w[L - 1 - q] = r[q];
+    for (int q = 0; q < F::NR; ++q) w[L - 1 - q] = r[q];
   }
   if (rows < L) {
 #pragma unroll
