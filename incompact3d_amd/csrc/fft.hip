@@ -14,7 +14,8 @@
 // imaginary part mode nx-k, so the two are divided by K at those two modes
 // (the real/imaginary split of waves(), poisson.f90:1740-1800).
 //
-// Passes over the half spectrum cw (nxh = nx/2+1, ny, nz), kx fastest:
+// Passes over the half spectrum cw (nxh = nx/2+1, ny, nz), kx fastest, rows
+// padded to whole 128-byte cache lines (row_pitch):
 //   1 r2c along x (real line packed as nx/2 complex points, FFT, unpack)
 //   2 c2c forward along y            (DCT-II for a non-periodic y)
 //   3 c2c forward along z, divide by -K (FP64), c2c inverse along z
@@ -64,6 +65,7 @@ struct PoissonTables {
 
 struct PoissonPlan {
   int nx, ny, nz, nxh;              // pressure-grid sizes (ny = nym when y is not periodic)
+  int np = 0;                       // row pitch of the spectral work array of this run
   int ydct;                         // 1 when y is non-periodic (poisson_010, poisson_11x)
   int xdct, zdct;                   // 1 when x / z are non-periodic (poisson_11x; x alone: poisson_100)
   double scale;                     // 1/(nx*ny*nz)
@@ -78,6 +80,15 @@ struct PoissonPlan {
   double *pf = nullptr;
   size_t pf_stride = 0;
 };
+
+// Spectral rows of whole cache lines.  With rows of nx/2+1 words the strided
+// passes' point rows of 128 or 256 bytes straddle one cache line more, which
+// two blocks, as a rule on different XCDs, then both fetch.
+template <typename T>
+static int row_pitch(int nxh) {
+  constexpr int W = 128 / (int)sizeof(cplx<T>);
+  return (nxh + W - 1) / W * W;
+}
 
 static int ilog2(int n) {
   int l = 0;
@@ -301,7 +312,7 @@ __device__ __forceinline__ int dct_row(int p, int N) { return p < (N >> 1) ? 2 *
 // X_k = (Z_k + conj Z_{M-k})/2 - i/2 e^{-2 pi i k/nx} (Z_k - conj Z_{M-k}), k = 0..M
 template <typename T, int M>
 __global__ void __launch_bounds__(FFT_THREADS) r2c_x_kernel(const T *__restrict__ in, cplx<T> *__restrict__ out,
-                                                             int nlines, int xdct, PoissonTables<T> tb) {
+                                                             int nlines, int np, int xdct, PoissonTables<T> tb) {
   using S = XShape<M>;
   constexpr int E = LineShape<M>::E, NT = S::NT, TL = S::TL;
   extern __shared__ __align__(16) unsigned char smem_raw[];
@@ -336,7 +347,7 @@ __global__ void __launch_bounds__(FFT_THREADS) r2c_x_kernel(const T *__restrict_
   for (int m = 0; m < E; ++m) ld.store(t + m * NT, x[m]);
   __syncthreads();
   if (valid) {
-    cplx<T> *dst = out + (size_t)line * (M + 1);
+    cplx<T> *dst = out + (size_t)line * np;
 #pragma unroll
     for (int m = 0; m < E; ++m) {
       const int k = t + m * NT;
@@ -361,7 +372,7 @@ __global__ void __launch_bounds__(FFT_THREADS) r2c_x_kernel(const T *__restrict_
 // Z_k = (X_k + conj X_{M-k}) + i e^{+2 pi i k/nx} (X_k - conj X_{M-k}),  k < M
 template <typename T, int M>
 __global__ void __launch_bounds__(FFT_THREADS) c2r_x_kernel(const cplx<T> *__restrict__ in, T *__restrict__ out,
-                                                             int nlines, int xdct, PoissonTables<T> tb) {
+                                                             int nlines, int np, int xdct, PoissonTables<T> tb) {
   using S = XShape<M>;
   constexpr int E = LineShape<M>::E, NT = S::NT, TL = S::TL;
   extern __shared__ __align__(16) unsigned char smem_raw[];
@@ -372,7 +383,7 @@ __global__ void __launch_bounds__(FFT_THREADS) c2r_x_kernel(const cplx<T> *__res
   const bool valid = line < nlines;
   stage_table(tw, tb.twx, M);
   stage_table(rt, tb.rtx, M + 1);
-  const cplx<T> *src = in + (size_t)line * (M + 1);
+  const cplx<T> *src = in + (size_t)line * np;
   cplx<T> xk[E], xm[E];
 #pragma unroll
   for (int m = 0; m < E; ++m) {
@@ -427,7 +438,7 @@ struct ZPass {
 // zdct), compiled separately so the periodic passes keep their registers.
 template <typename T, int N, int MODE, bool COS, bool EXTRA>
 __global__ void __launch_bounds__((SShape<T, N>::threads(EXTRA)))
-    strided_kernel(cplx<T> *__restrict__ cw, int nmain, int nxh, int ny, int nz, int ydct, double scale,
+    strided_kernel(cplx<T> *__restrict__ cw, int nmain, int nxh, int np, int ny, int nz, int ydct, double scale,
                    int zero_line, int xdct, int zdct, PoissonTables<T> tb) {
   using S = SShape<T, N>;
   constexpr int E = LineShape<N>::E, NT = S::NT, TL = S::TL, TLB = TL + (EXTRA ? 1 : 0);
@@ -457,8 +468,8 @@ __global__ void __launch_bounds__((SShape<T, N>::threads(EXTRA)))
     b = gg % nplanes;
   }
   constexpr bool ZL = ZPass<MODE>::value;
-  const size_t se = ZL ? (size_t)nxh * ny : (size_t)nxh;
-  const size_t base = ZL ? (size_t)b * nxh + a : (size_t)b * nxh * ny + a;
+  const size_t se = ZL ? (size_t)np * ny : (size_t)np;
+  const size_t base = ZL ? (size_t)b * np + a : (size_t)b * np * ny + a;
   stage_table(tw, ZL ? tb.twz : tb.twy, N);
   // the cosine transform of this pass: y in the y passes, z in the z pass
   const bool dct_here = ZL ? (MODE == FFT_Z_SOLVE && COS && zdct != 0) : ydct != 0;
@@ -926,7 +937,7 @@ static void build_penta_factors(const Context &c, const PoissonPlan &P, const st
 // (nx/2+1, :, nz/2+1) line is zeroed (poisson.f90:902-908).
 template <typename T>
 __global__ void __launch_bounds__(64) penta_y_kernel(cplx<T> *__restrict__ cw, const double *__restrict__ pf,
-                                                     size_t stride, int nxh, int ny, int nz, int nsys,
+                                                     size_t stride, int nxh, int np, int ny, int nz, int nsys,
                                                      double scale) {
   const int kx = blockIdx.x * blockDim.x + threadIdx.x;
   const int kz = blockIdx.y / nsys, par = blockIdx.y - kz * nsys;
@@ -936,7 +947,7 @@ __global__ void __launch_bounds__(64) penta_y_kernel(cplx<T> *__restrict__ cw, c
   const size_t line = ((size_t)(kzp * nsys + par) * nh) * nxh + kx;
   const double *F1 = pf + line, *F2 = pf + stride + line, *RP = pf + 2 * stride + line;
   const double *A1 = pf + 3 * stride + line, *B1 = pf + 4 * stride + line;
-  auto at = [&](int m) -> cplx<T> & { return cw[((size_t)kz * ny + (nsys * m + par)) * nxh + kx]; };
+  auto at = [&](int m) -> cplx<T> & { return cw[((size_t)kz * ny + (nsys * m + par)) * np + kx]; };
   if (kx == nxh - 1 && kz == (nz >> 1)) {
     for (int m = 0; m < nh; ++m) at(m) = cplx<T>{T(0), T(0)};
     return;
@@ -989,7 +1000,7 @@ __global__ void __launch_bounds__(64) penta_y_kernel(cplx<T> *__restrict__ cw, c
 // partner's results are conj(A) and -conj(iB) with the same K (the tables
 // are symmetric in ky and kz).
 template <typename T>
-__global__ void __launch_bounds__(256) split_divide_kernel(cplx<T> *__restrict__ cw, int nxh, int ny, int nz,
+__global__ void __launch_bounds__(256) split_divide_kernel(cplx<T> *__restrict__ cw, int nxh, int np, int ny, int nz,
                                                            double scale, PoissonTables<T> tb) {
   const size_t total = (size_t)nxh * ny * nz;
   const size_t q = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -998,9 +1009,9 @@ __global__ void __launch_bounds__(256) split_divide_kernel(cplx<T> *__restrict__
   const size_t r = q / nxh;
   const int ky = (int)(r % ny), kz = (int)(r / ny);
   const int kyp = ky ? ny - ky : 0, kzp = kz ? nz - kz : 0;
-  const size_t qp = ((size_t)kzp * ny + kyp) * nxh + a;
-  if (qp < q) return;   // the partner's thread writes both
-  const cplx<T> d = cw[q], dp = cw[qp];
+  const size_t o = r * np + a, op = ((size_t)kzp * ny + kyp) * np + a;
+  if (op < o) return;   // the partner's thread writes both
+  const cplx<T> d = cw[o], dp = cw[op];
   const int am = 2 * (nxh - 1) - a;
   const double tyv = tb.ty[ky], tzv = tb.tz[kz], ky2 = tb.ky2[ky], kz2 = tb.kz2[kz];
   const double txr = tb.tx[a], kx2r = tb.kx2[a], txi = tb.tx[am], kx2i = tb.kx2[am];
@@ -1011,8 +1022,8 @@ __global__ void __launch_bounds__(256) split_divide_kernel(cplx<T> *__restrict__
   const double fi = Ki < 1.0e-16 ? 0.0 : -scale / Ki;
   const double ar = 0.5 * ((double)d.x + (double)dp.x), ai = 0.5 * ((double)d.y - (double)dp.y);
   const double br = 0.5 * ((double)d.x - (double)dp.x), bi = 0.5 * ((double)d.y + (double)dp.y);
-  cw[q] = cplx<T>{(T)(ar * fr + br * fi), (T)(ai * fr + bi * fi)};
-  if (qp != q) cw[qp] = cplx<T>{(T)(ar * fr - br * fi), (T)(-ai * fr + bi * fi)};
+  cw[o] = cplx<T>{(T)(ar * fr + br * fi), (T)(ai * fr + bi * fi)};
+  if (op != o) cw[op] = cplx<T>{(T)(ar * fr - br * fi), (T)(-ai * fr + bi * fi)};
 }
 
 // ---------------------------------------------------------------- scratch without allocation
@@ -1123,13 +1134,13 @@ void poisson_free(Context &c) {
 }
 
 template <typename T, int M>
-static void launch_x(bool fwd, T *rhs, cplx<T> *cw, int nlines, int xdct, const PoissonTables<T> &tb,
+static void launch_x(bool fwd, T *rhs, cplx<T> *cw, int nlines, int np, int xdct, const PoissonTables<T> &tb,
                      hipStream_t st) {
   using S = XShape<M>;
   const dim3 grid((nlines + S::TL - 1) / S::TL), block(S::TL * S::NT);
   const size_t sh = S::template lds<T>();
-  if (fwd) hipLaunchKernelGGL((r2c_x_kernel<T, M>), grid, block, sh, st, rhs, cw, nlines, xdct, tb);
-  else hipLaunchKernelGGL((c2r_x_kernel<T, M>), grid, block, sh, st, cw, rhs, nlines, xdct, tb);
+  if (fwd) hipLaunchKernelGGL((r2c_x_kernel<T, M>), grid, block, sh, st, rhs, cw, nlines, np, xdct, tb);
+  else hipLaunchKernelGGL((c2r_x_kernel<T, M>), grid, block, sh, st, cw, rhs, nlines, np, xdct, tb);
 }
 
 template <typename T, int N, int MODE, bool COS, bool EXTRA>
@@ -1140,7 +1151,7 @@ static void launch_s1(const PoissonPlan &P, cplx<T> *cw, const PoissonTables<T> 
   // poisson_010 zeroes the (nx/2+1, :, nz/2+1) line (poisson.f90:902-908); poisson_11x does not
   const int zero_line = MODE == FFT_Z_SOLVE && P.ydct && !P.xdct;
   const bool zt = MODE == FFT_Z_SOLVE && !COS && S::ZTAB;
-  hipLaunchKernelGGL((strided_kernel<T, N, MODE, COS, EXTRA>), grid, block, S::lds(EXTRA, zt), st, cw, nmain, P.nxh,
+  hipLaunchKernelGGL((strided_kernel<T, N, MODE, COS, EXTRA>), grid, block, S::lds(EXTRA, zt), st, cw, nmain, P.nxh, P.np,
                      P.ny, P.nz, P.ydct, P.scale, zero_line, P.xdct, P.zdct, tb);
 }
 
@@ -1176,17 +1187,17 @@ static bool dispatch_s(int N, const PoissonPlan &P, cplx<T> *cw, const PoissonTa
 }
 
 template <typename T>
-static bool dispatch_x(bool fwd, int M, T *rhs, cplx<T> *cw, int nlines, int xdct, const PoissonTables<T> &tb,
+static bool dispatch_x(bool fwd, int M, T *rhs, cplx<T> *cw, int nlines, int np, int xdct, const PoissonTables<T> &tb,
                        hipStream_t st) {
   switch (M) {
-    case 8: launch_x<T, 8>(fwd, rhs, cw, nlines, xdct, tb, st); return true;
-    case 16: launch_x<T, 16>(fwd, rhs, cw, nlines, xdct, tb, st); return true;
-    case 32: launch_x<T, 32>(fwd, rhs, cw, nlines, xdct, tb, st); return true;
-    case 64: launch_x<T, 64>(fwd, rhs, cw, nlines, xdct, tb, st); return true;
-    case 128: launch_x<T, 128>(fwd, rhs, cw, nlines, xdct, tb, st); return true;
-    case 256: launch_x<T, 256>(fwd, rhs, cw, nlines, xdct, tb, st); return true;
-    case 512: launch_x<T, 512>(fwd, rhs, cw, nlines, xdct, tb, st); return true;
-    case 1024: launch_x<T, 1024>(fwd, rhs, cw, nlines, xdct, tb, st); return true;
+    case 8: launch_x<T, 8>(fwd, rhs, cw, nlines, np, xdct, tb, st); return true;
+    case 16: launch_x<T, 16>(fwd, rhs, cw, nlines, np, xdct, tb, st); return true;
+    case 32: launch_x<T, 32>(fwd, rhs, cw, nlines, np, xdct, tb, st); return true;
+    case 64: launch_x<T, 64>(fwd, rhs, cw, nlines, np, xdct, tb, st); return true;
+    case 128: launch_x<T, 128>(fwd, rhs, cw, nlines, np, xdct, tb, st); return true;
+    case 256: launch_x<T, 256>(fwd, rhs, cw, nlines, np, xdct, tb, st); return true;
+    case 512: launch_x<T, 512>(fwd, rhs, cw, nlines, np, xdct, tb, st); return true;
+    case 1024: launch_x<T, 1024>(fwd, rhs, cw, nlines, np, xdct, tb, st); return true;
     default: return false;
   }
 }
@@ -1194,24 +1205,35 @@ static bool dispatch_x(bool fwd, int M, T *rhs, cplx<T> *cw, int nlines, int xdc
 template <typename T>
 size_t poisson_work_bytes(const Context &c) {
   const auto *P = static_cast<const PoissonPlan *>(c.poisson);
-  return P ? (size_t)P->nxh * P->ny * P->nz * sizeof(cplx<T>) : 0;
+  return P ? (size_t)row_pitch<T>(P->nxh) * P->ny * P->nz * sizeof(cplx<T>) : 0;
 }
 template size_t poisson_work_bytes<double>(const Context &);
 template size_t poisson_work_bytes<float>(const Context &);
+template <typename T>
+size_t poisson_least_bytes(const Context &c) {
+  const auto *P = static_cast<const PoissonPlan *>(c.poisson);
+  return P ? (size_t)P->nxh * P->ny * P->nz * sizeof(cplx<T>) : 0;
+}
+template size_t poisson_least_bytes<double>(const Context &);
+template size_t poisson_least_bytes<float>(const Context &);
 
 // The five (stretched: seven) passes of the solve on the spectral work array
-// cw of poisson_work_bytes<T>(c) bytes; enqueues kernels only.
+// work of `bytes` bytes, its rows padded if poisson_work_bytes<T>(c) fit there,
+// unpadded from poisson_least_bytes<T>(c) on; enqueues kernels only.
 template <typename T>
-int poisson_run(const Context &c, T *rhs, void *work, hipStream_t st) {
-  const auto *P = static_cast<const PoissonPlan *>(c.poisson);
-  if (!P) return fail(X3D_ERR_STATE, "Poisson solver not initialised");
+int poisson_run(const Context &c, T *rhs, void *work, size_t bytes, hipStream_t st) {
+  if (!c.poisson) return fail(X3D_ERR_STATE, "Poisson solver not initialised");
+  if (bytes < poisson_least_bytes<T>(c)) return fail(X3D_ERR_ARG, "Poisson: work array too small");
+  PoissonPlan Q = *static_cast<const PoissonPlan *>(c.poisson);
+  Q.np = bytes >= poisson_work_bytes<T>(c) ? row_pitch<T>(Q.nxh) : Q.nxh;
+  const PoissonPlan *P = &Q;
   cplx<T> *cw = static_cast<cplx<T> *>(work);
   PoissonTables<T> tb;
   if constexpr (sizeof(T) == 8) tb = P->t64;
   else tb = P->t32;
   const int nlines = P->ny * P->nz, M = P->nx / 2;
   // sizes were checked by poisson_setup: every dispatch below finds its case
-  bool ok = dispatch_x<T>(true, M, rhs, cw, nlines, P->xdct, tb, st);
+  bool ok = dispatch_x<T>(true, M, rhs, cw, nlines, P->np, P->xdct, tb, st);
   ok = ok && dispatch_s<T, FFT_Y_FWD>(P->ny, *P, cw, tb, st);
   if (P->xdct && !P->ydct) {
     // poisson_100: forward z, the pairwise split and divide, inverse z
@@ -1219,7 +1241,7 @@ int poisson_run(const Context &c, T *rhs, void *work, hipStream_t st) {
     if (ok) {
       const size_t total = (size_t)P->nxh * P->ny * P->nz;
       hipLaunchKernelGGL((split_divide_kernel<T>), dim3((unsigned)((total + 255) / 256)), dim3(256), 0, st, cw,
-                         P->nxh, P->ny, P->nz, P->scale, tb);
+                         P->nxh, P->np, P->ny, P->nz, P->scale, tb);
     }
     ok = ok && dispatch_s<T, FFT_Z_INV>(P->nz, *P, cw, tb, st);
   } else if (P->ystret) {
@@ -1227,22 +1249,22 @@ int poisson_run(const Context &c, T *rhs, void *work, hipStream_t st) {
     ok = ok && dispatch_s<T, FFT_Z_FWD>(P->nz, *P, cw, tb, st);
     if (ok) {
       const dim3 grid((P->nxh + 63) / 64, P->ystret * P->nz), block(64);
-      hipLaunchKernelGGL((penta_y_kernel<T>), grid, block, 0, st, cw, P->pf, P->pf_stride, P->nxh, P->ny, P->nz,
-                         P->ystret, P->scale);
+      hipLaunchKernelGGL((penta_y_kernel<T>), grid, block, 0, st, cw, P->pf, P->pf_stride, P->nxh, P->np, P->ny,
+                         P->nz, P->ystret, P->scale);
     }
     ok = ok && dispatch_s<T, FFT_Z_INV>(P->nz, *P, cw, tb, st);
   } else {
     ok = ok && dispatch_s<T, FFT_Z_SOLVE>(P->nz, *P, cw, tb, st);
   }
   ok = ok && dispatch_s<T, FFT_Y_INV>(P->ny, *P, cw, tb, st);
-  ok = ok && dispatch_x<T>(false, M, rhs, cw, nlines, P->xdct, tb, st);
+  ok = ok && dispatch_x<T>(false, M, rhs, cw, nlines, P->np, P->xdct, tb, st);
   if (!ok) return fail(X3D_ERR_UNSUPPORTED, "Poisson: no FFT kernel for this size");
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return fail(X3D_ERR_HIP, std::string("poisson launch: ") + hipGetErrorString(e));
   return X3D_OK;
 }
-template int poisson_run<double>(const Context &, double *, void *, hipStream_t);
-template int poisson_run<float>(const Context &, float *, void *, hipStream_t);
+template int poisson_run<double>(const Context &, double *, void *, size_t, hipStream_t);
+template int poisson_run<float>(const Context &, float *, void *, size_t, hipStream_t);
 
 // The library's own work array, allocated at the first solve of each precision.
 template <typename T>
@@ -1251,7 +1273,7 @@ int poisson_solve(Context &c, T *rhs, hipStream_t st) {
   if (!P) return fail(X3D_ERR_STATE, "Poisson solver not initialised");
   void **cwp = sizeof(T) == 8 ? &P->cw64 : &P->cw32;
   if (!*cwp) X3D_HIP(hipMalloc(cwp, poisson_work_bytes<T>(c)));
-  return poisson_run<T>(c, rhs, *cwp, st);
+  return poisson_run<T>(c, rhs, *cwp, poisson_work_bytes<T>(c), st);
 }
 
 template int poisson_solve<double>(Context &, double *, hipStream_t);
@@ -1268,21 +1290,21 @@ template int poisson_solve<float>(Context &, float *, hipStream_t);
 // X(kx, ky, kz) = conj X(-kx, -ky, -kz).
 template <typename T>
 __global__ void __launch_bounds__(256) halfx_to_halfz(const cplx<T> *__restrict__ cw, cplx<T> *__restrict__ out,
-                                                      int nx, int ny, int nz, int nxh) {
+                                                      int nx, int ny, int nz, int nxh, int np) {
   const size_t total = (size_t)nx * ny * (nz / 2 + 1);
   const size_t stride = (size_t)gridDim.x * blockDim.x;
   for (size_t q = (size_t)blockIdx.x * blockDim.x + threadIdx.x; q < total; q += stride) {
     const int kx = (int)(q % nx);
     const size_t r = q / nx;
     const int ky = (int)(r % ny), kz = (int)(r / ny);
-    out[q] = kx < nxh ? cw[kx + (size_t)nxh * (ky + (size_t)ny * kz)]
-                      : cconj(cw[(nx - kx) + (size_t)nxh * ((ny - ky) % ny + (size_t)ny * ((nz - kz) % nz))]);
+    out[q] = kx < nxh ? cw[kx + (size_t)np * (ky + (size_t)ny * kz)]
+                      : cconj(cw[(nx - kx) + (size_t)np * ((ny - ky) % ny + (size_t)ny * ((nz - kz) % nz))]);
   }
 }
 
 template <typename T>
 __global__ void __launch_bounds__(256) halfz_to_halfx(const cplx<T> *__restrict__ in, cplx<T> *__restrict__ cw,
-                                                      int nx, int ny, int nz, int nxh) {
+                                                      int nx, int ny, int nz, int nxh, int np) {
   const int nzh = nz / 2 + 1;
   const size_t total = (size_t)nxh * ny * nz;
   const size_t stride = (size_t)gridDim.x * blockDim.x;
@@ -1290,7 +1312,7 @@ __global__ void __launch_bounds__(256) halfz_to_halfx(const cplx<T> *__restrict_
     const int kx = (int)(q % nxh);
     const size_t r = q / nxh;
     const int ky = (int)(r % ny), kz = (int)(r / ny);
-    cw[q] = kz < nzh ? in[kx + (size_t)nx * (ky + (size_t)ny * kz)]
+    cw[kx + (size_t)np * r] = kz < nzh ? in[kx + (size_t)nx * (ky + (size_t)ny * kz)]
                      : cconj(in[(nx - kx) % nx + (size_t)nx * ((ny - ky) % ny + (size_t)ny * (nz - kz))]);
   }
 }
@@ -1307,6 +1329,7 @@ int fft3d(Context &c, bool forward, const void *in, void *out, hipStream_t st) {
   PoissonPlan Q = *P;
   Q.xdct = Q.ydct = Q.zdct = 0;
   Q.ystret = 0;
+  Q.np = row_pitch<T>(Q.nxh);
   PoissonTables<T> tb;
   if constexpr (sizeof(T) == 8) tb = P->t64;
   else tb = P->t32;
@@ -1315,18 +1338,18 @@ int fft3d(Context &c, bool forward, const void *in, void *out, hipStream_t st) {
   const unsigned nb = (unsigned)std::min<size_t>((nout + 255) / 256, 65535u * 8u);
   bool ok;
   if (forward) {
-    ok = dispatch_x<T>(true, M, const_cast<T *>(static_cast<const T *>(in)), cw, nlines, 0, tb, st);
+    ok = dispatch_x<T>(true, M, const_cast<T *>(static_cast<const T *>(in)), cw, nlines, Q.np, 0, tb, st);
     ok = ok && dispatch_s<T, FFT_Y_FWD>(Q.ny, Q, cw, tb, st);
     ok = ok && dispatch_s<T, FFT_Z_FWD>(Q.nz, Q, cw, tb, st);
     if (ok)
       hipLaunchKernelGGL((halfx_to_halfz<T>), dim3(nb), dim3(256), 0, st, cw, static_cast<cplx<T> *>(out), Q.nx,
-                         Q.ny, Q.nz, Q.nxh);
+                         Q.ny, Q.nz, Q.nxh, Q.np);
   } else {
     hipLaunchKernelGGL((halfz_to_halfx<T>), dim3(nb), dim3(256), 0, st, static_cast<const cplx<T> *>(in), cw, Q.nx,
-                       Q.ny, Q.nz, Q.nxh);
+                       Q.ny, Q.nz, Q.nxh, Q.np);
     ok = dispatch_s<T, FFT_Z_INV>(Q.nz, Q, cw, tb, st);
     ok = ok && dispatch_s<T, FFT_Y_INV>(Q.ny, Q, cw, tb, st);
-    ok = ok && dispatch_x<T>(false, M, static_cast<T *>(out), cw, nlines, 0, tb, st);
+    ok = ok && dispatch_x<T>(false, M, static_cast<T *>(out), cw, nlines, Q.np, 0, tb, st);
   }
   if (!ok) return fail(X3D_ERR_UNSUPPORTED, "FFT: no kernel for this size");
   hipError_t e = hipGetLastError();

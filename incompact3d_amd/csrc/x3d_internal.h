@@ -192,11 +192,14 @@ int poisson_setup(Context &c);
 void poisson_free(Context &c);
 template <typename T>
 int poisson_solve(Context &c, T *rhs, hipStream_t st);
-// the solve on a caller-provided spectral work array of poisson_work_bytes
+// the solve on a caller-provided spectral work array: poisson_work_bytes for
+// rows of whole cache lines, poisson_least_bytes at least
 template <typename T>
 size_t poisson_work_bytes(const Context &c);
 template <typename T>
-int poisson_run(const Context &c, T *rhs, void *work, hipStream_t st);
+size_t poisson_least_bytes(const Context &c);
+template <typename T>
+int poisson_run(const Context &c, T *rhs, void *work, size_t bytes, hipStream_t st);
 // device address of the file-scope scratch array on `device` (taken at
 // x3d_init), nullptr before; POISSON_SCRATCH_BYTES bytes
 // decomp_2d_fft_3d on the pressure grid: real (nx,ny,nz) <-> complex
