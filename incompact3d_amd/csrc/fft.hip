@@ -269,10 +269,30 @@ struct LdLine {
   __device__ __forceinline__ cplx<T> load(int p) const { return buf[base + p + (p >> 4)]; }
 };
 
-template <typename T>
-__device__ __forceinline__ void stage_table(cplx<T> *dst, const cplx<T> *__restrict__ src, int n) {
-  for (int i = threadIdx.x; i < n; i += blockDim.x) dst[i] = src[i];
-}
+// Copy of a table of N words to LDS by NTHR threads, in two halves: load()
+// after the kernel has issued its line's loads, store() before the barrier,
+// so that the latencies of the tables and of the line overlap.  (Staged
+// first, the tables cost a pass two or three memory latencies before its own
+// loads went out.)
+template <typename V, int N, int NTHR>
+struct TableStage {
+  static constexpr int R = (N + NTHR - 1) / NTHR;
+  V v[R];
+  __device__ __forceinline__ void load(const V *__restrict__ src) {
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+      const int i = (int)threadIdx.x + r * NTHR;
+      v[r] = src[i < N ? i : N - 1];
+    }
+  }
+  __device__ __forceinline__ void store(V *dst) const {
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+      const int i = (int)threadIdx.x + r * NTHR;
+      if (i < N) dst[i] = v[r];
+    }
+  }
+};
 
 constexpr int FFT_THREADS = 256;
 
@@ -288,25 +308,59 @@ struct XShape {
 // strided blocks: TL kx x N points, NT threads per line.  TL = 256/NT lines
 // for FP64 and twice that for FP32, so that each point row a block reads is
 // 256 bytes either way (at most 64 lines, 512 threads).  The nx/2+1 kx lines
-// do not fill whole blocks: either the last column of blocks runs partly
-// empty, or (EXTRA) each block takes one of the remaining (kx, plane) lines
-// as well, on NT more threads.
+// do not fill whole blocks and the last column of blocks runs mostly empty.
+// (One line more per block instead, on a ninth wavefront, left a CU with one
+// block of the FP32 z pass where two of eight wavefronts fit: 512^3 653
+// against 418 us, 256^3 46 against 39 us.)
 template <typename T, int N>
 struct SShape {
   static constexpr int NT = LineShape<N>::NT;
   static constexpr int TL0 = (FFT_THREADS / NT) * (sizeof(T) == 4 ? 2 : 1);
   static constexpr int TL = TL0 < 64 ? TL0 : 64;
-  static constexpr int threads(bool extra) { return (TL + (extra ? 1 : 0)) * NT; }
+  static constexpr int threads() { return TL * NT; }
   // ztab: the z pass's tz and kz2 tables in FP64 (lines up to 256 points,
   // where the 4 KB keep two blocks per CU)
   static constexpr bool ZTAB = N <= 256;
-  static constexpr size_t lds(bool extra, bool ztab) {
-    return sizeof(cplx<T>) * ((size_t)(TL + (extra ? 1 : 0)) * N + 2 * N) + (ztab ? 2 * N * sizeof(double) : 0);
+  static constexpr size_t lds(bool ztab) {
+    return sizeof(cplx<T>) * ((size_t)TL * N + 2 * N) + (ztab ? 2 * N * sizeof(double) : 0);
   }
 };
 
 // row of point p under the even/odd reorder of poisson.f90:688-697 / :997-1008
 __device__ __forceinline__ int dct_row(int p, int N) { return p < (N >> 1) ? 2 * p : 2 * (N - 1 - p) + 1; }
+
+// A strided line's points t + m NT, m < E, of the line at `line` (point stride
+// se), in natural order or under the even/odd reorder.  Each half of them lies
+// at a constant distance, which is uniform, so that a pass holds one address
+// at a time and not sixteen (the FP32 z pass over 256 points: 73 registers
+// against 110).
+template <typename T, int N>
+__device__ __forceinline__ void load_strided(const cplx<T> *line, const size_t se, const int t, const bool reorder,
+                                             cplx<T> (&x)[LineShape<N>::E]) {
+  constexpr int E = LineShape<N>::E, NT = LineShape<N>::NT;
+  const ptrdiff_t d = (ptrdiff_t)se * (reorder ? 2 * NT : NT);
+  const cplx<T> *p = line + se * (size_t)(reorder ? 2 * t : t);
+#pragma unroll
+  for (int m = 0; m < E / 2; ++m, p += d) x[m] = *p;
+  p = line + se * (size_t)(reorder ? N - 1 - 2 * t : t + N / 2);
+  const ptrdiff_t d2 = reorder ? -d : d;
+#pragma unroll
+  for (int m = E / 2; m < E; ++m, p += d2) x[m] = *p;
+}
+template <typename T, int N>
+__device__ __forceinline__ void store_strided(cplx<T> *line, const size_t se, int t, const bool reorder,
+                                              const cplx<T> (&x)[LineShape<N>::E]) {
+  constexpr int E = LineShape<N>::E, NT = LineShape<N>::NT;
+  asm volatile("" : "+v"(t));   // the addresses are worked out here, not held since the loads
+  const ptrdiff_t d = (ptrdiff_t)se * (reorder ? 2 * NT : NT);
+  cplx<T> *p = line + se * (size_t)(reorder ? 2 * t : t);
+#pragma unroll
+  for (int m = 0; m < E / 2; ++m, p += d) *p = x[m];
+  p = line + se * (size_t)(reorder ? N - 1 - 2 * t : t + N / 2);
+  const ptrdiff_t d2 = reorder ? -d : d;
+#pragma unroll
+  for (int m = E / 2; m < E; ++m, p += d2) *p = x[m];
+}
 
 // ---------------------------------------------------------------- pass 1: r2c along x
 // X_k = (Z_k + conj Z_{M-k})/2 - i/2 e^{-2 pi i k/nx} (Z_k - conj Z_{M-k}), k = 0..M
@@ -321,22 +375,28 @@ __global__ void __launch_bounds__(FFT_THREADS) r2c_x_kernel(const T *__restrict_
   const int t = threadIdx.x % NT, l = threadIdx.x / NT;
   const int line = blockIdx.x * TL + l;
   const bool valid = line < nlines;
-  stage_table(tw, tb.twx, M);
-  stage_table(rt, tb.rtx, M + 1);
+  // lines past the end read the last one (no load branches)
+  const T *src = in + (size_t)(valid ? line : nlines - 1) * 2 * M;
   cplx<T> x[E];
   if (xdct) {
     // even/odd reorder along x (poisson.f90:1086-1095): point p of the FFT
     // input is row dct_row(p) of the line
-    const T *src = in + (size_t)line * 2 * M;
 #pragma unroll
     for (int m = 0; m < E; ++m) {
       const int q = t + m * NT;
-      x[m] = valid ? cplx<T>{src[dct_row(2 * q, 2 * M)], src[dct_row(2 * q + 1, 2 * M)]} : cplx<T>{T(0), T(0)};
+      x[m] = cplx<T>{src[dct_row(2 * q, 2 * M)], src[dct_row(2 * q + 1, 2 * M)]};
     }
   } else {
-    const cplx<T> *src = reinterpret_cast<const cplx<T> *>(in + (size_t)line * 2 * M);
 #pragma unroll
-    for (int m = 0; m < E; ++m) x[m] = valid ? src[t + m * NT] : cplx<T>{T(0), T(0)};
+    for (int m = 0; m < E; ++m) x[m] = reinterpret_cast<const cplx<T> *>(src)[t + m * NT];
+  }
+  {
+    TableStage<cplx<T>, M, TL * NT> s1;
+    TableStage<cplx<T>, M + 1, TL * NT> s2;
+    s1.load(tb.twx);
+    s2.load(tb.rtx);
+    s1.store(tw);
+    s2.store(rt);
   }
   __syncthreads();
   const LdLine<T> ld{buf, l * S::LP};
@@ -381,17 +441,27 @@ __global__ void __launch_bounds__(FFT_THREADS) c2r_x_kernel(const cplx<T> *__res
   const int t = threadIdx.x % NT, l = threadIdx.x / NT;
   const int line = blockIdx.x * TL + l;
   const bool valid = line < nlines;
-  stage_table(tw, tb.twx, M);
-  stage_table(rt, tb.rtx, M + 1);
-  const cplx<T> *src = in + (size_t)line * np;
+  const cplx<T> *src = in + (size_t)(valid ? line : nlines - 1) * np;
   cplx<T> xk[E], xm[E];
 #pragma unroll
   for (int m = 0; m < E; ++m) {
     const int k = t + m * NT;
-    xk[m] = valid ? src[k] : cplx<T>{T(0), T(0)};
-    xm[m] = valid ? src[M - k] : cplx<T>{T(0), T(0)};
-    if (xdct) {
-      // undo the cosine-transform shift: e^{+i pi k/(2 nx)} (poisson.f90:1428-1437)
+    xk[m] = src[k];
+    xm[m] = src[M - k];
+  }
+  {
+    TableStage<cplx<T>, M, TL * NT> s1;
+    TableStage<cplx<T>, M + 1, TL * NT> s2;
+    s1.load(tb.twx);
+    s2.load(tb.rtx);
+    s1.store(tw);
+    s2.store(rt);
+  }
+  if (xdct) {
+    // undo the cosine-transform shift: e^{+i pi k/(2 nx)} (poisson.f90:1428-1437)
+#pragma unroll
+    for (int m = 0; m < E; ++m) {
+      const int k = t + m * NT;
       xk[m] = cmul(cconj(tb.dctx[k]), xk[m]);
       xm[m] = cmul(cconj(tb.dctx[M - k]), xm[m]);
     }
@@ -436,61 +506,57 @@ struct ZPass {
 
 // COS: the poisson_11x z pass (cosine transform along x, and along z when
 // zdct), compiled separately so the periodic passes keep their registers.
-template <typename T, int N, int MODE, bool COS, bool EXTRA>
-__global__ void __launch_bounds__((SShape<T, N>::threads(EXTRA)))
-    strided_kernel(cplx<T> *__restrict__ cw, int nmain, int nxh, int np, int ny, int nz, int ydct, double scale,
+template <typename T, int N, int MODE, bool COS>
+__global__ void __launch_bounds__((SShape<T, N>::threads()))
+    strided_kernel(cplx<T> *__restrict__ cw, int nxh, int np, int ny, int ydct, double scale,
                    int zero_line, int xdct, int zdct, PoissonTables<T> tb) {
   using S = SShape<T, N>;
-  constexpr int E = LineShape<N>::E, NT = S::NT, TL = S::TL, TLB = TL + (EXTRA ? 1 : 0);
+  constexpr int E = LineShape<N>::E, NT = S::NT, TL = S::TL;
   extern __shared__ __align__(16) unsigned char smem_raw[];
   cplx<T> *buf = reinterpret_cast<cplx<T> *>(smem_raw);
-  cplx<T> *tw = buf + TLB * N, *dct = tw + N;
+  cplx<T> *tw = buf + TL * N, *dct = tw + N;
   const int tid = threadIdx.x;
   // line l of the block: a = kx, b = kz (y passes) or ky (z pass)
-  int l, t, a, b;
-  bool valid;
-  if (!EXTRA || tid < TL * NT) {
-    l = tid % TL;
-    t = tid / TL;
-    a = blockIdx.x * TL + l;
-    b = blockIdx.y;
-    valid = a < nxh;
-  } else {
-    // the extra line: g-th of the (nxh - nmain) x nplanes lines past the
-    // whole blocks (the host launches at least that many blocks)
-    const int nplanes = gridDim.y, ntail = (nxh - nmain) * nplanes;
-    const int g = blockIdx.y * gridDim.x + blockIdx.x;
-    l = TL;
-    t = tid - TL * NT;
-    valid = g < ntail;
-    const int gg = valid ? g : 0;
-    a = nmain + gg / nplanes;
-    b = gg % nplanes;
-  }
+  const int l = tid % TL, t = tid / TL, b = blockIdx.y;
+  const bool valid = (int)blockIdx.x * TL + l < nxh;
+  // lines past the last one compute on a copy of it (no load branches)
+  const int a = valid ? (int)blockIdx.x * TL + l : nxh - 1;
   constexpr bool ZL = ZPass<MODE>::value;
   const size_t se = ZL ? (size_t)np * ny : (size_t)np;
   const size_t base = ZL ? (size_t)b * np + a : (size_t)b * np * ny + a;
-  stage_table(tw, ZL ? tb.twz : tb.twy, N);
   // the cosine transform of this pass: y in the y passes, z in the z pass
   const bool dct_here = ZL ? (MODE == FFT_Z_SOLVE && COS && zdct != 0) : ydct != 0;
-  if (dct_here) stage_table(dct, ZL ? tb.dctz : tb.dcty, N);
+  const bool reorder_in = (MODE == FFT_Y_FWD || MODE == FFT_Z_SOLVE) && dct_here;
+  cplx<T> x[E];
+  load_strided<T, N>(cw + base, se, t, reorder_in, x);
+  // factors of this line's wavenumbers, for the divide after the transform
+  double lk[4] = {0.0, 0.0, 0.0, 0.0};
+  if constexpr (MODE == FFT_Z_SOLVE) {
+    lk[0] = tb.ky2[b];
+    lk[1] = tb.ty[b];
+    lk[2] = tb.kx2[a];
+    lk[3] = tb.tx[a];
+  }
   // the z pass reads tz and kz2 at its 16 points per thread: staged in LDS
   // with the twiddles instead of read from global memory after the FFT
   constexpr bool ZT = MODE == FFT_Z_SOLVE && !COS && SShape<T, N>::ZTAB;
   double *ztab = reinterpret_cast<double *>(dct + N);
-  if constexpr (ZT) {
-    for (int i = threadIdx.x; i < N; i += blockDim.x) {
-      ztab[i] = tb.tz[i];
-      ztab[N + i] = tb.kz2[i];
+  {
+    constexpr int NTHR = S::threads();
+    TableStage<cplx<T>, N, NTHR> s1, s2;
+    TableStage<double, ZT ? N : 1, NTHR> s3, s4;
+    s1.load(ZL ? tb.twz : tb.twy);
+    if (dct_here) s2.load(ZL ? tb.dctz : tb.dcty);
+    if constexpr (ZT) {
+      s3.load(tb.tz);
+      s4.load(tb.kz2);
     }
-  }
-  const bool reorder_in = (MODE == FFT_Y_FWD || MODE == FFT_Z_SOLVE) && dct_here;
-  cplx<T> x[E];
-#pragma unroll
-  for (int m = 0; m < E; ++m) {
-    const int p = t + m * NT;
-    const int row = reorder_in ? dct_row(p, N) : p;
-    x[m] = valid ? cw[base + (size_t)row * se] : cplx<T>{T(0), T(0)};
+    s1.store(tw);
+    if (dct_here) s2.store(dct);
+    if constexpr (ZT) {
+      s3.store(ztab);
+      s4.store(ztab + N);
+    }
   }
   if constexpr (MODE == FFT_Y_INV) {
     if (dct_here) {
@@ -500,7 +566,8 @@ __global__ void __launch_bounds__((SShape<T, N>::threads(EXTRA)))
 #pragma unroll
       for (int m = 0; m < E; ++m) {
         const int k = t + m * NT;
-        cm[m] = (valid && k > 0) ? cw[base + (size_t)(N - k) * se] : cplx<T>{T(0), T(0)};
+        cm[m] = cw[base + (size_t)(k > 0 ? N - k : 0) * se];
+        if (k == 0) cm[m] = cplx<T>{T(0), T(0)};
       }
       __syncthreads();   // dct table
 #pragma unroll
@@ -511,7 +578,7 @@ __global__ void __launch_bounds__((SShape<T, N>::threads(EXTRA)))
     }
   }
   __syncthreads();   // tables staged
-  const LdRows<T> ld{buf, TLB, l};
+  const LdRows<T> ld{buf, TL, l};
   fft_stages<T, N, MODE == FFT_Y_INV || MODE == FFT_Z_INV, 1>(x, t, ld, tw);
 
   if ((MODE == FFT_Y_FWD || MODE == FFT_Z_SOLVE) && dct_here) {
@@ -554,10 +621,10 @@ __global__ void __launch_bounds__((SShape<T, N>::threads(EXTRA)))
       }
       __syncthreads();
     }
-    if (valid && COS) {
-      const double ky2 = tb.ky2[b], tyv = tb.ty[b];
+    const double ky2 = lk[0], tyv = lk[1];
+    if constexpr (COS) {
       const int am = 2 * (nxh - 1) - a;
-      const double txr = tb.tx[a], kx2r = tb.kx2[a], txi = tb.tx[am], kx2i = tb.kx2[am];
+      const double txr = lk[3], kx2r = lk[2], txi = tb.tx[am], kx2i = tb.kx2[am];
 #pragma unroll
       for (int m = 0; m < E; ++m) {
         const int kz = t + m * NT;
@@ -575,9 +642,8 @@ __global__ void __launch_bounds__((SShape<T, N>::threads(EXTRA)))
           x[m] = cplx<T>{(T)(ar * fr + br * fi), (T)(ai * fr + bi * fi)};
         }
       }
-    } else if (valid) {
-      const double ky2 = tb.ky2[b], tyv = tb.ty[b];
-      const double txv = tb.tx[a], kx2 = tb.kx2[a];
+    } else {
+      const double txv = lk[3], kx2 = lk[2];
 #pragma unroll
       for (int m = 0; m < E; ++m) {
         const int kz = t + m * NT;
@@ -614,12 +680,7 @@ __global__ void __launch_bounds__((SShape<T, N>::threads(EXTRA)))
 
   if (valid) {
     const bool reorder_out = (MODE == FFT_Y_INV || MODE == FFT_Z_SOLVE) && dct_here;
-#pragma unroll
-    for (int m = 0; m < E; ++m) {
-      const int p = t + m * NT;
-      const int row = reorder_out ? dct_row(p, N) : p;
-      cw[base + (size_t)row * se] = x[m];
-    }
+    store_strided<T, N>(cw + base, se, t, reorder_out, x);
   }
 }
 
@@ -931,15 +992,23 @@ static void build_penta_factors(const Context &c, const PoissonPlan &P, const st
       }
 }
 
-// One thread per (kx, kz, system): forward elimination with the stored
-// multipliers (the scaled right-hand side read once, the eliminated values
-// written back), then the last 2x2 block and the back substitution.  The
-// (nx/2+1, :, nz/2+1) line is zeroed (poisson.f90:902-908).
+// One thread per real or imaginary part of (kx, kz, system), the two in
+// neighbouring lanes (they share the factors' loads): forward elimination with
+// the stored multipliers (the scaled right-hand side read once, the
+// eliminated values written back), then the last 2x2 block and the back
+// substitution.  The (nx/2+1, :, nz/2+1) line is zeroed (poisson.f90:902-908).
+// The chain along a line is serial and a 256x129x128 grid has only a
+// thousand wavefronts of lines, so the kernel's time is the latency of its
+// loads: rows are read PENTA_C at a time, the next group while the last one is
+// worked on (62 -> 45 us FP64, 55 -> 37 us FP32 on that grid; groups of 16: 60
+// and 39 us).
+constexpr int PENTA_C = 8;
 template <typename T>
 __global__ void __launch_bounds__(64) penta_y_kernel(cplx<T> *__restrict__ cw, const double *__restrict__ pf,
                                                      size_t stride, int nxh, int np, int ny, int nz, int nsys,
                                                      double scale) {
-  const int kx = blockIdx.x * blockDim.x + threadIdx.x;
+  const int tid = blockIdx.x * blockDim.x + threadIdx.x;
+  const int kx = tid >> 1, part = tid & 1;
   const int kz = blockIdx.y / nsys, par = blockIdx.y - kz * nsys;
   if (kx >= nxh) return;
   const int nh = ny / nsys, n = nh - 1;
@@ -947,45 +1016,93 @@ __global__ void __launch_bounds__(64) penta_y_kernel(cplx<T> *__restrict__ cw, c
   const size_t line = ((size_t)(kzp * nsys + par) * nh) * nxh + kx;
   const double *F1 = pf + line, *F2 = pf + stride + line, *RP = pf + 2 * stride + line;
   const double *A1 = pf + 3 * stride + line, *B1 = pf + 4 * stride + line;
-  auto at = [&](int m) -> cplx<T> & { return cw[((size_t)kz * ny + (nsys * m + par)) * np + kx]; };
+  T *const v = reinterpret_cast<T *>(cw) + 2 * (((size_t)kz * ny + par) * np + kx) + part;
+  const size_t sv = 2 * (size_t)nsys * np;        // row to row
   if (kx == nxh - 1 && kz == (nz >> 1)) {
-    for (int m = 0; m < nh; ++m) at(m) = cplx<T>{T(0), T(0)};
+    for (int m = 0; m < nh; ++m) v[(size_t)m * sv] = T(0);
     return;
   }
-  auto ld = [&](int m) {
-    const cplx<T> v = at(m);
-    return cplx<double>{(double)v.x * scale, (double)v.y * scale};
-  };
-  auto st = [&](int m, cplx<double> v) { at(m) = cplx<T>{(T)v.x, (T)v.y}; };
+  constexpr int C = PENTA_C;
   // forward: window (e0, e1, e2) = rows m, m+1, m+2
-  cplx<double> e0 = ld(0), e1 = ld(1), e2;
-  // unrolled so that the loads of later rows issue ahead of the chain
-#pragma unroll 4
-  for (int m = 0; m + 2 < nh; ++m) {
-    e2 = ld(m + 2);
-    const double s1 = F1[(size_t)m * nxh], s2 = F2[(size_t)m * nxh];
-    e1 = cplx<double>{e1.x - s1 * e0.x, e1.y - s1 * e0.y};
-    e2 = cplx<double>{e2.x - s2 * e0.x, e2.y - s2 * e0.y};
-    st(m, e0);
-    e0 = e1;
-    e1 = e2;
+  double e0 = (double)v[0] * scale, e1 = (double)v[sv] * scale;
+  {
+    T pv[C];
+    double p1[C], p2[C];
+    auto fetch = [&](int m0) {
+#pragma unroll
+      for (int q = 0; q < C; ++q) {
+        const int m = m0 + q < nh - 2 ? m0 + q : nh - 3;
+        pv[q] = v[(size_t)(m + 2) * sv];
+        p1[q] = F1[(size_t)m * nxh];
+        p2[q] = F2[(size_t)m * nxh];
+      }
+    };
+    fetch(0);
+    for (int m0 = 0; m0 + 2 < nh; m0 += C) {
+      T cv[C];
+      double c1[C], c2[C];
+#pragma unroll
+      for (int q = 0; q < C; ++q) {
+        cv[q] = pv[q];
+        c1[q] = p1[q];
+        c2[q] = p2[q];
+      }
+      fetch(m0 + C);
+#pragma unroll
+      for (int q = 0; q < C; ++q) {
+        const int m = m0 + q;
+        if (m + 2 >= nh) break;
+        double e2 = (double)cv[q] * scale;
+        e1 = e1 - c1[q] * e0;
+        e2 = e2 - c2[q] * e0;
+        v[(size_t)m * sv] = (T)e0;
+        e0 = e1;
+        e1 = e2;
+      }
+    }
   }
   // e0, e1 = rows n-1, n
   const double b1 = RP[(size_t)n * nxh], t1 = A1[(size_t)n * nxh];
-  cplx<double> xn = b1 != 0.0 ? cplx<double>{e1.x / b1 - t1 * e0.x, e1.y / b1 - t1 * e0.y} : cplx<double>{0.0, 0.0};
+  double xn = b1 != 0.0 ? e1 / b1 - t1 * e0 : 0.0;
   const double rp = RP[(size_t)(n - 1) * nxh], a1 = A1[(size_t)(n - 1) * nxh];
-  cplx<double> xm = {e0.x * rp - a1 * xn.x, e0.y * rp - a1 * xn.y};
-  st(n, xn);
-  st(n - 1, xm);
+  double xm = e0 * rp - a1 * xn;
+  v[(size_t)n * sv] = (T)xn;
+  v[(size_t)(n - 1) * sv] = (T)xm;
   // back substitution: (xm, xn) = rows i+1, i+2
-#pragma unroll 4
-  for (int i = nh - 3; i >= 0; --i) {
-    const cplx<T> v = at(i);
-    const double r = RP[(size_t)i * nxh], a = A1[(size_t)i * nxh], bb = B1[(size_t)i * nxh];
-    const cplx<double> x = {((double)v.x * r - a * xm.x) - bb * xn.x, ((double)v.y * r - a * xm.y) - bb * xn.y};
-    st(i, x);
-    xn = xm;
-    xm = x;
+  {
+    T pv[C];
+    double pr[C], pa[C], pb[C];
+    auto fetch = [&](int i0) {
+#pragma unroll
+      for (int q = 0; q < C; ++q) {
+        const int i = i0 - q > 0 ? i0 - q : 0;
+        pv[q] = v[(size_t)i * sv];
+        pr[q] = RP[(size_t)i * nxh];
+        pa[q] = A1[(size_t)i * nxh];
+        pb[q] = B1[(size_t)i * nxh];
+      }
+    };
+    fetch(nh - 3);
+    for (int i0 = nh - 3; i0 >= 0; i0 -= C) {
+      T cv[C];
+      double cr[C], ca[C], cb[C];
+#pragma unroll
+      for (int q = 0; q < C; ++q) {
+        cv[q] = pv[q];
+        cr[q] = pr[q];
+        ca[q] = pa[q];
+        cb[q] = pb[q];
+      }
+      fetch(i0 - C);
+#pragma unroll
+      for (int q = 0; q < C; ++q) {
+        if (i0 - q < 0) break;
+        const double x = ((double)cv[q] * cr[q] - ca[q] * xm) - cb[q] * xn;
+        v[(size_t)(i0 - q) * sv] = (T)x;
+        xn = xm;
+        xm = x;
+      }
+    }
   }
 }
 
@@ -1134,41 +1251,32 @@ void poisson_free(Context &c) {
 }
 
 template <typename T, int M>
-static void launch_x(bool fwd, T *rhs, cplx<T> *cw, int nlines, int np, int xdct, const PoissonTables<T> &tb,
+static void launch_x(bool fwd, T *rhs, cplx<T> *cw, int nlines, const PoissonPlan &P, const PoissonTables<T> &tb,
                      hipStream_t st) {
   using S = XShape<M>;
   const dim3 grid((nlines + S::TL - 1) / S::TL), block(S::TL * S::NT);
   const size_t sh = S::template lds<T>();
-  if (fwd) hipLaunchKernelGGL((r2c_x_kernel<T, M>), grid, block, sh, st, rhs, cw, nlines, np, xdct, tb);
-  else hipLaunchKernelGGL((c2r_x_kernel<T, M>), grid, block, sh, st, cw, rhs, nlines, np, xdct, tb);
+  if (fwd) hipLaunchKernelGGL((r2c_x_kernel<T, M>), grid, block, sh, st, rhs, cw, nlines, P.np, P.xdct, tb);
+  else hipLaunchKernelGGL((c2r_x_kernel<T, M>), grid, block, sh, st, cw, rhs, nlines, P.np, P.xdct, tb);
 }
 
-template <typename T, int N, int MODE, bool COS, bool EXTRA>
-static void launch_s1(const PoissonPlan &P, cplx<T> *cw, const PoissonTables<T> &tb, int nmain, int ncols,
-                      hipStream_t st) {
+template <typename T, int N, int MODE, bool COS>
+static void launch_s1(const PoissonPlan &P, cplx<T> *cw, const PoissonTables<T> &tb, hipStream_t st) {
   using S = SShape<T, N>;
-  const dim3 grid(ncols, ZPass<MODE>::value ? P.ny : P.nz), block(S::threads(EXTRA));
+  const dim3 grid((P.nxh + S::TL - 1) / S::TL, ZPass<MODE>::value ? P.ny : P.nz), block(S::threads());
   // poisson_010 zeroes the (nx/2+1, :, nz/2+1) line (poisson.f90:902-908); poisson_11x does not
   const int zero_line = MODE == FFT_Z_SOLVE && P.ydct && !P.xdct;
   const bool zt = MODE == FFT_Z_SOLVE && !COS && S::ZTAB;
-  hipLaunchKernelGGL((strided_kernel<T, N, MODE, COS, EXTRA>), grid, block, S::lds(EXTRA, zt), st, cw, nmain, P.nxh, P.np,
-                     P.ny, P.nz, P.ydct, P.scale, zero_line, P.xdct, P.zdct, tb);
+  hipLaunchKernelGGL((strided_kernel<T, N, MODE, COS>), grid, block, S::lds(zt), st, cw, P.nxh, P.np, P.ny, P.ydct,
+                     P.scale, zero_line, P.xdct, P.zdct, tb);
 }
 
 template <typename T, int N, int MODE>
 static void launch_s(const PoissonPlan &P, cplx<T> *cw, const PoissonTables<T> &tb, hipStream_t st) {
-  using S = SShape<T, N>;
-  const int ncols = P.nxh / S::TL, nmain = ncols * S::TL, rem = P.nxh - nmain;
   if constexpr (MODE == FFT_Z_SOLVE) {
-    // the cosine-x variant keeps whole blocks plus a partial last column
-    if (P.xdct) return launch_s1<T, N, MODE, true, false>(P, cw, tb, nmain, (P.nxh + S::TL - 1) / S::TL, st);
+    if (P.xdct) return launch_s1<T, N, MODE, true>(P, cw, tb, st);
   }
-  // FP32: one extra line per block when the blocks outnumber the remaining
-  // lines (measured at 256^3: 34/34/52 us against 43/43/63 for the y, y and z
-  // passes with a partial last column; FP64 measured slower with it, 65/66/89
-  // against 64/60/70 us)
-  if (sizeof(T) == 4 && rem > 0 && ncols >= rem) launch_s1<T, N, MODE, false, true>(P, cw, tb, nmain, ncols, st);
-  else launch_s1<T, N, MODE, false, false>(P, cw, tb, nmain, (P.nxh + S::TL - 1) / S::TL, st);
+  launch_s1<T, N, MODE, false>(P, cw, tb, st);
 }
 
 template <typename T, int MODE>
@@ -1187,17 +1295,17 @@ static bool dispatch_s(int N, const PoissonPlan &P, cplx<T> *cw, const PoissonTa
 }
 
 template <typename T>
-static bool dispatch_x(bool fwd, int M, T *rhs, cplx<T> *cw, int nlines, int np, int xdct, const PoissonTables<T> &tb,
+static bool dispatch_x(bool fwd, int M, T *rhs, cplx<T> *cw, int nlines, const PoissonPlan &P, const PoissonTables<T> &tb,
                        hipStream_t st) {
   switch (M) {
-    case 8: launch_x<T, 8>(fwd, rhs, cw, nlines, np, xdct, tb, st); return true;
-    case 16: launch_x<T, 16>(fwd, rhs, cw, nlines, np, xdct, tb, st); return true;
-    case 32: launch_x<T, 32>(fwd, rhs, cw, nlines, np, xdct, tb, st); return true;
-    case 64: launch_x<T, 64>(fwd, rhs, cw, nlines, np, xdct, tb, st); return true;
-    case 128: launch_x<T, 128>(fwd, rhs, cw, nlines, np, xdct, tb, st); return true;
-    case 256: launch_x<T, 256>(fwd, rhs, cw, nlines, np, xdct, tb, st); return true;
-    case 512: launch_x<T, 512>(fwd, rhs, cw, nlines, np, xdct, tb, st); return true;
-    case 1024: launch_x<T, 1024>(fwd, rhs, cw, nlines, np, xdct, tb, st); return true;
+    case 8: launch_x<T, 8>(fwd, rhs, cw, nlines, P, tb, st); return true;
+    case 16: launch_x<T, 16>(fwd, rhs, cw, nlines, P, tb, st); return true;
+    case 32: launch_x<T, 32>(fwd, rhs, cw, nlines, P, tb, st); return true;
+    case 64: launch_x<T, 64>(fwd, rhs, cw, nlines, P, tb, st); return true;
+    case 128: launch_x<T, 128>(fwd, rhs, cw, nlines, P, tb, st); return true;
+    case 256: launch_x<T, 256>(fwd, rhs, cw, nlines, P, tb, st); return true;
+    case 512: launch_x<T, 512>(fwd, rhs, cw, nlines, P, tb, st); return true;
+    case 1024: launch_x<T, 1024>(fwd, rhs, cw, nlines, P, tb, st); return true;
     default: return false;
   }
 }
@@ -1233,7 +1341,7 @@ int poisson_run(const Context &c, T *rhs, void *work, size_t bytes, hipStream_t 
   else tb = P->t32;
   const int nlines = P->ny * P->nz, M = P->nx / 2;
   // sizes were checked by poisson_setup: every dispatch below finds its case
-  bool ok = dispatch_x<T>(true, M, rhs, cw, nlines, P->np, P->xdct, tb, st);
+  bool ok = dispatch_x<T>(true, M, rhs, cw, nlines, *P, tb, st);
   ok = ok && dispatch_s<T, FFT_Y_FWD>(P->ny, *P, cw, tb, st);
   if (P->xdct && !P->ydct) {
     // poisson_100: forward z, the pairwise split and divide, inverse z
@@ -1248,16 +1356,16 @@ int poisson_run(const Context &c, T *rhs, void *work, size_t bytes, hipStream_t 
     // stretched y: z transform, pentadiagonal solves along y, inverse z
     ok = ok && dispatch_s<T, FFT_Z_FWD>(P->nz, *P, cw, tb, st);
     if (ok) {
-      const dim3 grid((P->nxh + 63) / 64, P->ystret * P->nz), block(64);
-      hipLaunchKernelGGL((penta_y_kernel<T>), grid, block, 0, st, cw, P->pf, P->pf_stride, P->nxh, P->np, P->ny,
-                         P->nz, P->ystret, P->scale);
+      const dim3 grid((2 * P->nxh + 63) / 64, P->ystret * P->nz), block(64);
+      hipLaunchKernelGGL((penta_y_kernel<T>), grid, block, 0, st, cw, P->pf, P->pf_stride, P->nxh, P->np,
+                         P->ny, P->nz, P->ystret, P->scale);
     }
     ok = ok && dispatch_s<T, FFT_Z_INV>(P->nz, *P, cw, tb, st);
   } else {
     ok = ok && dispatch_s<T, FFT_Z_SOLVE>(P->nz, *P, cw, tb, st);
   }
   ok = ok && dispatch_s<T, FFT_Y_INV>(P->ny, *P, cw, tb, st);
-  ok = ok && dispatch_x<T>(false, M, rhs, cw, nlines, P->np, P->xdct, tb, st);
+  ok = ok && dispatch_x<T>(false, M, rhs, cw, nlines, *P, tb, st);
   if (!ok) return fail(X3D_ERR_UNSUPPORTED, "Poisson: no FFT kernel for this size");
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return fail(X3D_ERR_HIP, std::string("poisson launch: ") + hipGetErrorString(e));
@@ -1338,7 +1446,7 @@ int fft3d(Context &c, bool forward, const void *in, void *out, hipStream_t st) {
   const unsigned nb = (unsigned)std::min<size_t>((nout + 255) / 256, 65535u * 8u);
   bool ok;
   if (forward) {
-    ok = dispatch_x<T>(true, M, const_cast<T *>(static_cast<const T *>(in)), cw, nlines, Q.np, 0, tb, st);
+    ok = dispatch_x<T>(true, M, const_cast<T *>(static_cast<const T *>(in)), cw, nlines, Q, tb, st);
     ok = ok && dispatch_s<T, FFT_Y_FWD>(Q.ny, Q, cw, tb, st);
     ok = ok && dispatch_s<T, FFT_Z_FWD>(Q.nz, Q, cw, tb, st);
     if (ok)
@@ -1349,7 +1457,7 @@ int fft3d(Context &c, bool forward, const void *in, void *out, hipStream_t st) {
                        Q.ny, Q.nz, Q.nxh, Q.np);
     ok = dispatch_s<T, FFT_Z_INV>(Q.nz, Q, cw, tb, st);
     ok = ok && dispatch_s<T, FFT_Y_INV>(Q.ny, Q, cw, tb, st);
-    ok = ok && dispatch_x<T>(false, M, static_cast<T *>(out), cw, nlines, Q.np, 0, tb, st);
+    ok = ok && dispatch_x<T>(false, M, static_cast<T *>(out), cw, nlines, Q, tb, st);
   }
   if (!ok) return fail(X3D_ERR_UNSUPPORTED, "FFT: no kernel for this size");
   hipError_t e = hipGetLastError();
