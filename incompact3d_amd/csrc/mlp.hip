@@ -127,13 +127,7 @@ struct Fwd16 {
   bf16x4 h[3][4];   // inputs of layers 2, 3, 4
 };
 
-// At[t]: this lane's operand of tile t (a register array, or GlobalTiles)
-struct GlobalTiles {
-  const bf16x4 *p;
-  int lane;
-  __device__ __forceinline__ bf16x4 operator[](int t) const { return p[t * 64 + lane]; }
-};
-
+// At[t]: this lane's operand of tile t (a register array)
 template <typename ACC>
 __device__ __forceinline__ f32x4 forward16(const ACC &At, const float *__restrict__ bias, bf16x4 x, int kb,
                                            Fwd16 &F) {
@@ -218,7 +212,7 @@ __global__ void __launch_bounds__(256) mlp_fwdbwd_kernel(const bf16x4 *__restric
                                                          const float *__restrict__ tgt, int n, bf16x4 *__restrict__ act,
                                                          float *__restrict__ loss_part) {
   __shared__ __align__(16) float sb[208];
-  __shared__ float red[256];
+  __shared__ float red[4];
   for (int i = threadIdx.x; i < 208; i += blockDim.x) sb[i] = bias[i];
   __syncthreads();
   const int lane = threadIdx.x & 63, kb = lane >> 4;
@@ -226,12 +220,17 @@ __global__ void __launch_bounds__(256) mlp_fwdbwd_kernel(const bf16x4 *__restric
   const int ntiles = (n + 15) / 16;
   const float gscale = 2.0f / (6.0f * (float)n);
   float lsum = 0.0f;
+  // every operand tile in registers from the start: a batch has a wave or two
+  // a SIMD, and a load in front of each MFMA was most of a tile's time
+  bf16x4 At[MLP_NTILES];
+#pragma unroll
+  for (int t = 0; t < MLP_NTILES; ++t) At[t] = tiles[t * 64 + lane];
   for (int tile = wave; tile < ntiles; tile += nwaves) {
     const int pt = tile * 16 + (lane & 15);
     const bool valid = pt < n;
     const bf16x4 xin = load_features(x, pt, n, kb);
     Fwd16 F;
-    const f32x4 y = forward16(GlobalTiles{tiles, lane}, sb, xin, kb, F);
+    const f32x4 y = forward16(At, sb, xin, kb, F);
     // dL/dy (rows 4kb..4kb+3 = outputs)
     f32x4 dy;
 #pragma unroll
@@ -262,7 +261,7 @@ __global__ void __launch_bounds__(256) mlp_fwdbwd_kernel(const bf16x4 *__restric
     bf16x4 gz[4];
 #pragma unroll
     for (int mt = 0; mt < 4; ++mt) {
-      f32x4 dh = mfma(tiles[(T_AT4 + mt) * 64 + lane], g, zero);
+      f32x4 dh = mfma(At[T_AT4 + mt], g, zero);
       bf16x4 q;
 #pragma unroll
       for (int i = 0; i < 4; ++i) q[i] = to_bf16(dh[i] * gelu_grad(F.z[2][mt][i]));
@@ -278,7 +277,7 @@ __global__ void __launch_bounds__(256) mlp_fwdbwd_kernel(const bf16x4 *__restric
       for (int mt = 0; mt < 4; ++mt) {
         f32x4 dh = zero;
 #pragma unroll
-        for (int kt = 0; kt < 4; ++kt) dh = mfma(tiles[(base + 4 * mt + kt) * 64 + lane], gz[kt], dh);
+        for (int kt = 0; kt < 4; ++kt) dh = mfma(At[base + 4 * mt + kt], gz[kt], dh);
         bf16x4 q;
 #pragma unroll
         for (int i = 0; i < 4; ++i) q[i] = to_bf16(dh[i] * gelu_grad(F.z[layer - 1][mt][i]));
@@ -289,11 +288,13 @@ __global__ void __launch_bounds__(256) mlp_fwdbwd_kernel(const bf16x4 *__restric
       for (int mt = 0; mt < 4; ++mt) gz[mt] = nz[mt];
     }
   }
-  red[threadIdx.x] = lsum;
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) lsum += __shfl_xor(lsum, off);
+  if (lane == 0) red[threadIdx.x >> 6] = lsum;
   __syncthreads();
   if (threadIdx.x == 0) {
     float s = 0.0f;
-    for (int i = 0; i < (int)blockDim.x; ++i) s += red[i];
+    for (int i = 0; i < (int)blockDim.x / 64; ++i) s += red[i];
     loss_part[blockIdx.x] = s;
   }
 }
@@ -308,115 +309,184 @@ __device__ __forceinline__ short act_at(const bf16x4 *__restrict__ act, int pt, 
   return r[col];
 }
 
-__global__ void __launch_bounds__(256) mlp_wgrad_kernel(const bf16x4 *__restrict__ act, int n,
-                                                        float *__restrict__ partial) {
-  const int layer = blockIdx.y;   // 0..3
+constexpr int WG_WAVES = 4;
+
+// Rows past the batch repeat its last one with a zero dZ.
+template <int LAYER>
+__device__ __forceinline__ void wgrad_layer(const bf16x4 *__restrict__ act, int n, float *__restrict__ out,
+                                            float (&red)[WG_WAVES][MLP_NH * MLP_NH + MLP_NH]) {
   // BF16 column offsets of dZ_l and H_{l-1} in a row, their widths
-  const int dcol = layer == 0 ? 4 * ACT_D1 : layer == 1 ? 4 * ACT_D2 : layer == 2 ? 4 * ACT_D3 : 4 * ACT_D4;
-  const int hcol = layer == 0 ? 4 * ACT_H0 : layer == 1 ? 4 * ACT_H1 : layer == 2 ? 4 * ACT_H2 : 4 * ACT_H3;
-  const int M = layer == 3 ? MLP_NOUT : MLP_NH, K = layer == 0 ? MLP_NIN : MLP_NH;
-  const int MT = layer == 3 ? 1 : 4, KT = layer == 0 ? 1 : 4;
-  const int woff = layer == 0 ? OFF_W1 : layer == 1 ? OFF_W2 : layer == 2 ? OFF_W3 : OFF_W4;
-  const int boff = layer == 0 ? OFF_B1 : layer == 1 ? OFF_B2 : layer == 2 ? OFF_B3 : OFF_B4;
+  constexpr int dcol = 4 * (LAYER == 0 ? ACT_D1 : LAYER == 1 ? ACT_D2 : LAYER == 2 ? ACT_D3 : ACT_D4);
+  constexpr int hcol = 4 * (LAYER == 0 ? ACT_H0 : LAYER == 1 ? ACT_H1 : LAYER == 2 ? ACT_H2 : ACT_H3);
+  constexpr int M = LAYER == 3 ? MLP_NOUT : MLP_NH, K = LAYER == 0 ? MLP_NIN : MLP_NH;
+  constexpr int MT = LAYER == 3 ? 1 : 4, KT = LAYER == 0 ? 1 : 4;
+  constexpr int woff = LAYER == 0 ? OFF_W1 : LAYER == 1 ? OFF_W2 : LAYER == 2 ? OFF_W3 : OFF_W4;
+  constexpr int boff = LAYER == 0 ? OFF_B1 : LAYER == 1 ? OFF_B2 : LAYER == 2 ? OFF_B3 : OFF_B4;
   const int lane = threadIdx.x & 63, kb = lane >> 4, r16 = lane & 15;
-  const int wv = threadIdx.x >> 6, nwv = blockDim.x >> 6;
+  const int wv = threadIdx.x >> 6;
   const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
-  f32x4 acc[4][4];
+  f32x4 acc[MT][KT];
+  float bacc[MT];
 #pragma unroll
-  for (int a = 0; a < 4; ++a)
+  for (int a = 0; a < MT; ++a) {
+    bacc[a] = 0.f;
 #pragma unroll
-    for (int b = 0; b < 4; ++b) acc[a][b] = zero;
-  float bacc[4] = {0.f, 0.f, 0.f, 0.f};
+    for (int b = 0; b < KT; ++b) acc[a][b] = zero;
+  }
   const int nch = (n + 15) / 16;
-  for (int ch = blockIdx.x * nwv + wv; ch < nch; ch += gridDim.x * nwv) {
-    const int p0 = ch * 16;
-    bf16x4 A[4], B[4];
+  for (int ch = blockIdx.x * WG_WAVES + wv; ch < nch; ch += gridDim.x * WG_WAVES) {
+    bf16x4 A[MT], B[KT];
 #pragma unroll
-    for (int mt = 0; mt < 4; ++mt) {
+    for (int j = 0; j < 4; ++j) {
+      const int pt = ch * 16 + 4 * kb + j;
+      const int pl = pt < n ? pt : n - 1;
 #pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        const int pt = p0 + 4 * kb + j;
-        A[mt][j] = (mt < MT && pt < n) ? act_at(act, pt, dcol + 16 * mt + r16) : (short)0;
-        B[mt][j] = (mt < KT && pt < n) ? act_at(act, pt, hcol + 16 * mt + r16) : (short)0;
+      for (int mt = 0; mt < MT; ++mt) {
+        const short d = act_at(act, pl, dcol + 16 * mt + r16);
+        A[mt][j] = pt < n ? d : (short)0;
       }
+#pragma unroll
+      for (int kt = 0; kt < KT; ++kt) B[kt][j] = act_at(act, pl, hcol + 16 * kt + r16);
     }
 #pragma unroll
-    for (int mt = 0; mt < 4; ++mt)
+    for (int mt = 0; mt < MT; ++mt) {
 #pragma unroll
-      for (int kt = 0; kt < 4; ++kt)
-        if (mt < MT && kt < KT) acc[mt][kt] = mfma(A[mt], B[kt], acc[mt][kt]);
-    // bias: lanes with kb == 0 sum dZ[pt][16 mt + r16] over the chunk
-    if (kb == 0) {
+      for (int kt = 0; kt < KT; ++kt) acc[mt][kt] = mfma(A[mt], B[kt], acc[mt][kt]);
+      // bias: this lane's four points of output 16 mt + r16
 #pragma unroll
-      for (int mt = 0; mt < 4; ++mt) {
-        if (mt < MT) {
-          float s = 0.f;
-          for (int q = 0; q < 16; ++q) {
-            const int pt = p0 + q;
-            if (pt < n) s += from_bf16(act_at(act, pt, dcol + 16 * mt + r16));
-          }
-          bacc[mt] += s;
-        }
-      }
+      for (int j = 0; j < 4; ++j) bacc[mt] += from_bf16(A[mt][j]);
     }
   }
   // sum the block's waves through LDS, write the block's partial
-  __shared__ float red[4][64 * 64 + 64];
 #pragma unroll
-  for (int mt = 0; mt < 4; ++mt)
+  for (int mt = 0; mt < MT; ++mt) {
 #pragma unroll
-    for (int kt = 0; kt < 4; ++kt)
+    for (int kt = 0; kt < KT; ++kt)
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const int m = 16 * mt + 4 * kb + i, k = 16 * kt + r16;
-        if (mt < MT && kt < KT) red[wv][m * 64 + k] = acc[mt][kt][i];
-      }
-  if (kb == 0) {
-#pragma unroll
-    for (int mt = 0; mt < 4; ++mt)
-      if (mt < MT) red[wv][4096 + 16 * mt + r16] = bacc[mt];
+      for (int i = 0; i < 4; ++i) red[wv][(16 * mt + 4 * kb + i) * MLP_NH + 16 * kt + r16] = acc[mt][kt][i];
+    bacc[mt] += __shfl_xor(bacc[mt], 16);
+    bacc[mt] += __shfl_xor(bacc[mt], 32);
+    if (kb == 0) red[wv][MLP_NH * MLP_NH + 16 * mt + r16] = bacc[mt];
   }
   __syncthreads();
-  float *out = partial + (size_t)blockIdx.x * MLP_NPARAM;
-  for (int idx = threadIdx.x; idx < M * K + M; idx += blockDim.x) {
+  for (int idx = threadIdx.x; idx < M * K + M; idx += WG_WAVES * 64) {
     int src, dst;
     if (idx < M * K) {
       const int m = idx / K, k = idx - m * K;
-      src = m * 64 + k;
+      src = m * MLP_NH + k;
       dst = woff + idx;
     } else {
-      src = 4096 + (idx - M * K);
+      src = MLP_NH * MLP_NH + (idx - M * K);
       dst = boff + (idx - M * K);
     }
     float s = 0.f;
-    for (int w = 0; w < nwv; ++w) s += red[w][src];
+#pragma unroll
+    for (int w = 0; w < WG_WAVES; ++w) s += red[w][src];
     out[dst] = s;
   }
 }
 
-// ---------------------------------------------------------------- Adam
-__global__ void mlp_adam_kernel(const float *__restrict__ partial, int nblk, float *__restrict__ grad,
-                                float *__restrict__ p, float *__restrict__ m, float *__restrict__ v, float lr,
-                                float b1, float b2, float eps, float c1, float c2, int apply) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= MLP_NPARAM) return;
-  float g = 0.f;
-  for (int b = 0; b < nblk; ++b) g += partial[(size_t)b * MLP_NPARAM + i];
-  grad[i] = g;
-  if (!apply) return;
-  const float mm = b1 * m[i] + (1.f - b1) * g;
-  const float vv = b2 * v[i] + (1.f - b2) * g * g;
-  m[i] = mm;
-  v[i] = vv;
-  p[i] = p[i] - lr * (mm / c1) / (sqrtf(vv / c2) + eps);
+__global__ void __launch_bounds__(WG_WAVES * 64) mlp_wgrad_kernel(const bf16x4 *__restrict__ act, int n,
+                                                                 float *__restrict__ partial) {
+  __shared__ float red[WG_WAVES][MLP_NH * MLP_NH + MLP_NH];
+  float *out = partial + (size_t)blockIdx.x * MLP_NPARAM;
+  switch (blockIdx.y) {
+    case 0: wgrad_layer<0>(act, n, out, red); break;
+    case 1: wgrad_layer<1>(act, n, out, red); break;
+    case 2: wgrad_layer<2>(act, n, out, red); break;
+    default: wgrad_layer<3>(act, n, out, red); break;
+  }
 }
 
-__global__ void mlp_loss_kernel(const float *__restrict__ part, int nblk, float *__restrict__ out, float inv) {
-  if (threadIdx.x == 0 && blockIdx.x == 0) {
-    float s = 0.f;
-    for (int b = 0; b < nblk; ++b) s += part[b];
-    out[0] = s * inv;
+// ---------------------------------------------------------------- Adam
+// Adds the blocks' partial gradients, updates the parameters and writes them
+// into the operand tiles; block 0 adds up the loss as well.  A block takes
+// ADAM_P parameters with ADAM_G threads each, every thread a strided set of
+// the partials and four sums in flight, so the reduction is spread over the
+// chip (one thread a parameter walked 256 partials one after the other: 60 us
+// of a training step on 8192 points; now 6 us with the packing and the loss,
+// which were kernels of 6 us each).
+constexpr int ADAM_P = 32, ADAM_G = 8;
+
+// Position of parameter i in the BF16 operand tiles (in shorts): its entry in
+// the forward tiles, and in the transposed ones (-1: none, layer 1).
+struct TileSlot {
+  int fwd, bwd;
+};
+__device__ __forceinline__ int tile_entry(int base, int kt_count, int row, int col) {
+  const int t = base + (row >> 4) * kt_count + (col >> 4);
+  return ((t * 64) + ((col & 15) >> 2) * 16 + (row & 15)) * 4 + (col & 3);
+}
+__device__ __forceinline__ TileSlot tile_slot(int i) {
+  if (i < OFF_B1) return {tile_entry(T_A1, 1, i / MLP_NIN, i % MLP_NIN), -1};
+  if (i >= OFF_W2 && i < OFF_B2) {
+    const int r = (i - OFF_W2) >> 6, c = (i - OFF_W2) & 63;
+    return {tile_entry(T_A2, 4, r, c), tile_entry(T_AT2, 4, c, r)};
   }
+  if (i >= OFF_W3 && i < OFF_B3) {
+    const int r = (i - OFF_W3) >> 6, c = (i - OFF_W3) & 63;
+    return {tile_entry(T_A3, 4, r, c), tile_entry(T_AT3, 4, c, r)};
+  }
+  if (i >= OFF_W4 && i < OFF_B4) {
+    const int r = (i - OFF_W4) >> 6, c = (i - OFF_W4) & 63;
+    return {tile_entry(T_A4, 4, r, c), tile_entry(T_AT4, 1, c, r)};
+  }
+  return {-1, -1};
+}
+__device__ __forceinline__ int bias_slot(int i) {
+  if (i >= OFF_B1 && i < OFF_W2) return i - OFF_B1;
+  if (i >= OFF_B2 && i < OFF_W3) return 64 + i - OFF_B2;
+  if (i >= OFF_B3 && i < OFF_W4) return 128 + i - OFF_B3;
+  if (i >= OFF_B4) return 192 + i - OFF_B4;
+  return -1;
+}
+
+__global__ void __launch_bounds__(ADAM_P *ADAM_G)
+    mlp_adam_kernel(const float *__restrict__ partial, int nblk, const float *__restrict__ loss_part, int nloss,
+                    float loss_scale, float *__restrict__ loss, float *__restrict__ grad, float *__restrict__ p,
+                    float *__restrict__ m, float *__restrict__ v, short *__restrict__ tiles,
+                    float *__restrict__ bias, float lr, float b1, float b2, float eps, float c1, float c2,
+                    int apply) {
+  const int q = threadIdx.x % ADAM_P, g = threadIdx.x / ADAM_P;
+  const int i = blockIdx.x * ADAM_P + q;
+  const int il = i < MLP_NPARAM ? i : MLP_NPARAM - 1;
+  float s[4] = {0.f, 0.f, 0.f, 0.f};
+  int b = g;
+  for (; b + 3 * ADAM_G < nblk; b += 4 * ADAM_G) {
+#pragma unroll
+    for (int k = 0; k < 4; ++k) s[k] += partial[(size_t)(b + k * ADAM_G) * MLP_NPARAM + il];
+  }
+  for (; b < nblk; b += ADAM_G) s[0] += partial[(size_t)b * MLP_NPARAM + il];
+  __shared__ float red[ADAM_G][ADAM_P], rl[ADAM_P * ADAM_G];
+  red[g][q] = (s[0] + s[1]) + (s[2] + s[3]);
+  if (blockIdx.x == 0) {
+    float l = 0.f;
+    for (int k = threadIdx.x; k < nloss; k += blockDim.x) l += loss_part[k];
+    rl[threadIdx.x] = l;
+  }
+  __syncthreads();
+  if (blockIdx.x == 0 && threadIdx.x == ADAM_P * ADAM_G - 1) {
+    float l = 0.f;
+    for (int k = 0; k < ADAM_P * ADAM_G; ++k) l += rl[k];
+    loss[0] = l * loss_scale;
+  }
+  if (g != 0 || i >= MLP_NPARAM) return;
+  float gr = 0.f;
+#pragma unroll
+  for (int k = 0; k < ADAM_G; ++k) gr += red[k][q];
+  grad[i] = gr;
+  if (!apply) return;
+  const float mm = b1 * m[i] + (1.f - b1) * gr;
+  const float vv = b2 * v[i] + (1.f - b2) * gr * gr;
+  m[i] = mm;
+  v[i] = vv;
+  const float w = p[i] - lr * (mm / c1) / (sqrtf(vv / c2) + eps);
+  p[i] = w;
+  const TileSlot ts = tile_slot(i);
+  if (ts.fwd >= 0) tiles[ts.fwd] = to_bf16(w);
+  if (ts.bwd >= 0) tiles[ts.bwd] = to_bf16(w);
+  const int bs = bias_slot(i);
+  if (bs >= 0) bias[bs] = w;
 }
 
 // ---------------------------------------------------------------- closure on the LES fields
@@ -529,6 +599,10 @@ int mlp_alloc(MlpDev *&out) {
   if (e == hipSuccess) e = hipMemset(M->m, 0, sizeof(float) * MLP_NPARAM);
   if (e == hipSuccess) e = hipMemset(M->v, 0, sizeof(float) * MLP_NPARAM);
   if (e == hipSuccess) e = hipMemset(M->master, 0, sizeof(float) * MLP_NPARAM);
+  // operands of the zero weights: the padding of the tiles stays zero, Adam
+  // writes the entries of parameters only
+  if (e == hipSuccess) e = hipMemset(M->tiles, 0, sizeof(bf16x4) * MLP_NTILES * 64);
+  if (e == hipSuccess) e = hipMemset(M->bias, 0, sizeof(float) * 208);
   if (e != hipSuccess) {
     mlp_free(M);
     return fail(X3D_ERR_HIP, std::string("mlp alloc: ") + hipGetErrorString(e));
@@ -587,11 +661,15 @@ int mlp_train_batch(MlpDev *M, const float *x, const float *t, int n, int apply,
     M->act_cap = n;
   }
   const int ntiles = (n + 15) / 16;
-  const int fb = std::min((ntiles + 3) / 4, MLP_WG_BLOCKS);
-  hipLaunchKernelGGL(mlp_fwdbwd_kernel, dim3(fb), dim3(256), 0, st, M->tiles, M->bias, x, t, n, M->act, M->loss);
-  hipLaunchKernelGGL(mlp_loss_kernel, dim3(1), dim3(64), 0, st, M->loss, fb, M->loss + MLP_WG_BLOCKS,
-                     1.0f / (6.0f * (float)n));
-  hipLaunchKernelGGL(mlp_wgrad_kernel, dim3(MLP_WG_BLOCKS, 4), dim3(256), 0, st, M->act, n, M->partial);
+  // two waves a block while that gives every block its own CU, four beyond
+  const int fw = ntiles <= 2 * MLP_WG_BLOCKS ? 2 : 4;
+  const int fb = std::min((ntiles + fw - 1) / fw, MLP_WG_BLOCKS);
+  hipLaunchKernelGGL(mlp_fwdbwd_kernel, dim3(fb), dim3(64 * fw), 0, st, M->tiles, M->bias, x, t, n, M->act, M->loss);
+  // two 16-point chunks for each of a block's four waves, up to MLP_WG_BLOCKS
+  // blocks a layer: a block's partial gradient costs as much to write and add
+  // up as a few chunks cost to compute
+  const int wb = std::max(1, std::min((ntiles + 7) / 8, MLP_WG_BLOCKS));
+  hipLaunchKernelGGL(mlp_wgrad_kernel, dim3(wb, 4), dim3(256), 0, st, M->act, n, M->partial);
   float c1 = 1.f, c2 = 1.f;
   const float b1 = 0.9f, b2 = 0.999f;
   if (apply) {
@@ -599,10 +677,11 @@ int mlp_train_batch(MlpDev *M, const float *x, const float *t, int n, int apply,
     c1 = 1.f - powf(b1, (float)M->step);
     c2 = 1.f - powf(b2, (float)M->step);
   }
-  hipLaunchKernelGGL(mlp_adam_kernel, dim3((MLP_NPARAM + 255) / 256), dim3(256), 0, st, M->partial, MLP_WG_BLOCKS,
-                     M->grad, M->master, M->m, M->v, lr, b1, b2, 1e-8f, c1, c2, apply);
+  hipLaunchKernelGGL(mlp_adam_kernel, dim3((MLP_NPARAM + ADAM_P - 1) / ADAM_P), dim3(ADAM_P * ADAM_G), 0, st,
+                     M->partial, wb, M->loss, fb, 1.0f / (6.0f * (float)n), M->loss + MLP_WG_BLOCKS, M->grad,
+                     M->master, M->m, M->v, reinterpret_cast<short *>(M->tiles), M->bias, lr, b1, b2, 1e-8f, c1, c2,
+                     apply);
   X3D_HIP(hipGetLastError());
-  if (apply) X3D_TRY(mlp_repack(M, st));
   if (loss_host) {
     X3D_HIP(hipMemcpyAsync(loss_host, M->loss + MLP_WG_BLOCKS, sizeof(float), hipMemcpyDeviceToHost, st));
     X3D_HIP(hipStreamSynchronize(st));

@@ -78,6 +78,7 @@ struct x3d_solver {
   bool plain = false;          // ... and the step is AB3 on a periodic box
   size_t n = 0;
   int nx = 0, ny = 0, nz = 0;
+  void *slab = nullptr;        // the allocation that holds the arrays below (diag, w64, lesw, nfb, ycoord: own)
   double *u64[3] = {nullptr, nullptr, nullptr};   // current velocity (FP64)
   float *u32[3] = {nullptr, nullptr, nullptr};    // its FP32 copy (precision 1)
   double *u64b[3] = {nullptr, nullptr, nullptr};  // next-step buffers (AB3 writes here,
@@ -727,54 +728,56 @@ int tgv_stats(Context &c, x3d_solver *S, double out4[4]) {
 int alloc_solver(Context &c, x3d_solver *S) {
   const size_t n = S->n;
   const size_t es = S->precision == 0 ? 8 : 4;
-  for (int i = 0; i < 3; ++i) {
-    X3D_HIP(hipMalloc(&S->u64[i], n * 8));
-    if (S->precision == 1) X3D_HIP(hipMalloc(&S->u32[i], n * 4));
-    if (S->fused) {
-      // (the general FP32 step updates u64 in place)
-      if (S->precision == 0 || S->plain) X3D_HIP(hipMalloc(&S->u64b[i], n * 8));
-      if (S->precision == 1) X3D_HIP(hipMalloc(&S->u32b[i], n * 4));
-    }
-    if (S->split) X3D_HIP(hipMalloc(&S->res[i], n * 4));
-    for (int j = 0; j < 3; ++j) {
-      X3D_HIP(hipMalloc(&S->hist[i][j], n * es));
-      X3D_HIP(hipMemsetAsync(S->hist[i][j], 0, n * es, c.stream));
-    }
-  }
   const size_t np = (size_t)c.nxm * c.nym * c.nzm;
   const size_t nw = n > np ? n : np;
-  for (int i = 0; i < 5; ++i) X3D_HIP(hipMalloc(&S->w[i], nw * es));
-  X3D_HIP(hipMalloc(&S->partial, 8 * 1024 * sizeof(double)));
+  // one allocation holds every array (a hipMalloc each took most of the time
+  // of creating a solver)
+  struct Part {
+    void **p;
+    size_t bytes;
+  };
+  std::vector<Part> parts;
+  auto part = [&](auto **p, size_t bytes) { parts.push_back({(void **)p, (bytes + 255) / 256 * 256}); };
+  for (int i = 0; i < 3; ++i) {
+    part(&S->u64[i], n * 8);
+    if (S->precision == 1) part(&S->u32[i], n * 4);
+    if (S->fused) {
+      // (the general FP32 step updates u64 in place)
+      if (S->precision == 0 || S->plain) part(&S->u64b[i], n * 8);
+      if (S->precision == 1) part(&S->u32b[i], n * 4);
+    }
+    if (S->split) part(&S->res[i], n * 4);
+    for (int j = 0; j < 3; ++j) part(&S->hist[i][j], n * es);
+  }
+  for (int i = 0; i < 5; ++i) part(&S->w[i], nw * es);
+  part(&S->partial, 8 * 1024 * sizeof(double));
   // div u* partials: RED_BLOCKS pairs (per-operator step) or one pair per
-  // block of the fused z divergence sweep (at most nx * ny / 16 blocks)
-  X3D_HIP(hipMalloc(&S->divp, 2 * ((size_t)S->nx * S->ny + 1024) * sizeof(double)));
-  X3D_HIP(hipMalloc(&S->red, 8 * sizeof(double)));
-  if (S->wall1 || S->walln) X3D_HIP(hipMalloc(&S->wallg, 4 * (size_t)S->nx * S->nz * sizeof(double)));
+  // block of the fused z divergence sweep (at most nx * ny / 8 blocks and a
+  // partly filled one per plane)
+  part(&S->divp, 2 * ((size_t)S->nx * S->ny + 1024) * sizeof(double));
+  part(&S->red, 8 * sizeof(double));
+  if (S->wall1 || S->walln) part(&S->wallg, 4 * (size_t)S->nx * S->nz * sizeof(double));
+  size_t total = 0;
+  for (const Part &q : parts) total += q.bytes;
+  X3D_HIP(hipMalloc(&S->slab, total));
+  char *at = static_cast<char *>(S->slab);
+  for (const Part &q : parts) {
+    *q.p = at;
+    at += q.bytes;
+  }
+  for (int i = 0; i < 3; ++i)
+    for (int j = 0; j < 3; ++j) X3D_HIP(hipMemsetAsync(S->hist[i][j], 0, n * es, c.stream));
   X3D_HIP(hipStreamSynchronize(c.stream));
   return X3D_OK;
 }
 
 void free_solver(x3d_solver *S) {
-  for (int i = 0; i < 3; ++i) {
-    if (S->u64[i]) (void)hipFree(S->u64[i]);
-    if (S->u32[i]) (void)hipFree(S->u32[i]);
-    if (S->u64b[i]) (void)hipFree(S->u64b[i]);
-    if (S->u32b[i]) (void)hipFree(S->u32b[i]);
-    if (S->res[i]) (void)hipFree(S->res[i]);
-    for (int j = 0; j < 3; ++j)
-      if (S->hist[i][j]) (void)hipFree(S->hist[i][j]);
-  }
-  for (int i = 0; i < 5; ++i)
-    if (S->w[i]) (void)hipFree(S->w[i]);
+  if (S->slab) (void)hipFree(S->slab);
   for (int i = 0; i < 4; ++i)
     if (S->w64[i]) (void)hipFree(S->w64[i]);
   if (S->diag) (void)hipFree(S->diag);
   if (S->lesw) (void)hipFree(S->lesw);
   if (S->nfb) (void)hipFree(S->nfb);
-  if (S->partial) (void)hipFree(S->partial);
-  if (S->divp) (void)hipFree(S->divp);
-  if (S->red) (void)hipFree(S->red);
-  if (S->wallg) (void)hipFree(S->wallg);
   if (S->ycoord) (void)hipFree(S->ycoord);
 }
 
