@@ -16,7 +16,7 @@ HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
 BUILD = os.path.join(HERE, "_build")
 LIB = os.path.join(HERE, "libx3d.so")
-SOURCES = ["capi.cpp", "schemes.cpp", "lines_f64.hip", "lines_f32.hip", "fft.hip", "fields.hip", "solver.hip",
+SOURCES = ["capi.cpp", "schemes.cpp", "lines_f64.hip", "lines_f32.hip", "lines_anchored_f64.hip", "lines_anchored_f32.hip", "fft.hip", "fields.hip", "solver.hip",
            "momentum.hip", "projection.hip", "bounded.hip", "les.hip", "mlp.hip", "capi_les.cpp", "channel.hip", "capi_host.cpp"]
 ARCH = os.environ.get("X3D_OFFLOAD_ARCH", "gfx950")
 

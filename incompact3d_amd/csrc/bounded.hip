@@ -69,8 +69,9 @@ void edge_table(int op, int n_in, int n_out, const Sten<double> &s, int bc1, int
   }
 }
 
-// The packed factors of a set on anchored segments of L rows, and the chain
-// depth of those segments.
+// The packed factors of a set on anchored segments of L rows (their
+// Sherman-Morrison word too, zero in the rows between), and the chain depth of
+// those segments.
 std::vector<double> padded_rows(const TriSet &t, int n, int L, double tol, int *P, int *K) {
   *P = (n + L - 1) / L;
   std::vector<double> pk(4 * (size_t)*P * L), gf(*P, 1.0), gb(*P, 1.0);
@@ -83,6 +84,7 @@ std::vector<double> padded_rows(const TriSet &t, int n, int L, double tol, int *
         q[0] = t.fs[e];
         q[1] = t.fw[e];
         q[2] = t.ff[e] * t.fw[e];
+        q[3] = t.sm[e];
       } else {
         q[0] = -1.0;
         q[2] = -1.0;
@@ -95,21 +97,47 @@ std::vector<double> padded_rows(const TriSet &t, int n, int L, double tol, int *
   return pk;
 }
 
+// One precision's table of segments of L rows: packed rows, then the weights.
+template <typename T>
+int upload_table(const TriSet &t, int n, int L, double tol, const double *W, AnchorTab<T> *out) {
+  std::vector<double> p = padded_rows(t, n, L, tol, &out->P, &out->K);
+  p.insert(p.end(), W, W + EDGE_WORDS);
+  const std::vector<T> h(p.begin(), p.end());
+  X3D_HIP(hipMalloc(&out->pk, h.size() * sizeof(T)));
+  X3D_HIP(hipMemcpy(out->pk, h.data(), h.size() * sizeof(T), hipMemcpyHostToDevice));
+  return X3D_OK;
+}
+
+template <typename T>
+int upload_tables(const TriSet &t, int n, const double *W, AnchorTab<T> (&out)[2]) {
+  constexpr int L = sizeof(T) == 8 ? SEG_L64 : SEG_L32;
+  const double tol = sizeof(T) == 8 ? 1e-18 : 1e-9;
+  if (n < 2 * L) return X3D_OK;
+  X3D_TRY(upload_table<T>(t, n, L, tol, W, &out[0]));
+  // lines just over 1024 threads of full rows: segments one row longer too
+  if ((n + L - 1) / L * (128 / (int)sizeof(T)) > 1024) X3D_TRY(upload_table<T>(t, n, L + 1, tol, W, &out[1]));
+  return X3D_OK;
+}
+
 }  // namespace
 
-// Lines of two FP32 segments or more get tables (shorter ones run on the
-// per-operator kernels).
+// Lines of two segments or more get tables, periodic ones only where neither
+// the wavefront kernels (x) nor whole segments (y, z) cover them.
 int bounded_setup(Context &c) {
   for (int d = 0; d < 3; ++d) {
     const DirCoef &D = c.dir[d];
-    if (D.bc1 == 0 || D.bcn == 0) continue;
-    if (D.nm < 2 * SEG_L32) continue;
+    const bool per = D.bc1 == 0;
+    if (per != (D.bcn == 0)) continue;
+    if (per) {
+      const int V = D.n / 64;
+      if (d == 0 ? (D.n % 64 == 0 && (V == 1 || V == 2 || V == 4 || V == 8)) : D.n % SEG_L32 == 0) continue;
+    }
     for (int op = 0; op < 6; ++op)
       for (int par = 0; par < 2; ++par) {
         // parities the reference has: both for the derivatives on the
         // velocity points, odd (0) and even (1) operands alike; the even one
         // for the other staggered operators
-        if (par == 0 && (op == OP_INTERVP || op == OP_DERPV || op == OP_INTERPV)) continue;
+        if (!per && par == 0 && (op == OP_INTERVP || op == OP_DERPV || op == OP_INTERPV)) continue;
         LineCall<double> call;
         X3D_TRY(make_line_call<double>(c, d, op, par, &call));
         int set = -1;
@@ -118,18 +146,20 @@ int bounded_setup(Context &c) {
         if (set < 0) return fail(X3D_ERR_STATE, "bounded tables: unknown coefficient set");
         const TriSet &t = c.sets[set];
         const int n_out = call.n_out, n_in = op == OP_DERPV || op == OP_INTERPV ? D.nm : D.n;
+        if (n_in < 8 || n_out < 8) continue;
         BoundTab &b = c.btab[d][op][par];
-        double W[EDGE_WORDS];
-        edge_table(op, n_in, n_out, D.s, D.bc1, D.bcn, par, W);
-        std::vector<double> p64 = padded_rows(t, n_out, SEG_L64, 1e-18, &b.P64, &b.K64);
-        std::vector<double> p32 = padded_rows(t, n_out, SEG_L32, 1e-9, &b.P32, &b.K32);
-        p64.insert(p64.end(), W, W + EDGE_WORDS);
-        p32.insert(p32.end(), W, W + EDGE_WORDS);
-        std::vector<float> f32(p32.begin(), p32.end());
-        X3D_HIP(hipMalloc(&b.d64, p64.size() * sizeof(double)));
-        X3D_HIP(hipMalloc(&b.d32, f32.size() * sizeof(float)));
-        X3D_HIP(hipMemcpy(b.d64, p64.data(), p64.size() * sizeof(double), hipMemcpyHostToDevice));
-        X3D_HIP(hipMemcpy(b.d32, f32.data(), f32.size() * sizeof(float), hipMemcpyHostToDevice));
+        double W[EDGE_WORDS] = {};
+        if (!per) edge_table(op, n_in, n_out, D.s, D.bc1, D.bcn, par, W);
+        b.set64[0] = t.d64;
+        b.set32[0] = t.d32;
+        for (const TriSet &f : c.sets)
+          if (f.name[0] == t.name[0] && same_set(f, t)) {
+            b.set64[1] = f.d64;
+            b.set32[1] = f.d32;
+            break;
+          }
+        X3D_TRY(upload_tables<double>(t, n_out, W, b.t64));
+        X3D_TRY(upload_tables<float>(t, n_out, W, b.t32));
       }
   }
   return X3D_OK;
@@ -139,8 +169,10 @@ void bounded_free(Context &c) {
   for (auto &d : c.btab)
     for (auto &o : d)
       for (BoundTab &b : o) {
-        if (b.d64) (void)hipFree(b.d64);
-        if (b.d32) (void)hipFree(b.d32);
+        for (auto &t : b.t64)
+          if (t.pk) (void)hipFree(t.pk);
+        for (auto &t : b.t32)
+          if (t.pk) (void)hipFree(t.pk);
         b = BoundTab();
       }
 }
@@ -162,23 +194,6 @@ struct BMomArgs {
   const T *m1, *m2, *m4;        // stretched y: ppy, pp2y, pp4y*ppy (null: uniform)
   MomUpdate<T> up;              // x sweep
 };
-
-// The rows of a segment to memory; NT: streaming stores.
-template <typename T, int L, bool NT>
-__device__ __forceinline__ void store_rows(T *p, const unsigned off, const unsigned step, const T (&v)[L],
-                                           const int rows) {
-  if (rows == L) {
-#pragma unroll
-    for (int m = 0; m < L; ++m) {
-      if constexpr (NT) st_nt(p, off + (unsigned)m * step, v[m]);
-      else at(p, off + (unsigned)m * step) = v[m];
-    }
-  } else {
-#pragma unroll
-    for (int m = 0; m < L; ++m)
-      if (m < rows) at(p, off + (unsigned)m * step) = v[m];
-  }
-}
 
 // -1/2 D1(u_d u_c) - 1/2 u_d D1(u_c) + nu D2(u_c) of the rows of a segment:
 // the right-hand sides from the windows.

@@ -1,5 +1,6 @@
 #pragma once
-// Segmented solves of lines with free-slip or no-slip ends.
+// Segmented solves of lines with free-slip or no-slip ends, and of periodic
+// lines that are no whole number of segments.
 //
 // The n_out rows of a line are cut into P segments of L, one thread each, as
 // in seg_solve, but anchored at both ends: segments 0 .. P-3 start at s L, the
@@ -108,6 +109,23 @@ __device__ __forceinline__ void bound_rhs(const T (&win)[L + 2 * HW], T (&w)[L],
 #pragma unroll
     for (int m = 1; m < L; ++m)
       if (m >= rows) w[m] = T(0);
+  }
+}
+
+// The rows of a segment to memory; NT: streaming stores.
+template <typename T, int L, bool NT>
+__device__ __forceinline__ void store_rows(T *p, const unsigned off, const unsigned step, const T (&v)[L],
+                                           const int rows) {
+  if (rows == L) {
+#pragma unroll
+    for (int m = 0; m < L; ++m) {
+      if constexpr (NT) st_nt(p, off + (unsigned)m * step, v[m]);
+      else at(p, off + (unsigned)m * step) = v[m];
+    }
+  } else {
+#pragma unroll
+    for (int m = 0; m < L; ++m)
+      if (m < rows) at(p, off + (unsigned)m * step) = v[m];
   }
 }
 
@@ -268,31 +286,34 @@ struct BoundCopy {
   }
 };
 
-// Table of one operator of a bounded direction at precision T (null: none).
+// Table of one operator of a direction at precision T (null: none): segments
+// of the precision's length, or (longer) one row longer.
 template <typename T>
 struct BoundDev {
   const T *pk = nullptr, *edge = nullptr;
   int P = 0, K = 0;
 };
 template <typename T>
-BoundDev<T> bound_dev(const Context &c, int dir, int op, int par) {
+BoundDev<T> bound_dev(const Context &c, int dir, int op, int par, bool longer = false) {
   const BoundTab &b = c.btab[dir][op][par];
+  const AnchorTab<T> *t;
+  if constexpr (sizeof(T) == 8) t = &b.t64[longer ? 1 : 0];
+  else t = &b.t32[longer ? 1 : 0];
   BoundDev<T> d;
-  constexpr int L = sizeof(T) == 8 ? SEG_L64 : SEG_L32;
-  const T *p = sizeof(T) == 8 ? (const T *)b.d64 : (const T *)b.d32;
-  if (!p) return d;
-  d.P = sizeof(T) == 8 ? b.P64 : b.P32;
-  d.K = sizeof(T) == 8 ? b.K64 : b.K32;
-  d.pk = p;
-  d.edge = p + 4 * (size_t)d.P * L;
+  if (!t->pk) return d;
+  const int L = (sizeof(T) == 8 ? SEG_L64 : SEG_L32) + (longer ? 1 : 0);
+  d.P = t->P;
+  d.K = t->K;
+  d.pk = t->pk;
+  d.edge = t->pk + 4 * (size_t)d.P * L;
   return d;
 }
 
 // Launch shape: TL lines of 128 bytes a row (fewer where the block or its LDS
 // would not fit) x P segments; extra(TL) words of LDS beside the solve's.
-template <typename T>
+template <typename T, int LEN = sizeof(T) == 8 ? SEG_L64 : SEG_L32>
 struct BoundShape {
-  static constexpr int L = sizeof(T) == 8 ? SEG_L64 : SEG_L32;
+  static constexpr int L = LEN;
   int P = 0, TL = 0;
   size_t shmem = 0;
   template <typename F>

@@ -3,4 +3,5 @@
 
 namespace x3d {
 template int launch_line<double>(const LineCall<double> &, hipStream_t);
+template int launch_der1_triple<double>(const Context &, int, const LineTriple<double> &, int, int, int, const double *, hipStream_t);
 }  // namespace x3d

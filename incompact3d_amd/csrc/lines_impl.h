@@ -48,6 +48,10 @@ struct LineArgs {
   long long sa_in, sb_in, se_in;      // input strides (elements)
   long long sa_out, sb_out, se_out;   // output strides
   int row;                            // LDS row stride (x mode)
+  // blockIdx.z > 0: further operands of a batch (seg_line_kernel and
+  // xwave_kernel; same operator, same coefficients)
+  const T *ub[2], *accb[2];
+  T *tb[2];
 };
 
 // Window offsets an interior row needs: U(i-HL) .. U(i+HR).
@@ -869,6 +873,10 @@ __global__ void __launch_bounds__(1024) seg_line_kernel(const LineArgs<T> A, con
   const int line = threadIdx.x, seg = threadIdx.y;
   const int tid = seg * TL + line, nthr = TL * P;
   const int n = A.n_out;
+  const int item = (int)blockIdx.z;
+  const T *const u = item == 0 ? A.u : A.ub[item - 1];
+  const T *const acc = item == 0 ? A.acc : A.accb[item - 1];
+  T *const t = item == 0 ? A.t : A.tb[item - 1];
   T *cs = smem, *cf = cs + 4 * n, *cb = cf + P * TL, *gf = cb + P * TL, *gb = gf + P, *x0s = gb + P,
     *xns = x0s + TL;
   const int a = blockIdx.x * TL + line, b = blockIdx.y;
@@ -887,7 +895,7 @@ __global__ void __launch_bounds__(1024) seg_line_kernel(const LineArgs<T> A, con
 #pragma unroll
   for (int k = 0; k < L + 8; ++k) {
     const unsigned o = base + wrap(e0 - 4 + k) * step;
-    T x = at(A.u, o);
+    T x = at(u, o);
     if (EPI && A.u2) x *= at(A.u2, o);
     win[k] = x;
   }
@@ -910,27 +918,27 @@ __global__ void __launch_bounds__(1024) seg_line_kernel(const LineArgs<T> A, con
     for (int m = 0; m < L; ++m) {
       const unsigned o = base + (unsigned)(e0 + m) * step;
       mm[m] = A.mul ? at(A.mul, o) : T(1);
-      aa[m] = A.acc ? at(A.acc, o) : T(0);
+      aa[m] = acc ? at(acc, o) : T(0);
     }
 #pragma unroll
     for (int m = 0; m < L; ++m) {
       T r = w[0][m];
       if (A.mul) r *= mm[m];
       r = A.rc * r;
-      if (A.acc) r = A.ac * aa[m] + r;
-      st_nt(A.t, base + (unsigned)(e0 + m) * step, r);
+      if (acc) r = A.ac * aa[m] + r;
+      st_nt(t, base + (unsigned)(e0 + m) * step, r);
     }
   } else {
 #pragma unroll
-    for (int m = 0; m < L; ++m) st_nt(A.t, base + (unsigned)(e0 + m) * step, w[0][m]);
+    for (int m = 0; m < L; ++m) st_nt(t, base + (unsigned)(e0 + m) * step, w[0][m]);
   }
 }
 
 template <typename T, int OP>
-static int launch_seg_line(const LineArgs<T> &a, T rden, const YzShape<T> &Y, bool epi, int kdepth,
+static int launch_seg_line(const LineArgs<T> &a, T rden, const YzShape<T> &Y, bool epi, int kdepth, int batch,
                            hipStream_t st) {
   // the segment solve needs one line per block row and every segment full
-  const dim3 grid((a.na + Y.TL - 1) / Y.TL, a.nb), block(Y.TL, Y.P);
+  const dim3 grid((a.na + Y.TL - 1) / Y.TL, a.nb, batch), block(Y.TL, Y.P);
   const size_t shmem = Y.shmem;
   constexpr int L = YzShape<T>::L;
   if (epi) hipLaunchKernelGGL((seg_line_kernel<T, OP, L, true>), grid, block, shmem, st, a, rden, kdepth);
@@ -1142,6 +1150,10 @@ __global__ void __launch_bounds__(256) xwave_kernel(const LineArgs<T> A, int nli
   const int nwaves = (gridDim.x * blockDim.x) >> 6;
   const int n = A.n_out;   // == n_in == 64*V
   const int e0 = lane * V;
+  const int item = (int)blockIdx.z;
+  const T *const u = item == 0 ? A.u : A.ub[item - 1];
+  const T *const acc = item == 0 ? A.acc : A.accb[item - 1];
+  T *const t = item == 0 ? A.t : A.tb[item - 1];
   // 512-point lines read their coefficients from LDS for every line (laid
   // out [coefficient][point of the lane][lane], conflict-free) instead of
   // holding 4V of them in registers
@@ -1167,7 +1179,7 @@ __global__ void __launch_bounds__(256) xwave_kernel(const LineArgs<T> A, int nli
   // the next line's input is loaded while the current one is solved
   T nxt_u[V], nxt_u2[V];
   if (wave < nlines) {
-    load_run<T, V>(A.u + (long long)wave * n + e0, nxt_u);
+    load_run<T, V>(u + (long long)wave * n + e0, nxt_u);
     if (EPI && A.u2) load_run<T, V>(A.u2 + (long long)wave * n + e0, nxt_u2);
   }
   for (int ln = wave; ln < nlines; ln += nwaves) {
@@ -1180,7 +1192,7 @@ __global__ void __launch_bounds__(256) xwave_kernel(const LineArgs<T> A, int nli
       for (int m = 0; m < V; ++m) own[m] *= nxt_u2[m];
     }
     if (ln + nwaves < nlines) {
-      load_run<T, V>(A.u + base + (long long)nwaves * n, nxt_u);
+      load_run<T, V>(u + base + (long long)nwaves * n, nxt_u);
       if (EPI && A.u2) load_run<T, V>(A.u2 + base + (long long)nwaves * n, nxt_u2);
     }
     // window U(e0-HL .. e0+V+HR-1): own points plus neighbour lanes' points
@@ -1219,13 +1231,13 @@ __global__ void __launch_bounds__(256) xwave_kernel(const LineArgs<T> A, int nli
 #pragma unroll
       for (int m = 0; m < V; ++m) res[m] = A.rc * res[m];
     }
-    if (EPI && A.acc) {
+    if (EPI && acc) {
       T aa[V];
-      load_run<T, V>(A.acc + base, aa);
+      load_run<T, V>(acc + base, aa);
 #pragma unroll
       for (int m = 0; m < V; ++m) res[m] = A.ac * aa[m] + res[m];
     }
-    store_run<T, V>(A.t + base, res);
+    store_run<T, V>(t + base, res);
   }
 }
 
@@ -1236,10 +1248,10 @@ static void launch_xv(const LineArgs<T> &a, bool epi, int nlines, dim3 grid, dim
 }
 
 template <typename T, int OP>
-static int launch_xwave(const LineArgs<T> &a, bool epi, int nlines, hipStream_t st) {
+static int launch_xwave(const LineArgs<T> &a, bool epi, int nlines, int batch, hipStream_t st) {
   const int V = a.n_out / 64;
   const int waves = nlines < 16384 ? nlines : 16384;
-  const dim3 grid((waves + 3) / 4), block(256);
+  const dim3 grid((waves + 3) / 4, 1, batch), block(256);
   switch (V) {
     case 1: launch_xv<T, OP, 1>(a, epi, nlines, grid, block, st); break;
     case 2: launch_xv<T, OP, 2>(a, epi, nlines, grid, block, st); break;
@@ -1365,12 +1377,12 @@ int launch_line(const LineCall<T> &c, hipStream_t st) {
       !c.pp && aligned16(c.u) && aligned16(c.u2) && aligned16(c.t) && aligned16(c.acc) && aligned16(c.mul)) {
     const int nlines = ny * nz;
     switch (c.op) {
-      case OP_DER1: return launch_xwave<T, OP_DER1>(a, epi, nlines, st);
-      case OP_DER2: return launch_xwave<T, OP_DER2>(a, epi, nlines, st);
-      case OP_DERVP: return launch_xwave<T, OP_DERVP>(a, epi, nlines, st);
-      case OP_INTERVP: return launch_xwave<T, OP_INTERVP>(a, epi, nlines, st);
-      case OP_DERPV: return launch_xwave<T, OP_DERPV>(a, epi, nlines, st);
-      case OP_INTERPV: return launch_xwave<T, OP_INTERPV>(a, epi, nlines, st);
+      case OP_DER1: return launch_xwave<T, OP_DER1>(a, epi, nlines, 1, st);
+      case OP_DER2: return launch_xwave<T, OP_DER2>(a, epi, nlines, 1, st);
+      case OP_DERVP: return launch_xwave<T, OP_DERVP>(a, epi, nlines, 1, st);
+      case OP_INTERVP: return launch_xwave<T, OP_INTERVP>(a, epi, nlines, 1, st);
+      case OP_DERPV: return launch_xwave<T, OP_DERPV>(a, epi, nlines, 1, st);
+      case OP_INTERPV: return launch_xwave<T, OP_INTERPV>(a, epi, nlines, 1, st);
     }
   }
   YzShape<T> Y;
@@ -1378,13 +1390,18 @@ int launch_line(const LineCall<T> &c, hipStream_t st) {
     const int K = c.tri.kdepth > 0 ? c.tri.kdepth : Y.P;
     const T rden = c.tri.rden;
     switch (c.op) {
-      case OP_DER1: return launch_seg_line<T, OP_DER1>(a, rden, Y, epi, K, st);
-      case OP_DER2: return launch_seg_line<T, OP_DER2>(a, rden, Y, epi, K, st);
-      case OP_DERVP: return launch_seg_line<T, OP_DERVP>(a, rden, Y, epi, K, st);
-      case OP_INTERVP: return launch_seg_line<T, OP_INTERVP>(a, rden, Y, epi, K, st);
-      case OP_DERPV: return launch_seg_line<T, OP_DERPV>(a, rden, Y, epi, K, st);
-      case OP_INTERPV: return launch_seg_line<T, OP_INTERPV>(a, rden, Y, epi, K, st);
+      case OP_DER1: return launch_seg_line<T, OP_DER1>(a, rden, Y, epi, K, 1, st);
+      case OP_DER2: return launch_seg_line<T, OP_DER2>(a, rden, Y, epi, K, 1, st);
+      case OP_DERVP: return launch_seg_line<T, OP_DERVP>(a, rden, Y, epi, K, 1, st);
+      case OP_INTERVP: return launch_seg_line<T, OP_INTERVP>(a, rden, Y, epi, K, 1, st);
+      case OP_DERPV: return launch_seg_line<T, OP_DERPV>(a, rden, Y, epi, K, 1, st);
+      case OP_INTERPV: return launch_seg_line<T, OP_INTERPV>(a, rden, Y, epi, K, 1, st);
     }
+  }
+  {
+    bool done = false;
+    X3D_TRY(launch_anchored<T>(c, nullptr, &done, st));
+    if (done) return X3D_OK;
   }
   WallShape<T> Wsh;
   const size_t fin = (size_t)nx * ny * nz / (size_t)(c.dir == 1 ? ny : nz) * (size_t)n_in * sizeof(T);
@@ -1412,5 +1429,65 @@ int launch_line(const LineCall<T> &c, hipStream_t st) {
   return fail(X3D_ERR_ARG, "unknown line operator");
 }
 
+
+// Three first derivatives along dir (x3d_internal.h), pp as in LineCall.
+template <typename T>
+int launch_der1_triple(const Context &c, int dir, const LineTriple<T> &b, int nx, int ny, int nz, const T *pp,
+                       hipStream_t st) {
+  const DirCoef &D = c.dir[dir];
+  LineCall<T> L;
+  X3D_TRY(make_line_call<T>(c, dir, OP_DER1, b.par[0], &L));
+  L.pp = pp;
+  L.nx = nx;
+  L.ny = ny;
+  L.nz = nz;
+  const bool epi = b.acc[0] || b.acc[1] || b.acc[2];
+  const bool whole = !pp && (size_t)nx * ny * nz * sizeof(T) < ((size_t)1 << 32);
+  // one coefficient set serves both parities of a periodic direction
+  if (whole && D.bc1 == 0 && same_set(c.sets[D.set_d1_even], c.sets[D.set_d1_odd])) {
+    LineArgs<T> a{};
+    a.u = b.u[0]; a.t = b.t[0]; a.acc = b.acc[0];
+    for (int i = 0; i < 2; ++i) {
+      a.ub[i] = b.u[i + 1];
+      a.tb[i] = b.t[i + 1];
+      a.accb[i] = b.acc[i + 1];
+    }
+    a.ac = a.rc = T(1);
+    a.pk = L.tri.pk;
+    a.alfa = L.tri.alfa; a.sm_den = L.tri.sm_den; a.rden = L.tri.rden;
+    a.s = L.s;
+    a.n_in = a.n_out = D.n;
+    const int V = D.n / 64;
+    bool al = true;
+    for (int i = 0; i < 3; ++i) al = al && aligned16(b.u[i]) && aligned16(b.t[i]) && aligned16(b.acc[i]);
+    if (dir == 0 && D.n % 64 == 0 && (V == 1 || V == 2 || V == 4 || V == 8) && al)
+      return launch_xwave<T, OP_DER1>(a, epi, ny * nz, 3, st);
+    YzShape<T> Y;
+    if (dir != 0 && Y.plan(D.n, 1, 1)) {
+      if (dir == 1) {
+        a.na = nx; a.nb = nz; a.se_in = nx; a.sa_in = 1; a.sb_in = (long long)nx * ny;
+      } else {
+        a.na = nx; a.nb = ny; a.se_in = (long long)nx * ny; a.sa_in = 1; a.sb_in = nx;
+      }
+      a.se_out = a.se_in; a.sa_out = a.sa_in; a.sb_out = a.sb_in;
+      return launch_seg_line<T, OP_DER1>(a, L.tri.rden, Y, epi, L.tri.kdepth > 0 ? L.tri.kdepth : Y.P, 3, st);
+    }
+  }
+  bool done = false;
+  X3D_TRY(launch_anchored<T>(L, &b, &done, st));
+  if (done) return X3D_OK;
+  for (int i = 0; i < 3; ++i) {
+    X3D_TRY(make_line_call<T>(c, dir, OP_DER1, b.par[i], &L));
+    L.pp = pp;
+    L.nx = nx;
+    L.ny = ny;
+    L.nz = nz;
+    L.u = b.u[i];
+    L.t = b.t[i];
+    L.acc = b.acc[i];
+    X3D_TRY(launch_line<T>(L, st));
+  }
+  return X3D_OK;
+}
 
 }  // namespace x3d

@@ -203,6 +203,30 @@ int momentum_component(const Context &c, const T *const u[3], int comp, T *W, T 
   return X3D_OK;
 }
 
+// Three first derivatives along d in one launch, with the metric of a
+// stretched y mesh as line() applies it.
+template <typename T>
+int der1_triple(const Context &c, int d, const LineTriple<T> &b, int nx, int ny, int nz) {
+  return launch_der1_triple<T>(c, d, b, nx, ny, nz, d == 1 ? metric<T>(c, M_PPY) : nullptr, c.stream);
+}
+
+// g[3*d + comp] = d u_comp / d x_d, parity 0 along the component's own
+// direction and 1 across it
+template <typename T>
+int nine_gradients(const Context &c, const T *const u[3], T *const g[9], int nx, int ny, int nz) {
+  for (int d = 0; d < 3; ++d) {
+    LineTriple<T> b;
+    for (int comp = 0; comp < 3; ++comp) {
+      b.u[comp] = u[comp];
+      b.t[comp] = g[3 * d + comp];
+      b.acc[comp] = nullptr;
+      b.par[comp] = d == comp ? 0 : 1;
+    }
+    X3D_TRY(der1_triple<T>(c, d, b, nx, ny, nz));
+  }
+  return X3D_OK;
+}
+
 // ---------------------------------------------------------------- LES (les_models.f90)
 // SGS force of the current velocity into sgs[3] (compute precision):
 // Smagorinsky in the nonconservative form (sgs_mom_nonconservative,
@@ -211,15 +235,18 @@ int momentum_component(const Context &c, const T *const u[3], int comp, T *W, T 
 template <typename T>
 int stress_divergence(const Context &c, T *const t[6], T *const sgs[3], int nx, int ny, int nz) {
   // les_models.f90:1384-1440; t = xx yy zz xy xz yz
-  X3D_TRY(line<T>(c, 0, OP_DER1, 0, t[0], nullptr, sgs[0], nullptr, nullptr, 0, 1, nx, ny, nz));
-  X3D_TRY(line<T>(c, 0, OP_DER1, 0, t[3], nullptr, sgs[1], nullptr, nullptr, 0, 1, nx, ny, nz));
-  X3D_TRY(line<T>(c, 0, OP_DER1, 0, t[4], nullptr, sgs[2], nullptr, nullptr, 0, 1, nx, ny, nz));
-  X3D_TRY(line<T>(c, 1, OP_DER1, 0, t[3], nullptr, sgs[0], sgs[0], nullptr, 1, 1, nx, ny, nz));
-  X3D_TRY(line<T>(c, 1, OP_DER1, 1, t[1], nullptr, sgs[1], sgs[1], nullptr, 1, 1, nx, ny, nz));
-  X3D_TRY(line<T>(c, 1, OP_DER1, 0, t[5], nullptr, sgs[2], sgs[2], nullptr, 1, 1, nx, ny, nz));
-  X3D_TRY(line<T>(c, 2, OP_DER1, 0, t[4], nullptr, sgs[0], sgs[0], nullptr, 1, 1, nx, ny, nz));
-  X3D_TRY(line<T>(c, 2, OP_DER1, 0, t[5], nullptr, sgs[1], sgs[1], nullptr, 1, 1, nx, ny, nz));
-  X3D_TRY(line<T>(c, 2, OP_DER1, 0, t[2], nullptr, sgs[2], sgs[2], nullptr, 1, 1, nx, ny, nz));
+  const int idx[3][3] = {{0, 3, 4}, {3, 1, 5}, {4, 5, 2}};   // [direction][component]
+  const int par[3][3] = {{0, 0, 0}, {0, 1, 0}, {0, 0, 0}};
+  for (int d = 0; d < 3; ++d) {
+    LineTriple<T> b;
+    for (int comp = 0; comp < 3; ++comp) {
+      b.u[comp] = t[idx[d][comp]];
+      b.t[comp] = sgs[comp];
+      b.acc[comp] = d == 0 ? nullptr : sgs[comp];
+      b.par[comp] = par[d][comp];
+    }
+    X3D_TRY(der1_triple<T>(c, d, b, nx, ny, nz));
+  }
   return X3D_OK;
 }
 
@@ -234,10 +261,7 @@ int compute_sgs(const Context &c, x3d_solver *S, const T *const u[3], T *const s
   T *nut = f + 15 * n, *ta = f + 16 * n;
   // the nine gradients with the parities of smag (les_models.f90:210-238):
   // g[3*d + comp] = d u_comp / d x_d, parity 0 when d == comp
-  for (int d = 0; d < 3; ++d)
-    for (int comp = 0; comp < 3; ++comp)
-      X3D_TRY(line<T>(c, d, OP_DER1, d == comp ? 0 : 1, u[comp], nullptr, g[3 * d + comp], nullptr, nullptr, 0, 1,
-                      nx, ny, nz));
+  X3D_TRY(nine_gradients<T>(c, u, g, nx, ny, nz));
   const T *cg[9];
   for (int i = 0; i < 9; ++i) cg[i] = g[i];
   const double delta = std::cbrt(c.dir[0].d * c.dir[1].d * c.dir[2].d);   // les_models.f90:36-39
@@ -695,11 +719,7 @@ int tgv_stats(Context &c, x3d_solver *S, double out4[4]) {
   const T *u[3];
   for (int i = 0; i < 3; ++i) u[i] = sizeof(T) == 8 ? (const T *)S->u64[i] : (const T *)S->u32[i];
   // (dux/dx, duy/dx, duz/dx, dux/dy, ..., duz/dz) with the parities of Case-TGV.f90:262-270
-  for (int d = 0; d < 3; ++d)
-    for (int comp = 0; comp < 3; ++comp) {
-      const int pv = d == comp ? 0 : 1;
-      X3D_TRY(line<T>(c, d, OP_DER1, pv, u[comp], nullptr, g[3 * d + comp], nullptr, nullptr, 0, 1, nx, ny, nz));
-    }
+  X3D_TRY(nine_gradients<T>(c, u, g, nx, ny, nz));
   // laplacian per component: d2x + d2y + d2z (Case-TGV.f90:330-360)
   for (int comp = 0; comp < 3; ++comp)
     for (int d = 0; d < 3; ++d) {

@@ -98,13 +98,22 @@ struct DirCoef {
   int set_c6 = -1, set_ci6p = -1, set_ci6 = -1, set_cip6 = -1, set_ciip6 = -1;
 };
 
-// Tables of one operator on the bounded lines of a direction (bounded_impl.h):
-// padded packed factors and closure weights, FP64 and FP32 copies, segments
-// and chain depth of each precision.
+// Tables of one operator on anchored segments (bounded_impl.h): padded packed
+// factors and closure weights, segments and chain depth; [0] segments of the
+// precision's length, [1] one row longer (where blocks of the first would have
+// more than 1024 threads).  set64, set32: the coefficient set they are of, and
+// the first one of the direction with the same coefficients, which is what a
+// caller's arrays are matched to.
+template <typename T>
+struct AnchorTab {
+  T *pk = nullptr;
+  int P = 0, K = 0;
+};
 struct BoundTab {
-  double *d64 = nullptr;
-  float *d32 = nullptr;
-  int P64 = 0, P32 = 0, K64 = 0, K32 = 0;
+  const double *set64[2] = {nullptr, nullptr};
+  const float *set32[2] = {nullptr, nullptr};
+  AnchorTab<double> t64[2];
+  AnchorTab<float> t32[2];
 };
 
 struct Context {
@@ -171,6 +180,24 @@ struct LineCall {
   const T *mul = nullptr;
   T ac = T(1), rc = T(1);
 };
+
+// Three first derivatives along one direction, t[i] = acc[i] + D1 u[i] (acc
+// null: none), each with its parity, in one launch where a batched kernel
+// covers the lines.
+template <typename T>
+struct LineTriple {
+  const T *u[3], *acc[3];
+  T *t[3];
+  int par[3];
+};
+template <typename T>
+int launch_der1_triple(const Context &c, int dir, const LineTriple<T> &b, int nx, int ny, int nz, const T *pp,
+                       hipStream_t st);
+
+// lines_anchored.hip: one operator on anchored segments; *done tells whether
+// the call was covered
+template <typename T>
+int launch_anchored(const LineCall<T> &c, const LineTriple<T> *triple, bool *done, hipStream_t st);
 
 template <typename T>
 int launch_line(const LineCall<T> &c, hipStream_t st);
