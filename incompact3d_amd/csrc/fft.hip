@@ -194,10 +194,13 @@ struct Dft<T, 16, INV> {
 };
 
 // ---------------------------------------------------------------- line FFT
-// Points per thread and threads per line for a line of N points.
+// Points per thread and threads per line for a line of N points: 16, so that
+// lines of up to 256 points exchange once; 8 for lines of up to 64, which
+// exchange once with that too and belong to grids of few lines, where twice
+// the threads count for more.
 template <int N>
 struct LineShape {
-  static constexpr int E = N >= 16 ? 16 : N;
+  static constexpr int E = N >= 128 ? 16 : 8;
   static constexpr int NT = N / E;
 };
 
@@ -296,27 +299,32 @@ struct TableStage {
 
 constexpr int FFT_THREADS = 256;
 
-// x blocks: XT lines of M = nx/2 complex points, NT threads per line.
+// x blocks: TL lines of M = nx/2 complex points, NT threads per line.  Short
+// lines run in blocks of one wavefront: a 64^3 grid has 4096 lines of 32
+// points, 32 blocks of 256 threads with 16 points each, 256 of these.
 template <int M>
 struct XShape {
   static constexpr int NT = LineShape<M>::NT;
-  static constexpr int TL = FFT_THREADS / NT;
+  static constexpr int THREADS = M <= 64 ? 64 : FFT_THREADS;
+  static constexpr int TL = THREADS / NT;
   static constexpr int LP = M + M / 16;             // padded line length in LDS
   template <typename T>
   static constexpr size_t lds() { return sizeof(cplx<T>) * ((size_t)TL * LP + 2 * M + 1); }
 };
-// strided blocks: TL kx x N points, NT threads per line.  TL = 256/NT lines
-// for FP64 and twice that for FP32, so that each point row a block reads is
-// 256 bytes either way (at most 64 lines, 512 threads).  The nx/2+1 kx lines
-// do not fill whole blocks and the last column of blocks runs mostly empty.
+// strided blocks: TL kx x N points, NT threads per line.  Point rows of 256
+// bytes for lines of 128 and 256 points, 128 bytes for the others: the long
+// ones for their LDS, the short ones because their grids have few lines (64^3:
+// 64 blocks of 64 lines, half of them past nx/2+1, against 320 of 8 in FP64).
+// The nx/2+1 kx lines do not fill whole blocks and the last column of blocks
+// runs mostly empty.
 // (One line more per block instead, on a ninth wavefront, left a CU with one
 // block of the FP32 z pass where two of eight wavefronts fit: 512^3 653
 // against 418 us, 256^3 46 against 39 us.)
 template <typename T, int N>
 struct SShape {
   static constexpr int NT = LineShape<N>::NT;
-  static constexpr int TL0 = (FFT_THREADS / NT) * (sizeof(T) == 4 ? 2 : 1);
-  static constexpr int TL = TL0 < 64 ? TL0 : 64;
+  static constexpr int LINE = 128 / (int)sizeof(cplx<T>);   // kx per cache line
+  static constexpr int TL = N == 128 || N == 256 ? 2 * LINE : (N <= 512 ? LINE : LINE / 2);
   static constexpr int threads() { return TL * NT; }
   // ztab: the z pass's tz and kz2 tables in FP64 (lines up to 256 points,
   // where the 4 KB keep two blocks per CU)
@@ -365,7 +373,7 @@ __device__ __forceinline__ void store_strided(cplx<T> *line, const size_t se, in
 // ---------------------------------------------------------------- pass 1: r2c along x
 // X_k = (Z_k + conj Z_{M-k})/2 - i/2 e^{-2 pi i k/nx} (Z_k - conj Z_{M-k}), k = 0..M
 template <typename T, int M>
-__global__ void __launch_bounds__(FFT_THREADS) r2c_x_kernel(const T *__restrict__ in, cplx<T> *__restrict__ out,
+__global__ void __launch_bounds__(XShape<M>::THREADS) r2c_x_kernel(const T *__restrict__ in, cplx<T> *__restrict__ out,
                                                              int nlines, int np, int xdct, PoissonTables<T> tb) {
   using S = XShape<M>;
   constexpr int E = LineShape<M>::E, NT = S::NT, TL = S::TL;
@@ -431,7 +439,7 @@ __global__ void __launch_bounds__(FFT_THREADS) r2c_x_kernel(const T *__restrict_
 // ---------------------------------------------------------------- pass 5: c2r along x
 // Z_k = (X_k + conj X_{M-k}) + i e^{+2 pi i k/nx} (X_k - conj X_{M-k}),  k < M
 template <typename T, int M>
-__global__ void __launch_bounds__(FFT_THREADS) c2r_x_kernel(const cplx<T> *__restrict__ in, T *__restrict__ out,
+__global__ void __launch_bounds__(XShape<M>::THREADS) c2r_x_kernel(const cplx<T> *__restrict__ in, T *__restrict__ out,
                                                              int nlines, int np, int xdct, PoissonTables<T> tb) {
   using S = XShape<M>;
   constexpr int E = LineShape<M>::E, NT = S::NT, TL = S::TL;
