@@ -40,6 +40,16 @@ constexpr int MLP_WG_BLOCKS = 256;   // blocks of the weight-gradient kernel
 // ---------------------------------------------------------------- BF16 helpers
 // round to nearest even: gfx950's v_cvt_pk_bf16_f32
 __device__ __forceinline__ short to_bf16(float f) { return __builtin_bit_cast(short, (__bf16)f); }
+// four at once, as two pairs (one by one they take four conversions and two
+// moves)
+__device__ __forceinline__ bf16x4 to_bf16(f32x4 f) {
+  typedef float f2 __attribute__((ext_vector_type(2)));
+  typedef __bf16 b2 __attribute__((ext_vector_type(2)));
+  struct {
+    b2 lo, hi;
+  } r = {__builtin_convertvector((f2{f[0], f[1]}), b2), __builtin_convertvector((f2{f[2], f[3]}), b2)};
+  return __builtin_bit_cast(bf16x4, r);
+}
 __device__ __forceinline__ float from_bf16(short h) { return __uint_as_float(((unsigned)(unsigned short)h) << 16); }
 
 // GELU in the tanh form of Hendrycks & Gimpel (2016),
@@ -127,7 +137,12 @@ struct Fwd16 {
   bf16x4 h[3][4];   // inputs of layers 2, 3, 4
 };
 
-// At[t]: this lane's operand of tile t (a register array)
+// At[t]: this lane's operand of tile t (a register array, or LdsTiles)
+struct LdsTiles {
+  const bf16x4 *p;
+  int lane;
+  __device__ __forceinline__ bf16x4 operator[](int t) const { return p[t * 64 + lane]; }
+};
 template <typename ACC>
 __device__ __forceinline__ f32x4 forward16(const ACC &At, const float *__restrict__ bias, bf16x4 x, int kb,
                                            Fwd16 &F) {
@@ -137,10 +152,10 @@ __device__ __forceinline__ f32x4 forward16(const ACC &At, const float *__restric
   for (int mt = 0; mt < 4; ++mt) {
     const f32x4 acc = mfma(At[T_A1 + mt], x, *reinterpret_cast<const f32x4 *>(bias + 16 * mt + 4 * kb));
     F.z[0][mt] = acc;
-    bf16x4 h;
+    f32x4 h;
 #pragma unroll
-    for (int i = 0; i < 4; ++i) h[i] = to_bf16(gelu(acc[i]));
-    F.h[0][mt] = h;
+    for (int i = 0; i < 4; ++i) h[i] = gelu(acc[i]);
+    F.h[0][mt] = to_bf16(h);
   }
 #pragma unroll
   for (int layer = 1; layer < 3; ++layer) {
@@ -151,10 +166,10 @@ __device__ __forceinline__ f32x4 forward16(const ACC &At, const float *__restric
 #pragma unroll
       for (int kt = 0; kt < 4; ++kt) acc = mfma(At[base + 4 * mt + kt], F.h[layer - 1][kt], acc);
       F.z[layer][mt] = acc;
-      bf16x4 h;
+      f32x4 h;
 #pragma unroll
-      for (int i = 0; i < 4; ++i) h[i] = to_bf16(gelu(acc[i]));
-      F.h[layer][mt] = h;
+      for (int i = 0; i < 4; ++i) h[i] = gelu(acc[i]);
+      F.h[layer][mt] = to_bf16(h);
     }
   }
   f32x4 y = *reinterpret_cast<const f32x4 *>(bias + 192 + 4 * kb);
@@ -165,13 +180,13 @@ __device__ __forceinline__ f32x4 forward16(const ACC &At, const float *__restric
 
 // feature tile from a point-major (N x 10) FP32 array
 __device__ __forceinline__ bf16x4 load_features(const float *__restrict__ x, int pt, int n, int kb) {
-  bf16x4 v;
+  f32x4 v;
 #pragma unroll
   for (int j = 0; j < 4; ++j) {
     const int f = 4 * kb + j;
-    v[j] = to_bf16((pt < n && f < MLP_NIN) ? x[(size_t)pt * MLP_NIN + f] : 0.0f);
+    v[j] = (pt < n && f < MLP_NIN) ? x[(size_t)pt * MLP_NIN + f] : 0.0f;
   }
-  return v;
+  return to_bf16(v);
 }
 
 // ---------------------------------------------------------------- inference on feature arrays
@@ -244,9 +259,7 @@ __global__ void __launch_bounds__(256) mlp_fwdbwd_kernel(const bf16x4 *__restric
       }
       dy[i] = d;
     }
-    bf16x4 g;
-#pragma unroll
-    for (int i = 0; i < 4; ++i) g[i] = to_bf16(dy[i]);
+    const bf16x4 g = to_bf16(dy);
     bf16x4 *row = act + (size_t)pt * ACT_ROW;
     if (valid) {
       row[ACT_H0 + kb] = xin;
@@ -262,9 +275,10 @@ __global__ void __launch_bounds__(256) mlp_fwdbwd_kernel(const bf16x4 *__restric
 #pragma unroll
     for (int mt = 0; mt < 4; ++mt) {
       f32x4 dh = mfma(At[T_AT4 + mt], g, zero);
-      bf16x4 q;
+      f32x4 dz;
 #pragma unroll
-      for (int i = 0; i < 4; ++i) q[i] = to_bf16(dh[i] * gelu_grad(F.z[2][mt][i]));
+      for (int i = 0; i < 4; ++i) dz[i] = dh[i] * gelu_grad(F.z[2][mt][i]);
+      const bf16x4 q = to_bf16(dz);
       gz[mt] = q;
       if (valid) row[ACT_D3 + 4 * mt + kb] = q;
     }
@@ -278,9 +292,10 @@ __global__ void __launch_bounds__(256) mlp_fwdbwd_kernel(const bf16x4 *__restric
         f32x4 dh = zero;
 #pragma unroll
         for (int kt = 0; kt < 4; ++kt) dh = mfma(At[base + 4 * mt + kt], gz[kt], dh);
-        bf16x4 q;
+        f32x4 dz;
 #pragma unroll
-        for (int i = 0; i < 4; ++i) q[i] = to_bf16(dh[i] * gelu_grad(F.z[layer - 1][mt][i]));
+        for (int i = 0; i < 4; ++i) dz[i] = dh[i] * gelu_grad(F.z[layer - 1][mt][i]);
+        const bf16x4 q = to_bf16(dz);
         nz[mt] = q;
         if (valid) row[(layer == 2 ? ACT_D2 : ACT_D1) + 4 * mt + kb] = q;
       }
@@ -505,18 +520,27 @@ struct ClosureArgs {
 // gradients are read once (coalesced), cross-lane reads build the four
 // 16-point MFMA input tiles, the outputs come back to the point's own lane,
 // and the fallback / projection epilogue runs on all 64 lanes.
+//
+// Bound by the issue of vector instructions: a tile of 16 points takes about
+// 880, of them 48 GELUs a lane with an exp2 and a reciprocal each at a quarter
+// rate, 17 of the 30 us at 64^3 FP32; its MFMAs run beside them.  Weights in
+// LDS: held in registers (80 of them) they left one wave a SIMD and moved
+// through accumulation registers, 33.2 us.
 template <typename T>
 __global__ void __launch_bounds__(256) closure_kernel(const bf16x4 *__restrict__ tiles, const float *__restrict__ bias,
                                                      const ClosureArgs<T> A, int *__restrict__ nfallback) {
   __shared__ __align__(16) float sb[208];
+  __shared__ __align__(16) bf16x4 sw[T_AT4 * 64];
   __shared__ int cnt;
   for (int i = threadIdx.x; i < 208; i += blockDim.x) sb[i] = bias[i];
+#pragma unroll
+  for (int i = 0; i < T_AT4 * 64 / 256; ++i) sw[threadIdx.x + 256 * i] = tiles[threadIdx.x + 256 * i];
   if (threadIdx.x == 0) cnt = 0;
   __syncthreads();
   const int lane = threadIdx.x & 63, kb = lane >> 4, r16 = lane & 15;
-  bf16x4 At[40];
-#pragma unroll
-  for (int t = 0; t < 40; ++t) At[t] = tiles[t * 64 + lane];
+  // the weights stay in LDS: held in registers (80, half of them moved out of
+  // accumulation registers for every tile) they left two waves a SIMD
+  const LdsTiles At{sw, lane};
   const long long wave = (blockIdx.x * (long long)blockDim.x + threadIdx.x) >> 6;
   const long long nwaves = (gridDim.x * (long long)blockDim.x) >> 6;
   const long long nchunks = (long long)((A.n + 63) / 64);
@@ -535,14 +559,16 @@ __global__ void __launch_bounds__(256) closure_kernel(const bf16x4 *__restrict__
 #pragma nounroll
     for (int t = 0; t < 4; ++t) {
       // input tile t: column r16 is point 16t + r16, rows 4kb..4kb+3 its features
+      asm volatile("" ::: "memory");   // keep the weight reads inside the loop
       const int src = 16 * t + r16;
-      bf16x4 x;
+      f32x4 xt;
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
         const float c0 = __shfl(xf[j], src), c1 = __shfl(xf[4 + j], src);
         const float c2 = j == 0 ? __shfl(xf[8], src) : (j == 1 ? A.dfeat : 0.f);
-        x[j] = to_bf16(kb == 0 ? c0 : (kb == 1 ? c1 : (kb == 2 ? c2 : 0.f)));
+        xt[j] = kb == 0 ? c0 : (kb == 1 ? c1 : (kb == 2 ? c2 : 0.f));
       }
+      const bf16x4 x = to_bf16(xt);
       Fwd16 F;
       const f32x4 y = forward16(At, sb, x, kb, F);
       // outputs 0..3 of column r16 sit in lane r16, outputs 4..5 in lane 16 + r16
