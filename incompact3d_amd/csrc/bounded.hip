@@ -114,8 +114,7 @@ int upload_tables(const TriSet &t, int n, const double *W, AnchorTab<T> (&out)[2
   const double tol = sizeof(T) == 8 ? 1e-18 : 1e-9;
   if (n < 2 * L) return X3D_OK;
   X3D_TRY(upload_table<T>(t, n, L, tol, W, &out[0]));
-  // lines just over 1024 threads of full rows: segments one row longer too
-  if ((n + L - 1) / L * (128 / (int)sizeof(T)) > 1024) X3D_TRY(upload_table<T>(t, n, L + 1, tol, W, &out[1]));
+  if (n >= 2 * (L + 1)) X3D_TRY(upload_table<T>(t, n, L + 1, tol, W, &out[1]));
   return X3D_OK;
 }
 
@@ -195,6 +194,12 @@ struct BMomArgs {
   MomUpdate<T> up;              // x sweep
 };
 
+// Blocks up to this many threads run a kernel whose register budget is theirs:
+// the budget of 1024 threads, 128 registers, spilled 10 (L = 9, NT = 2) to 14
+// (L = 8, NT = 3, x) of them: 65^3 FP64 16.6 -> 14.4 us a y or z sweep, the
+// channel's y sweep 96 -> 84.  (Blocks of x lines are smaller: their LDS.)
+constexpr int BMOM_FEW = 512;
+
 // -1/2 D1(u_d u_c) - 1/2 u_d D1(u_c) + nu D2(u_c) of the rows of a segment:
 // the right-hand sides from the windows.
 template <typename T, int L>
@@ -215,8 +220,8 @@ __device__ __forceinline__ void bmom_rhs(const BMomArgs<T> &A, const T (&wc)[L +
 // points (128 bytes), each input is read once.  NT: 2 where the two first
 // derivatives have the same factors (no-slip ends), else 3.  Bound by the
 // latency of its loads and of the two carry chains, like mom_yz_kernel.
-template <typename T, int L, int NT>
-__global__ void __launch_bounds__(1024) bmom_yz_kernel(const BMomArgs<T> A) {
+template <typename T, int L, int NT, int MAXT>
+__global__ void __launch_bounds__(MAXT) bmom_yz_kernel(const BMomArgs<T> A) {
   extern __shared__ __align__(16) unsigned char smem_raw[];
   T *smem = reinterpret_cast<T *>(smem_raw);
   const int TL = blockDim.x, P = A.P, n = A.n;
@@ -301,9 +306,12 @@ __global__ void __launch_bounds__(1024) bmom_yz_kernel(const BMomArgs<T> A) {
 
 // x lines: TL whole lines are one contiguous piece of memory, staged in LDS
 // (odd line stride: the threads of a wave fall into different banks), solved
-// as above and written back in order with the velocity update.
+// as above and written back in order with the velocity update.  A thread has
+// all its loads of a stage in flight together: one after another they were a
+// chain of memory latencies (65^3 FP64: 20.8 -> 18.2 us; bproj_x_kernel 13.4
+// -> 10.1).
 template <typename T, int L, int NT>
-__global__ void __launch_bounds__(1024) bmom_x_kernel(const BMomArgs<T> A) {
+__global__ void __launch_bounds__(BMOM_FEW) bmom_x_kernel(const BMomArgs<T> A) {
   extern __shared__ __align__(16) unsigned char smem_raw[];
   T *smem = reinterpret_cast<T *>(smem_raw);
   const int TL = blockDim.x, P = A.P, n = A.n, row = A.row;
@@ -316,19 +324,32 @@ __global__ void __launch_bounds__(1024) bmom_x_kernel(const BMomArgs<T> A) {
   const bool along = comp == 0;
   const int l0 = (int)blockIdx.x * TL;
   const int tot = min(TL, A.na - l0) * n;
-  const long long base = (long long)l0 * n;
+  const unsigned base = (unsigned)l0 * (unsigned)n;   // (a field is under 4 GiB)
   const float rn = 1.0f / (float)n;
   const T *src[NT];
 #pragma unroll
   for (int t = 0; t < NT; ++t) src[t] = A.pk[along][NT == 2 ? t + 1 : t];
-  for (int idx = tid; idx < tot; idx += nthr) {
-    const int l = small_div(idx, n, rn);
-    td[l * row + idx - l * n] = A.u[0][base + idx];
-    if (!along) tt[l * row + idx - l * n] = A.u[comp][base + idx];
-  }
+  BoundCopy<T, NT> cp;
+  cp.load(src, tid, nthr, CW);
+  {
+    // n <= P L: at most L points a thread
+    T r0[L], r1[L];
 #pragma unroll
-  for (int t = 0; t < NT; ++t)
-    for (int i = tid; i < CW; i += nthr) cs[t * CW + i] = src[t][i];
+    for (int m = 0; m < L; ++m) {
+      const unsigned o = (base + (unsigned)min(tid + m * nthr, tot - 1)) * (unsigned)sizeof(T);
+      r0[m] = at(A.u[0], o);
+      if (!along) r1[m] = at(A.u[comp], o);
+    }
+#pragma unroll
+    for (int m = 0; m < L; ++m) {
+      const int idx = tid + m * nthr;
+      if (idx >= tot) continue;
+      const int l = small_div(idx, n, rn), q = l * row + idx - l * n;
+      td[q] = r0[m];
+      if (!along) tt[q] = r1[m];
+    }
+  }
+  cp.store(cs, src, tid, nthr, CW);
   __syncthreads();
   const int e0 = bound_first<L>(seg, P, n), rows = bound_rows<L>(seg, P, n);
   auto clamp = [&](int j) { return j < 0 ? 0 : (j >= n ? n - 1 : j); };
@@ -354,24 +375,43 @@ __global__ void __launch_bounds__(1024) bmom_x_kernel(const BMomArgs<T> A) {
   __syncthreads();
   const T *const tc = along ? td : tt;
   const MomUpdate<T> &U = A.up;
-  for (int idx = tid; idx < tot; idx += nthr) {
-    const int l = small_div(idx, n, rn), i = idx - l * n;
-    const long long o = base + idx;
-    const T ac = A.acc[comp] ? A.acc[comp][o] : T(0);
-    const T f2 = U.nterms >= 2 ? U.f2[comp][o] : T(0), f3 = U.nterms >= 3 ? U.f3[comp][o] : T(0);
-    const T rot = U.rot[comp] ? U.rot[comp][o] : T(0);
-    const double uo = sizeof(T) == 8 ? (double)tc[l * row + i] : U.u64[comp][o];
-    const T f1 = mom_forced(U, comp, ac + tr[l * row + i], rot);
-    A.out[comp][o] = f1;
-    const int ln = l0 + l, k = ln / U.ny, j = ln - k * U.ny;
-    const double un = pre_correc_point(U, comp, i, j, k, mom_increment(U, f1, f2, f3) + uo);
-    U.u64[comp][o] = un;
-    if constexpr (sizeof(T) == 4) U.u32[comp][o] = (float)un;
+  // the points' indices are worked out again rather than held through the solve
+  int t1 = tid;
+  asm volatile("" : "+v"(t1));
+  constexpr int H = 4;
+#pragma unroll
+  for (int m0 = 0; m0 < L; m0 += H) {
+    T ac[H], f2[H], f3[H], rot[H];
+    double uo[H];
+#pragma unroll
+    for (int h = 0; h < H; ++h) {
+      if (m0 + h >= L) continue;
+      const unsigned e = base + (unsigned)min(t1 + (m0 + h) * nthr, tot - 1), o = e * (unsigned)sizeof(T);
+      ac[h] = A.acc[comp] ? at(A.acc[comp], o) : T(0);
+      f2[h] = U.nterms >= 2 ? at(U.f2[comp], o) : T(0);
+      f3[h] = U.nterms >= 3 ? at(U.f3[comp], o) : T(0);
+      rot[h] = U.rot[comp] ? at(U.rot[comp], o) : T(0);
+      if constexpr (sizeof(T) == 4) uo[h] = U.u64[comp][e];
+    }
+#pragma unroll
+    for (int h = 0; h < H; ++h) {
+      const int idx = t1 + (m0 + h) * nthr;
+      if (m0 + h >= L || idx >= tot) continue;
+      const int l = small_div(idx, n, rn), i = idx - l * n;
+      const unsigned e = base + (unsigned)idx;
+      if constexpr (sizeof(T) == 8) uo[h] = (double)tc[l * row + i];
+      const T f1 = mom_forced(U, comp, ac[h] + tr[l * row + i], rot[h]);
+      at(A.out[comp], e * (unsigned)sizeof(T)) = f1;
+      const int ln = l0 + l, k = ln / U.ny, j = ln - k * U.ny;
+      const double un = pre_correc_point(U, comp, i, j, k, mom_increment(U, f1, f2[h], f3[h]) + uo[h]);
+      U.u64[comp][e] = un;
+      if constexpr (sizeof(T) == 4) at(U.u32[comp], e * (unsigned)sizeof(T)) = (float)un;
+    }
   }
 }
 
 template <typename T>
-static bool bmom_plan(const Context &c, int dir, BoundShape<T> *Y, int *nt) {
+static bool bmom_plan(const Context &c, int dir, BoundPick<T> *Y, int *nt) {
   const DirCoef &D = c.dir[dir];
   const bool same = same_set(c.sets[D.set_d1_even], c.sets[D.set_d1_odd]);
   *nt = same ? 2 : 3;
@@ -382,27 +422,43 @@ static bool bmom_plan(const Context &c, int dir, BoundShape<T> *Y, int *nt) {
   const bool stretched = dir == 1 && c.p.istret != 0;
   return Y->plan(n, *nt, 3, [&](int TL) {
     return dir == 0 ? 2 * (size_t)TL * row : (stretched ? 3 * (size_t)n : (size_t)0);
-  });
+  }) && (dir != 0 || Y->TL * Y->P <= BMOM_FEW);
 }
 
 template <typename T>
 bool bounded_momentum_ok(const Context &c, int dir) {
-  BoundShape<T> Y;
+  BoundPick<T> Y;
   int nt;
   return bmom_plan<T>(c, dir, &Y, &nt);
 }
 template bool bounded_momentum_ok<double>(const Context &, int);
 template bool bounded_momentum_ok<float>(const Context &, int);
 
+template <typename T, int L>
+static void launch_bmom_x(const BMomArgs<T> &A, int nt, dim3 grid, dim3 block, size_t sh, hipStream_t st) {
+  if (nt == 2) hipLaunchKernelGGL((bmom_x_kernel<T, L, 2>), grid, block, sh, st, A);
+  else hipLaunchKernelGGL((bmom_x_kernel<T, L, 3>), grid, block, sh, st, A);
+}
+
+template <typename T, int L>
+static void launch_bmom_yz(const BMomArgs<T> &A, int nt, dim3 grid, dim3 block, size_t sh, hipStream_t st) {
+  const bool few = block.x * block.y <= BMOM_FEW;
+  if (nt == 2 && few) hipLaunchKernelGGL((bmom_yz_kernel<T, L, 2, BMOM_FEW>), grid, block, sh, st, A);
+  else if (nt == 2) hipLaunchKernelGGL((bmom_yz_kernel<T, L, 2, 1024>), grid, block, sh, st, A);
+  else if (few) hipLaunchKernelGGL((bmom_yz_kernel<T, L, 3, BMOM_FEW>), grid, block, sh, st, A);
+  else hipLaunchKernelGGL((bmom_yz_kernel<T, L, 3, 1024>), grid, block, sh, st, A);
+}
+
 template <typename T>
 int launch_bounded_momentum(const Context &c, int dir, const MomIO<T> &io, hipStream_t st) {
   const int nx = c.p.nx, ny = c.p.ny, nz = c.p.nz;
-  BoundShape<T> Y;
+  BoundPick<T> Y;
   int nt = 0;
   if (!bmom_plan<T>(c, dir, &Y, &nt)) return fail(X3D_ERR_UNSUPPORTED, "bounded momentum sweep: line not covered");
   if ((size_t)nx * ny * nz * sizeof(T) >= ((size_t)1 << 32))
     return fail(X3D_ERR_UNSUPPORTED, "bounded momentum sweep: field larger than 4 GiB");
   const DirCoef &D = c.dir[dir];
+  constexpr int L = BoundShape<T>::L;
   BMomArgs<T> A{};
   for (int i = 0; i < 3; ++i) {
     A.u[i] = io.u[i];
@@ -412,8 +468,9 @@ int launch_bounded_momentum(const Context &c, int dir, const MomIO<T> &io, hipSt
   for (int along = 0; along < 2; ++along) {
     // the product u_d u_c is even along d for the component along it, odd
     // otherwise; u_c the other way round (transeq.f90:125-146)
-    const BoundDev<T> t[3] = {bound_dev<T>(c, dir, OP_DER1, along), bound_dev<T>(c, dir, OP_DER1, 1 - along),
-                              bound_dev<T>(c, dir, OP_DER2, 1 - along)};
+    const BoundDev<T> t[3] = {bound_dev<T>(c, dir, OP_DER1, along, Y.longer),
+                              bound_dev<T>(c, dir, OP_DER1, 1 - along, Y.longer),
+                              bound_dev<T>(c, dir, OP_DER2, 1 - along, Y.longer)};
     for (int q = 0; q < 3; ++q) {
       A.pk[along][q] = t[q].pk;
       A.edge[along][q] = t[q].edge;
@@ -431,8 +488,8 @@ int launch_bounded_momentum(const Context &c, int dir, const MomIO<T> &io, hipSt
     A.row = D.n | 1;
     X3D_TRY(fill_update<T>(c, io, &A.up));
     const dim3 grid((A.na + Y.TL - 1) / Y.TL, 1, 3);
-    if (nt == 2) hipLaunchKernelGGL((bmom_x_kernel<T, BoundShape<T>::L, 2>), grid, block, Y.shmem, st, A);
-    else hipLaunchKernelGGL((bmom_x_kernel<T, BoundShape<T>::L, 3>), grid, block, Y.shmem, st, A);
+    if (Y.longer) launch_bmom_x<T, L + 1>(A, nt, grid, block, Y.shmem, st);
+    else launch_bmom_x<T, L>(A, nt, grid, block, Y.shmem, st);
   } else {
     if (io.nterms) return fail(X3D_ERR_ARG, "the velocity update belongs to the x sweep");
     if (dir == 1) {
@@ -447,8 +504,8 @@ int launch_bounded_momentum(const Context &c, int dir, const MomIO<T> &io, hipSt
       A.na = nx * ny; A.nb = 1; A.sb = 0; A.se = (long long)nx * ny;
     }
     const dim3 grid((A.na + Y.TL - 1) / Y.TL, A.nb, 3);
-    if (nt == 2) hipLaunchKernelGGL((bmom_yz_kernel<T, BoundShape<T>::L, 2>), grid, block, Y.shmem, st, A);
-    else hipLaunchKernelGGL((bmom_yz_kernel<T, BoundShape<T>::L, 3>), grid, block, Y.shmem, st, A);
+    if (Y.longer) launch_bmom_yz<T, L + 1>(A, nt, grid, block, Y.shmem, st);
+    else launch_bmom_yz<T, L>(A, nt, grid, block, Y.shmem, st);
   }
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return fail(X3D_ERR_HIP, std::string("bounded momentum launch: ") + hipGetErrorString(e));
@@ -566,11 +623,25 @@ __global__ void __launch_bounds__(1024) bproj_x_kernel(const BProjArgs<T> A) {
   const T *const in = A.in[comp], *const pk = comp == 0 ? A.pkD : A.pkI;
   const long long bi = (long long)l0 * n_in, bo = (long long)l0 * n_out;
   const float rni = 1.0f / (float)n_in, rno = 1.0f / (float)n_out;
-  for (int idx = tid; idx < nl * n_in; idx += nthr) {
-    const int l = small_div(idx, n_in, rni);
-    tile[l * row + idx - l * n_in] = in[bi + idx];
+  const T *const src[1] = {pk};
+  BoundCopy<T, 1> cp;
+  cp.load(src, tid, nthr, CW);
+  {
+    // n_in <= P L + 1: at most L + 1 points a thread (L where n_in < n_out)
+    constexpr int R = PV ? L : L + 1;
+    const int tot = nl * n_in;
+    T r[R];
+#pragma unroll
+    for (int m = 0; m < R; ++m) r[m] = in[bi + min(tid + m * nthr, tot - 1)];
+#pragma unroll
+    for (int m = 0; m < R; ++m) {
+      const int idx = tid + m * nthr;
+      if (idx >= tot) continue;
+      const int l = small_div(idx, n_in, rni);
+      tile[l * row + idx - l * n_in] = r[m];
+    }
   }
-  for (int i = tid; i < CW; i += nthr) cs[i] = pk[i];
+  cp.store(cs, src, tid, nthr, CW);
   __syncthreads();
   const int e0 = bound_first<L>(seg, P, n_out), rows = bound_rows<L>(seg, P, n_out);
   const T *const pl = tile + line * row;
@@ -590,17 +661,30 @@ __global__ void __launch_bounds__(1024) bproj_x_kernel(const BProjArgs<T> A) {
   for (int m = 0; m < L; ++m)
     if (m < rows) tile[line * row + e0 + m] = w[0][m];
   __syncthreads();
-  for (int idx = tid; idx < nl * n_out; idx += nthr) {
+  int t1 = tid;   // as in bmom_x_kernel
+  asm volatile("" : "+v"(t1));
+  const int tot = nl * n_out;
+  T *const out = A.out[comp];
+  double *const u64 = A.cv.u64[comp];
+  double uo[L];
+  if (PV && A.cv.apply) {
+#pragma unroll
+    for (int m = 0; m < L; ++m) uo[m] = u64[bo + min(t1 + m * nthr, tot - 1)];
+  }
+#pragma unroll
+  for (int m = 0; m < L; ++m) {
+    const int idx = t1 + m * nthr;
+    if (idx >= tot) continue;
     const int l = small_div(idx, n_out, rno), i = idx - l * n_out;
     const T g = tile[l * row + i];
     if constexpr (!PV) {
-      A.out[comp][bo + idx] = g;
+      out[bo + idx] = g;
     } else {
       const int ln = l0 + l, k = ln / A.cv.ny, j = ln - k * A.cv.ny;
       store_wall(A.cv, comp, i, j, k, g);
       if (A.cv.apply) {
-        const double u = A.cv.u64[comp][bo + idx] - (double)g;
-        A.cv.u64[comp][bo + idx] = u;
+        const double u = uo[m] - (double)g;
+        u64[bo + idx] = u;
         if (A.cv.u32[comp]) A.cv.u32[comp][bo + idx] = (float)u;
       }
     }
@@ -612,7 +696,7 @@ static int proj_out(const DirCoef &D, bool pv) { return pv ? D.n : D.nm; }
 static int proj_in(const DirCoef &D, bool pv) { return pv ? D.nm : D.n; }
 
 template <typename T>
-static bool bproj_plan(const Context &c, int dir, bool pv, BoundShape<T> *Y) {
+static bool bproj_plan(const Context &c, int dir, bool pv, BoundPick<T> *Y) {
   const DirCoef &D = c.dir[dir];
   const int row = D.n | 1;
   if (dir == 0) return Y->plan(proj_out(D, pv), 1, 1, [&](int TL) { return (size_t)TL * row; });
@@ -621,7 +705,7 @@ static bool bproj_plan(const Context &c, int dir, bool pv, BoundShape<T> *Y) {
 
 template <typename T>
 bool bounded_projection_ok(const Context &c, int dir) {
-  BoundShape<T> Y;
+  BoundPick<T> Y;
   if (!bound_dev<T>(c, dir, OP_DERVP, 0).pk) return false;
   for (int op : {OP_INTERVP, OP_DERPV, OP_INTERPV})
     if (!bound_dev<T>(c, dir, op, 1).pk) return false;
@@ -630,17 +714,33 @@ bool bounded_projection_ok(const Context &c, int dir) {
 template bool bounded_projection_ok<double>(const Context &, int);
 template bool bounded_projection_ok<float>(const Context &, int);
 
+template <typename T, int L>
+static void launch_bproj_x(const BProjArgs<T> &A, bool pv, dim3 grid, dim3 block, size_t sh, hipStream_t st) {
+  if (pv) hipLaunchKernelGGL((bproj_x_kernel<T, L, true>), grid, block, sh, st, A);
+  else hipLaunchKernelGGL((bproj_x_kernel<T, L, false>), grid, block, sh, st, A);
+}
+
+template <typename T, int L>
+static void launch_bproj_yz(const BProjArgs<T> &A, int sw, dim3 grid, dim3 block, size_t sh, hipStream_t st) {
+  switch (sw) {
+    case SW_DIV_Y: hipLaunchKernelGGL((bproj_yz_kernel<T, L, SW_DIV_Y>), grid, block, sh, st, A); break;
+    case SW_DIV_Z: hipLaunchKernelGGL((bproj_yz_kernel<T, L, SW_DIV_Z>), grid, block, sh, st, A); break;
+    case SW_GRAD_Z: hipLaunchKernelGGL((bproj_yz_kernel<T, L, SW_GRAD_Z>), grid, block, sh, st, A); break;
+    default: hipLaunchKernelGGL((bproj_yz_kernel<T, L, SW_GRAD_Y>), grid, block, sh, st, A); break;
+  }
+}
+
 template <typename T>
 int launch_bounded_projection(const Context &c, int sw, const ProjIO<T> &io, hipStream_t st) {
   const int dir = (sw == SW_DIV_X || sw == SW_GRAD_X) ? 0 : (sw == SW_DIV_Y || sw == SW_GRAD_Y) ? 1 : 2;
   const bool pv = sw >= SW_GRAD_Z;
   const DirCoef &D = c.dir[dir];
-  BoundShape<T> Y;
+  BoundPick<T> Y;
   if (!bproj_plan<T>(c, dir, pv, &Y)) return fail(X3D_ERR_UNSUPPORTED, "bounded projection sweep: line not covered");
   if ((size_t)c.p.nx * c.p.ny * c.p.nz * sizeof(T) >= ((size_t)1 << 32))
     return fail(X3D_ERR_UNSUPPORTED, "bounded projection sweep: field larger than 4 GiB");
-  const BoundDev<T> tI = bound_dev<T>(c, dir, pv ? OP_INTERPV : OP_INTERVP, 1);
-  const BoundDev<T> tD = bound_dev<T>(c, dir, pv ? OP_DERPV : OP_DERVP, pv ? 1 : 0);
+  const BoundDev<T> tI = bound_dev<T>(c, dir, pv ? OP_INTERPV : OP_INTERVP, 1, Y.longer);
+  const BoundDev<T> tD = bound_dev<T>(c, dir, pv ? OP_DERPV : OP_DERVP, pv ? 1 : 0, Y.longer);
   BProjArgs<T> A{};
   for (int i = 0; i < 3; ++i) {
     A.in[i] = io.in[i];
@@ -664,8 +764,8 @@ int launch_bounded_projection(const Context &c, int sw, const ProjIO<T> &io, hip
     A.row = D.n | 1;
     if (pv) X3D_TRY(fill_corvel<T>(c, io, &A.cv));
     const dim3 grid((A.na + Y.TL - 1) / Y.TL, 1, 3);
-    if (pv) hipLaunchKernelGGL((bproj_x_kernel<T, L, true>), grid, block, Y.shmem, st, A);
-    else hipLaunchKernelGGL((bproj_x_kernel<T, L, false>), grid, block, Y.shmem, st, A);
+    if (Y.longer) launch_bproj_x<T, L + 1>(A, pv, grid, block, Y.shmem, st);
+    else launch_bproj_x<T, L>(A, pv, grid, block, Y.shmem, st);
   } else {
     if (dir == 1) {
       // x is on the pressure grid; z on the velocity grid in both passes
@@ -680,12 +780,8 @@ int launch_bounded_projection(const Context &c, int sw, const ProjIO<T> &io, hip
       A.divp = io.divp;
       if (io.divp_blocks) *io.divp_blocks = (int)(grid.x * grid.y);
     }
-    switch (sw) {
-      case SW_DIV_Y: hipLaunchKernelGGL((bproj_yz_kernel<T, L, SW_DIV_Y>), grid, block, Y.shmem, st, A); break;
-      case SW_DIV_Z: hipLaunchKernelGGL((bproj_yz_kernel<T, L, SW_DIV_Z>), grid, block, Y.shmem, st, A); break;
-      case SW_GRAD_Z: hipLaunchKernelGGL((bproj_yz_kernel<T, L, SW_GRAD_Z>), grid, block, Y.shmem, st, A); break;
-      default: hipLaunchKernelGGL((bproj_yz_kernel<T, L, SW_GRAD_Y>), grid, block, Y.shmem, st, A); break;
-    }
+    if (Y.longer) launch_bproj_yz<T, L + 1>(A, sw, grid, block, Y.shmem, st);
+    else launch_bproj_yz<T, L>(A, sw, grid, block, Y.shmem, st);
   }
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return fail(X3D_ERR_HIP, std::string("bounded projection launch: ") + hipGetErrorString(e));

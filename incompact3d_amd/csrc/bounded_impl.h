@@ -331,6 +331,39 @@ struct BoundShape {
   }
 };
 
+// Segment length of a sweep: one row longer where a block's lines then need
+// fewer wavefronts on the fullest of a compute unit's four SIMDs.  Bounded
+// lines have 2^k + 1 points: in segments of 8 rows 129 points take 17 x 16
+// threads, a fifth wavefront for the last segment, and 6.8 wavefronts a
+// compute unit were resident on average; in segments of 9 rows they take
+// 15 x 16, four wavefronts.  256 x 129 x 128: y momentum sweep FP64 124 -> 84,
+// FP32 64 -> 44 us, y gradient sweep 54 -> 45 and 31 -> 21 us.  Where the count
+// a SIMD stays (65 points: 3 wavefronts or 2) the shorter segments are as fast
+// (momentum) or faster (gradient 8.9 against 9.8, 6.6 against 8.0 us at 65^3).
+template <typename T>
+struct BoundPick {
+  bool longer = false;
+  int P = 0, TL = 0;
+  size_t shmem = 0;
+  template <typename F>
+  bool plan(int n_out, int nt, int nrhs, F extra) {
+    BoundShape<T> Y;
+    BoundShape<T, BoundShape<T>::L + 1> Z;
+    if (!Y.plan(n_out, nt, nrhs, extra)) return false;
+    P = Y.P; TL = Y.TL; shmem = Y.shmem;
+    // (a block has a thread for each row of a line)
+    if (Z.plan(n_out, nt, nrhs, extra) && Z.TL * Z.P >= n_out &&
+        (Z.TL * Z.P + 255) / 256 * Y.TL < (Y.TL * Y.P + 255) / 256 * Z.TL) {
+      longer = true;
+      P = Z.P; TL = Z.TL; shmem = Z.shmem;
+    }
+    return true;
+  }
+  bool plan(int n_out, int nt, int nrhs) {
+    return plan(n_out, nt, nrhs, [](int) { return (size_t)0; });
+  }
+};
+
 // ---------------------------------------------------------------- velocity update
 // What the x momentum sweep does with a finished right-hand side besides
 // storing it, on boxes with bounded directions and in RK3: the channel's

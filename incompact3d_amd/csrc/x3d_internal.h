@@ -100,8 +100,8 @@ struct DirCoef {
 
 // Tables of one operator on anchored segments (bounded_impl.h): padded packed
 // factors and closure weights, segments and chain depth; [0] segments of the
-// precision's length, [1] one row longer (where blocks of the first would have
-// more than 1024 threads).  set64, set32: the coefficient set they are of, and
+// precision's length, [1] one row longer (BoundPick; single operators where
+// blocks of the first would have more than 1024 threads).  set64, set32: the coefficient set they are of, and
 // the first one of the direction with the same coefficients, which is what a
 // caller's arrays are matched to.
 template <typename T>

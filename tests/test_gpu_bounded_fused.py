@@ -38,6 +38,10 @@ CASES = {
     "wall-s3-256": dict(nx=256, ny=129, nz=16, itimescheme=5, istret=3, **WALL),
     "wall-free-x": dict(nx=33, ny=33, nz=32, itimescheme=5, **{**WALL, "nclx1": 1, "nclxn": 1}),
     "wall-free-yn": dict(nx=64, ny=33, nz=16, itimescheme=5, **{**WALL, "nclyn": 1}),
+    # segments one row longer in x; blocks over 512 threads
+    "free-x-129": dict(nx=129, ny=32, nz=16, nclx1=1, nclxn=1, xlx=math.pi, itimescheme=5),
+    "free-y-513": dict(nx=64, ny=513, nz=16, ncly1=1, nclyn=1, yly=math.pi, itimescheme=5),
+    "wall-s2-513": dict(nx=64, ny=513, nz=16, itimescheme=3, istret=2, isecondder=5, **{**WALL, "dt": 5e-4}),
     "free-y1-wall-yn": dict(nx=64, ny=65, nz=16, itimescheme=3, **{**WALL, "ncly1": 1}),
 }
 
