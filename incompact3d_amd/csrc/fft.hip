@@ -1003,25 +1003,39 @@ static void build_penta_factors(const Context &c, const PoissonPlan &P, const st
 
 // One thread per real or imaginary part of (kx, kz, system), the two in
 // neighbouring lanes (they share the factors' loads): forward elimination with
-// the stored multipliers (the scaled right-hand side read once, the
-// eliminated values written back), then the last 2x2 block and the back
-// substitution.  The (nx/2+1, :, nz/2+1) line is zeroed (poisson.f90:902-908).
-// The chain along a line is serial and a 256x129x128 grid has only a
-// thousand wavefronts of lines, so the kernel's time is the latency of its
-// loads: rows are read PENTA_C at a time, the next group while the last one is
-// worked on (62 -> 45 us FP64, 55 -> 37 us FP32 on that grid; groups of 16: 60
-// and 39 us).
+// the stored multipliers (the scaled right-hand side read once), then the last
+// 2x2 block and the back substitution.  The (nx/2+1, :, nz/2+1) line is zeroed
+// (poisson.f90:902-908).
+//
+// Bound by memory: the chain along a line is serial and a 256x129x128 grid has
+// only a thousand wavefronts of lines, so rows are read PENTA_C at a time, the
+// next group while the last one is worked on (groups of 16 are slower).  LDS:
+// the eliminated values stay there (in T, as they would in memory) instead of
+// going out and coming back, where a wavefront's lines are at most
+// PENTA_LDS bytes: five blocks a compute unit.  kz and nz-kz share one factor
+// plane: blocks eight apart, on one XCD, have the same lines of the two, so
+// that its L2 serves the second one; tiles of 32 lines run through the planes
+// and stay on an XCD with their neighbours, whose cache lines they share.
+// 256x129x128: 45 -> 36 us FP64, 37 -> 32 us FP32 (at 32 KB a block, which
+// leaves room for four, FP64 took two rounds and 48 us); 62 and 55 without the
+// rows in flight.
 constexpr int PENTA_C = 8;
-template <typename T>
+constexpr size_t PENTA_LDS = 31 * 1024;
+template <typename T, bool LDS>
 __global__ void __launch_bounds__(64) penta_y_kernel(cplx<T> *__restrict__ cw, const double *__restrict__ pf,
                                                      size_t stride, int nxh, int np, int ny, int nz, int nsys,
-                                                     double scale) {
-  const int tid = blockIdx.x * blockDim.x + threadIdx.x;
-  const int kx = tid >> 1, part = tid & 1;
-  const int kz = blockIdx.y / nsys, par = blockIdx.y - kz * nsys;
-  if (kx >= nxh) return;
+                                                     double scale, int tiles) {
+  extern __shared__ __align__(16) unsigned char penta_raw[];
+  T *const keep = reinterpret_cast<T *>(penta_raw) + threadIdx.x;   // [row][64]
+  const int unit = (int)(blockIdx.x & 7) * (int)(gridDim.x >> 4) + (int)(blockIdx.x >> 4);
+  const int par = unit / tiles;
+  const int l = (unit - par * tiles) * 32 + (int)(threadIdx.x >> 1), part = threadIdx.x & 1;
+  const int kzp = l / nxh, kx = l - kzp * nxh;   // factor plane
+  if (par >= nsys || 2 * kzp > nz) return;
+  const bool mirror = blockIdx.x & 8;
+  if (mirror && (kzp == 0 || 2 * kzp == nz)) return;
+  const int kz = mirror ? nz - kzp : kzp;
   const int nh = ny / nsys, n = nh - 1;
-  const int kzp = kz <= nz - kz ? kz : nz - kz;   // factor plane: kz and nz-kz share one
   const size_t line = ((size_t)(kzp * nsys + par) * nh) * nxh + kx;
   const double *F1 = pf + line, *F2 = pf + stride + line, *RP = pf + 2 * stride + line;
   const double *A1 = pf + 3 * stride + line, *B1 = pf + 4 * stride + line;
@@ -1064,7 +1078,8 @@ __global__ void __launch_bounds__(64) penta_y_kernel(cplx<T> *__restrict__ cw, c
         double e2 = (double)cv[q] * scale;
         e1 = e1 - c1[q] * e0;
         e2 = e2 - c2[q] * e0;
-        v[(size_t)m * sv] = (T)e0;
+        if constexpr (LDS) keep[64 * m] = (T)e0;
+        else v[(size_t)m * sv] = (T)e0;
         e0 = e1;
         e1 = e2;
       }
@@ -1085,7 +1100,7 @@ __global__ void __launch_bounds__(64) penta_y_kernel(cplx<T> *__restrict__ cw, c
 #pragma unroll
       for (int q = 0; q < C; ++q) {
         const int i = i0 - q > 0 ? i0 - q : 0;
-        pv[q] = v[(size_t)i * sv];
+        if constexpr (!LDS) pv[q] = v[(size_t)i * sv];
         pr[q] = RP[(size_t)i * nxh];
         pa[q] = A1[(size_t)i * nxh];
         pb[q] = B1[(size_t)i * nxh];
@@ -1097,7 +1112,8 @@ __global__ void __launch_bounds__(64) penta_y_kernel(cplx<T> *__restrict__ cw, c
       double cr[C], ca[C], cb[C];
 #pragma unroll
       for (int q = 0; q < C; ++q) {
-        cv[q] = pv[q];
+        if constexpr (LDS) cv[q] = keep[64 * (i0 - q > 0 ? i0 - q : 0)];
+        else cv[q] = pv[q];
         cr[q] = pr[q];
         ca[q] = pa[q];
         cb[q] = pb[q];
@@ -1365,9 +1381,15 @@ int poisson_run(const Context &c, T *rhs, void *work, size_t bytes, hipStream_t 
     // stretched y: z transform, pentadiagonal solves along y, inverse z
     ok = ok && dispatch_s<T, FFT_Z_FWD>(P->nz, *P, cw, tb, st);
     if (ok) {
-      const dim3 grid((2 * P->nxh + 63) / 64, P->ystret * P->nz), block(64);
-      hipLaunchKernelGGL((penta_y_kernel<T>), grid, block, 0, st, cw, P->pf, P->pf_stride, P->nxh, P->np,
-                         P->ny, P->nz, P->ystret, P->scale);
+      const int tiles = (P->nxh * (P->nz / 2 + 1) + 31) / 32;
+      const dim3 grid((tiles * P->ystret + 7) / 8 * 16), block(64);
+      const size_t lds = (size_t)(P->ny / P->ystret - 2) * 64 * sizeof(T);
+      if (lds <= PENTA_LDS)
+        hipLaunchKernelGGL((penta_y_kernel<T, true>), grid, block, lds, st, cw, P->pf, P->pf_stride, P->nxh, P->np,
+                           P->ny, P->nz, P->ystret, P->scale, tiles);
+      else
+        hipLaunchKernelGGL((penta_y_kernel<T, false>), grid, block, 0, st, cw, P->pf, P->pf_stride, P->nxh, P->np,
+                           P->ny, P->nz, P->ystret, P->scale, tiles);
     }
     ok = ok && dispatch_s<T, FFT_Z_INV>(P->nz, *P, cw, tb, st);
   } else {
