@@ -57,9 +57,10 @@ int launch_finish_absmax(const double *partial, int nb, size_t n, double *out2, 
 // channel.hip
 int launch_channel_init(double *ux, double *uy, double *uz, const double *yc, int nx, int ny, int nz, double noise,
                         unsigned long long seed, hipStream_t st);
-int launch_bulk(const double *u, const double *ppy, int nx, int ny, int nz, double coeff, double constant,
-                double *partial, double *out2, hipStream_t st);
-int launch_cfr_shift(double *u, float *u32, const double *out2, size_t n, hipStream_t st);
+int launch_bulk(const double *u, const double *ppy, int nx, int ny, int nz, double coeff, double *partial,
+                double *out, hipStream_t st);
+int launch_cfr(double *u, float *u32, const double *ppy, int nx, int ny, int nz, double coeff, double constant,
+               double *partial, hipStream_t st);
 template <typename T>
 int launch_add_const(T *f, double c, size_t n, hipStream_t st);
 template <typename T>
@@ -398,9 +399,8 @@ int pre_correc(const Context &c, x3d_solver *S, double gdt) {
 int channel_cfr(const Context &c, x3d_solver *S) {
   if (S->forcing != 1) return X3D_OK;
   const double coeff = c.dir[1].d / (c.p.yly * (double)((long long)S->nx * S->nz));
-  X3D_TRY(launch_bulk(S->u64[0], c.p.istret != 0 ? c.ppy64 : nullptr, S->nx, S->ny, S->nz, coeff, S->fvalue,
-                      S->partial, S->red, c.stream));
-  return launch_cfr_shift(S->u64[0], S->u32[0], S->red, S->n, c.stream);
+  return launch_cfr(S->u64[0], S->u32[0], c.p.istret != 0 ? c.ppy64 : nullptr, S->nx, S->ny, S->nz, coeff, S->fvalue,
+                    S->partial, c.stream);
 }
 
 // momentum_forcing_channel (Case-Channel.f90:396-420) on component comp's
@@ -1101,7 +1101,7 @@ int x3d_solver_bulk_velocity(x3d_solver *S, double *ub) {
   if (!S || !ub) return fail(X3D_ERR_ARG, "null pointer");
   const double coeff = c->dir[1].d / (c->p.yly * (double)((long long)S->nx * S->nz));
   X3D_TRY(sync_velocity(*c, S));
-  X3D_TRY(launch_bulk(S->u64[0], c->p.istret != 0 ? c->ppy64 : nullptr, S->nx, S->ny, S->nz, coeff, 0.0, S->partial,
+  X3D_TRY(launch_bulk(S->u64[0], c->p.istret != 0 ? c->ppy64 : nullptr, S->nx, S->ny, S->nz, coeff, S->partial,
                       S->red, c->stream));
   X3D_HIP(hipMemcpyAsync(ub, S->red, sizeof(double), hipMemcpyDeviceToHost, c->stream));
   X3D_HIP(hipStreamSynchronize(c->stream));
