@@ -193,97 +193,126 @@ __device__ __forceinline__ void mom_line(const MomArgs<T> &A, const LineCoef<T, 
 
 // ---------------------------------------------------------------- x sweep (one wavefront per line)
 // GEN: the general velocity update (RK3, bounded y or z) in place of plain AB3.
-template <typename T, int V, bool GEN>
+// ALL: a wavefront takes the three components of a line one after another, else
+// that of blockIdx.z.  Bound by memory, 18 fields in all (20 with u_x read for
+// each component): 256^3 FP64 494 -> 441 us (5.5 TB/s), FP32 283 -> 251, the
+// channel's 256x129x128 FP64 133 -> 110.
+template <typename T, int V, bool GEN, bool ALL>
 __global__ void __launch_bounds__(256) mom_x_kernel(const MomArgs<T> A, int nlines) {
   const int lane = threadIdx.x & 63;
   const int wave = (blockIdx.x * blockDim.x + threadIdx.x) >> 6;
   const int nwaves = (gridDim.x * blockDim.x) >> 6;
   const int n = A.n;
   const int e0 = lane * V;
-  const int comp = (int)blockIdx.z;
-  const T *const uc_in = A.uc[comp], *const acc_in = A.acc[comp], *const f2_in = A.f2[comp],
-                *const f3_in = A.f3[comp];
   LineCoef<T, V> C;
   C.load(A, lane);
-  // the next line's velocities are loaded before this line is solved, so
-  // that their latency overlaps the solves (each wave loops over several lines)
-  T pud[V], puc[V];
+  // the next velocities (u_x of the next line last) are loaded before this
+  // component is solved, so that their latency overlaps the solves (each wave
+  // loops over several lines)
+  T ud[V], uc[V], nx[V], nd[V];
+  const int c0 = ALL ? 0 : (int)blockIdx.z, c1 = ALL ? 3 : c0 + 1;
   if (wave < nlines) {
-    load_run<T, V>(A.ud + (long long)wave * n + e0, pud);
-    load_run<T, V>(uc_in + (long long)wave * n + e0, puc);
+    load_run<T, V>(A.ud + (long long)wave * n + e0, nd);
+    if constexpr (!ALL) load_run<T, V>(A.uc[c0] + (long long)wave * n + e0, nx);
   }
   for (int ln = wave; ln < nlines; ln += nwaves) {
     const long long base = (long long)ln * n + e0;
-    T ud[V], uc[V];
 #pragma unroll
-    for (int m = 0; m < V; ++m) { ud[m] = pud[m]; uc[m] = puc[m]; }
-    if (ln + nwaves < nlines) {
-      load_run<T, V>(A.ud + (long long)(ln + nwaves) * n + e0, pud);
-      load_run<T, V>(uc_in + (long long)(ln + nwaves) * n + e0, puc);
-    }
-    T r[V];
-    mom_line<T, V>(A, C, ud, uc, r, lane);
-    // every epilogue input is read before the first store (the compiler
-    // cannot move loads above stores to possibly aliasing arrays)
-    T acc[V], f2[V], f3[V];
-    if constexpr (GEN) {
-      const MomUpdate<T> &U = A.up;
-      T rot[V];
-      double un[V];
-      load_run<T, V>(acc_in + base, acc);
-      if (U.nterms >= 2) load_run<T, V>(U.f2[comp] + base, f2);
-      if (U.nterms >= 3) load_run<T, V>(U.f3[comp] + base, f3);
-      if (U.rot[comp]) load_run<T, V>(U.rot[comp] + base, rot);
-      if constexpr (sizeof(T) == 4) load_run<double, V>(U.u64[comp] + base, un);
-      const int lu = __builtin_amdgcn_readfirstlane(ln), k = lu / U.ny, j = lu - k * U.ny;
+    for (int m = 0; m < V; ++m) ud[m] = nd[m];
+#pragma unroll 1
+    for (int comp = c0; comp < c1; ++comp) {
+      const T *const acc_in = A.acc[comp], *const f2_in = A.f2[comp], *const f3_in = A.f3[comp];
+      const bool more = ln + nwaves < nlines;
+      if constexpr (ALL) {
+        if (comp == 0) {
 #pragma unroll
-      for (int m = 0; m < V; ++m) {
-        r[m] = mom_forced(U, comp, acc[m] + r[m], rot[m]);
-        const double uo = sizeof(T) == 8 ? (double)uc[m] : un[m];
-        un[m] = pre_correc_point(U, comp, e0 + m, j, k, mom_increment(U, r[m], f2[m], f3[m]) + uo);
-      }
-      store_run<T, V>(A.out[comp] + base, r);
-      store_run<double, V>(U.u64[comp] + base, un);
-      if constexpr (sizeof(T) == 4) {
-        float sh[V];
+          for (int m = 0; m < V; ++m) uc[m] = ud[m];
+        } else {
 #pragma unroll
-        for (int m = 0; m < V; ++m) sh[m] = (float)un[m];
-        store_run<float, V>(U.u32[comp] + base, sh);
-      }
-      continue;
-    }
-    if (acc_in) load_run<T, V>(acc_in + base, acc);
-    if (A.nterms >= 2) load_run<T, V>(f2_in + base, f2);
-    if (A.nterms >= 3) load_run<T, V>(f3_in + base, f3);
-    if (acc_in) {
-#pragma unroll
-      for (int m = 0; m < V; ++m) r[m] = acc[m] + r[m];
-    }
-    store_run<T, V>(A.out[comp] + base, r);
-    if (A.nterms) {
-      // AB3 with FP64 accumulation: du = a f1 + b f2 + c f3, u_new = du + u_old
-      double du[V];
-#pragma unroll
-      for (int m = 0; m < V; ++m) {
-        if (A.nterms == 1) du[m] = A.ca * (double)r[m];
-        else if (A.nterms == 2) du[m] = A.ca * (double)r[m] + A.cb * (double)f2[m];
-        else du[m] = A.ca * (double)r[m] + A.cb * (double)f2[m] + A.cc * (double)f3[m];
-      }
-      if constexpr (sizeof(T) == 8) {
-        // u_c is the FP64 velocity itself
-        double un[V];
-#pragma unroll
-        for (int m = 0; m < V; ++m) un[m] = du[m] + (double)uc[m];
-        store_run<double, V>(A.u_new[comp] + base, un);
+          for (int m = 0; m < V; ++m) uc[m] = nx[m];
+        }
+        if (comp < 2) load_run<T, V>(A.uc[comp + 1] + base, nx);
+        else if (more) load_run<T, V>(A.ud + base + (long long)nwaves * n, nd);
       } else {
-        float d[V], sh[V];
+#pragma unroll
+        for (int m = 0; m < V; ++m) uc[m] = nx[m];
+        if (more) {
+          load_run<T, V>(A.ud + base + (long long)nwaves * n, nd);
+          load_run<T, V>(A.uc[comp] + base + (long long)nwaves * n, nx);
+        }
+      }
+      // every epilogue input is read before the first store (the compiler
+      // cannot move loads above stores to possibly aliasing arrays), and ahead
+      // of the solves where there are registers for it
+      constexpr bool EARLY = V * sizeof(T) <= 32;
+      T r[V], acc[V], f2[V], f3[V], rot[V];
+      double un[V];
+      auto inputs = [&] {
+        if constexpr (GEN) {
+          const MomUpdate<T> &U = A.up;
+          load_run<T, V>(acc_in + base, acc);
+          if (U.nterms >= 2) load_run<T, V>(U.f2[comp] + base, f2);
+          if (U.nterms >= 3) load_run<T, V>(U.f3[comp] + base, f3);
+          if (U.rot[comp]) load_run<T, V>(U.rot[comp] + base, rot);
+          if constexpr (sizeof(T) == 4) load_run<double, V>(U.u64[comp] + base, un);
+        } else {
+          if (acc_in) load_run<T, V>(acc_in + base, acc);
+          if (A.nterms >= 2) load_run<T, V>(f2_in + base, f2);
+          if (A.nterms >= 3) load_run<T, V>(f3_in + base, f3);
+        }
+      };
+      if constexpr (EARLY) inputs();
+      mom_line<T, V>(A, C, ud, uc, r, lane);
+      if constexpr (!EARLY) inputs();
+      if constexpr (GEN) {
+        const MomUpdate<T> &U = A.up;
+        const int lu = __builtin_amdgcn_readfirstlane(ln), k = lu / U.ny, j = lu - k * U.ny;
 #pragma unroll
         for (int m = 0; m < V; ++m) {
-          d[m] = (float)du[m];
-          sh[m] = (float)(du[m] + (double)uc[m]);
+          r[m] = mom_forced(U, comp, acc[m] + r[m], rot[m]);
+          const double uo = sizeof(T) == 8 ? (double)uc[m] : un[m];
+          un[m] = pre_correc_point(U, comp, e0 + m, j, k, mom_increment(U, r[m], f2[m], f3[m]) + uo);
         }
-        store_run<float, V>(A.delta[comp] + base, d);
-        store_run<float, V>(A.shadow[comp] + base, sh);
+        store_run<T, V>(A.out[comp] + base, r);
+        store_run<double, V>(U.u64[comp] + base, un);
+        if constexpr (sizeof(T) == 4) {
+          float sh[V];
+#pragma unroll
+          for (int m = 0; m < V; ++m) sh[m] = (float)un[m];
+          store_run<float, V>(U.u32[comp] + base, sh);
+        }
+        continue;
+      }
+      if (acc_in) {
+#pragma unroll
+        for (int m = 0; m < V; ++m) r[m] = acc[m] + r[m];
+      }
+      store_run<T, V>(A.out[comp] + base, r);
+      if (A.nterms) {
+        // AB3 with FP64 accumulation: du = a f1 + b f2 + c f3, u_new = du + u_old
+        double du[V];
+#pragma unroll
+        for (int m = 0; m < V; ++m) {
+          if (A.nterms == 1) du[m] = A.ca * (double)r[m];
+          else if (A.nterms == 2) du[m] = A.ca * (double)r[m] + A.cb * (double)f2[m];
+          else du[m] = A.ca * (double)r[m] + A.cb * (double)f2[m] + A.cc * (double)f3[m];
+        }
+        if constexpr (sizeof(T) == 8) {
+          // u_c is the FP64 velocity itself
+          double un[V];
+#pragma unroll
+          for (int m = 0; m < V; ++m) un[m] = du[m] + (double)uc[m];
+          store_run<double, V>(A.u_new[comp] + base, un);
+        } else {
+          float d[V], sh[V];
+#pragma unroll
+          for (int m = 0; m < V; ++m) {
+            d[m] = (float)du[m];
+            sh[m] = (float)(du[m] + (double)uc[m]);
+          }
+          store_run<float, V>(A.delta[comp] + base, d);
+          store_run<float, V>(A.shadow[comp] + base, sh);
+        }
       }
     }
   }
@@ -320,13 +349,13 @@ bool momentum_fusable(const Context &c) {
   return true;
 }
 
-template <typename T, bool GEN>
+template <typename T, bool GEN, bool ALL>
 static void launch_mom_x(const MomArgs<T> &A, int V, int nlines, dim3 grid, dim3 block, hipStream_t st) {
   switch (V) {
-    case 1: hipLaunchKernelGGL((mom_x_kernel<T, 1, GEN>), grid, block, 0, st, A, nlines); break;
-    case 2: hipLaunchKernelGGL((mom_x_kernel<T, 2, GEN>), grid, block, 0, st, A, nlines); break;
-    case 4: hipLaunchKernelGGL((mom_x_kernel<T, 4, GEN>), grid, block, 0, st, A, nlines); break;
-    default: hipLaunchKernelGGL((mom_x_kernel<T, 8, GEN>), grid, block, 0, st, A, nlines); break;
+    case 1: hipLaunchKernelGGL((mom_x_kernel<T, 1, GEN, ALL>), grid, block, 0, st, A, nlines); break;
+    case 2: hipLaunchKernelGGL((mom_x_kernel<T, 2, GEN, ALL>), grid, block, 0, st, A, nlines); break;
+    case 4: hipLaunchKernelGGL((mom_x_kernel<T, 4, GEN, ALL>), grid, block, 0, st, A, nlines); break;
+    default: hipLaunchKernelGGL((mom_x_kernel<T, 8, GEN, ALL>), grid, block, 0, st, A, nlines); break;
   }
 }
 
@@ -374,15 +403,24 @@ int launch_momentum(const Context &c, int dir, const MomIO<T> &io, int nx, int n
       if (io.nterms && (sizeof(T) == 8 ? !io.u_new[i] : (!io.delta[i] || !io.shadow[i])))
         return fail(X3D_ERR_ARG, "momentum: AB3 output buffers missing");
     const int nlines = ny * nz;
-    const int waves = nlines < 8192 ? nlines : 8192;
-    const dim3 grid((waves + 3) / 4, 1, 3), block(256);
+    // Up to 8192 lines there are too few wavefronts to put a line's components
+    // into one (128 x 64^2: 1715 us a step against 1740; 128^3 with 16384 lines:
+    // 1532 against 1510).  The wavefronts' lines are of one number each; FP64
+    // has two wavefronts a SIMD and gains from the loads ahead (256^3: 441 us
+    // with 8192, 475 with 65536), FP32 from more of them (267 and 251).
+    const bool all = nlines > 8192;
+    const int most = sizeof(T) == 8 ? 8192 : 65536, per = (nlines + most - 1) / most;
+    const int waves = (nlines + per - 1) / per;
+    const dim3 grid((waves + 3) / 4, 1, all ? 1 : 3), block(256);
     if (io.general) {
       X3D_TRY(fill_update<T>(c, io, &A.up));
       for (int i = 0; i < 3; ++i)
         if (!io.acc[i]) return fail(X3D_ERR_ARG, "momentum: the x sweep comes last");
-      launch_mom_x<T, true>(A, V, nlines, grid, block, st);
+      if (all) launch_mom_x<T, true, true>(A, V, nlines, grid, block, st);
+      else launch_mom_x<T, true, false>(A, V, nlines, grid, block, st);
     } else {
-      launch_mom_x<T, false>(A, V, nlines, grid, block, st);
+      if (all) launch_mom_x<T, false, true>(A, V, nlines, grid, block, st);
+      else launch_mom_x<T, false, false>(A, V, nlines, grid, block, st);
     }
   } else {
     if (io.nterms) return fail(X3D_ERR_ARG, "AB3 is fused into the x sweep only");
