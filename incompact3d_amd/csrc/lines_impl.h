@@ -1142,6 +1142,79 @@ __device__ __forceinline__ void store_run(T *__restrict__ p, const T (&in)[V]) {
 }
 
 
+// A line of 64 V points between memory order (PER consecutive points a lane and
+// access, so that a wavefront's access covers one piece of memory) and run
+// order (V consecutive points a lane), through the wavefront's own piece of
+// LDS: chunks of PER points, one chunk's gap after every 16 (run order reads
+// them Q apart).  In run order a lane's 16-byte accesses are V points apart:
+// 512^3 FP64 x lines, 64 bytes apart, 490 -> 389 (derx) and 406 us (derxx) in
+// memory order; 256-point lines, 32 bytes apart, 54 -> 47 and 63 -> 52.
+template <typename T, int V, int PER>
+struct LineTile {
+  static constexpr int Q = V / PER, WORDS = Q > 1 ? 68 * V : 1;
+  static_assert(Q * PER == V, "whole chunks");
+  T *p;                          // WORDS
+  int lane;
+  __device__ __forceinline__ LineTile(T *all) : p(all + (threadIdx.x >> 6) * WORDS), lane(threadIdx.x & 63) {}
+  // point of the line that element m is in memory order
+  __device__ __forceinline__ int point(int m) const { return ((m / PER) * 64 + lane) * PER + m % PER; }
+  __device__ __forceinline__ static int pos(int c) { return (c + (c >> 4)) * PER; }
+  __device__ __forceinline__ static void fence() {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+  }
+  template <typename S>
+  __device__ __forceinline__ void load(const S *__restrict__ line, S (&mem)[V]) const {
+#pragma unroll
+    for (int q = 0; q < Q; ++q) {
+      S x[PER];
+      load_run<S, PER>(line + (q * 64 + lane) * PER, x);
+#pragma unroll
+      for (int r = 0; r < PER; ++r) mem[q * PER + r] = x[r];
+    }
+  }
+  template <typename S>
+  __device__ __forceinline__ void store(S *__restrict__ line, const S (&mem)[V]) const {
+#pragma unroll
+    for (int q = 0; q < Q; ++q) {
+      S x[PER];
+#pragma unroll
+      for (int r = 0; r < PER; ++r) x[r] = mem[q * PER + r];
+      store_run<S, PER>(line + (q * 64 + lane) * PER, x);
+    }
+  }
+  __device__ __forceinline__ void to_run(const T (&mem)[V], T (&run)[V]) const {
+    move<true>(mem, run);
+  }
+  __device__ __forceinline__ void to_memory(const T (&run)[V], T (&mem)[V]) const {
+    move<false>(run, mem);
+  }
+  template <bool RUN>
+  __device__ __forceinline__ void move(const T (&from)[V], T (&to)[V]) const {
+    if constexpr (Q == 1) {
+#pragma unroll
+      for (int m = 0; m < V; ++m) to[m] = from[m];
+    } else {
+#pragma unroll
+      for (int q = 0; q < Q; ++q) {
+        T x[PER];
+#pragma unroll
+        for (int r = 0; r < PER; ++r) x[r] = from[q * PER + r];
+        store_run<T, PER>(p + pos(RUN ? q * 64 + lane : lane * Q + q), x);
+      }
+      fence();
+#pragma unroll
+      for (int q = 0; q < Q; ++q) {
+        T x[PER];
+        load_run<T, PER>(p + pos(RUN ? lane * Q + q : q * 64 + lane), x);
+#pragma unroll
+        for (int r = 0; r < PER; ++r) to[q * PER + r] = x[r];
+      }
+      fence();
+    }
+  }
+};
+
 template <typename T, int OP, int V, bool EPI>
 __global__ void __launch_bounds__(256) xwave_kernel(const LineArgs<T> A, int nlines) {
   constexpr int HL = Halo<OP>::L, HR = Halo<OP>::R, W = V + HL + HR;
@@ -1176,24 +1249,27 @@ __global__ void __launch_bounds__(256) xwave_kernel(const LineArgs<T> A, int nli
       sm[m] = A.pk[4 * e + 3];
     }
   }
+  constexpr int PER = V * sizeof(T) > 16 ? 16 / (int)sizeof(T) : V;
+  using Tile = LineTile<T, V, PER>;
+  __shared__ __align__(16) T lines[4 * Tile::WORDS];
+  const Tile tile(lines);
   // the next line's input is loaded while the current one is solved
   T nxt_u[V], nxt_u2[V];
   if (wave < nlines) {
-    load_run<T, V>(u + (long long)wave * n + e0, nxt_u);
-    if (EPI && A.u2) load_run<T, V>(A.u2 + (long long)wave * n + e0, nxt_u2);
+    tile.load(u + (long long)wave * n, nxt_u);
+    if (EPI && A.u2) tile.load(A.u2 + (long long)wave * n, nxt_u2);
   }
   for (int ln = wave; ln < nlines; ln += nwaves) {
-    const long long base = (long long)ln * n + e0;
+    const long long base = (long long)ln * n;
     T own[V];
-#pragma unroll
-    for (int m = 0; m < V; ++m) own[m] = nxt_u[m];
     if (EPI && A.u2) {
 #pragma unroll
-      for (int m = 0; m < V; ++m) own[m] *= nxt_u2[m];
+      for (int m = 0; m < V; ++m) nxt_u[m] *= nxt_u2[m];
     }
+    tile.to_run(nxt_u, own);
     if (ln + nwaves < nlines) {
-      load_run<T, V>(u + base + (long long)nwaves * n, nxt_u);
-      if (EPI && A.u2) load_run<T, V>(A.u2 + base + (long long)nwaves * n, nxt_u2);
+      tile.load(u + base + (long long)nwaves * n, nxt_u);
+      if (EPI && A.u2) tile.load(A.u2 + base + (long long)nwaves * n, nxt_u2);
     }
     // window U(e0-HL .. e0+V+HR-1): own points plus neighbour lanes' points
     T v[W];
@@ -1215,15 +1291,12 @@ __global__ void __launch_bounds__(256) xwave_kernel(const LineArgs<T> A, int nli
       }
     }
     wave_solve<T, V>(r, fs, fw, ffw, sm, A.alfa, A.rden, lane);
-#pragma unroll
-    for (int m = 0; m < V; ++m) v[m] = r[m];
     // epilogue and store
     T res[V];
-#pragma unroll
-    for (int m = 0; m < V; ++m) res[m] = v[m];
+    tile.to_memory(r, res);
     if (EPI && A.mul) {
       T mm[V];
-      load_run<T, V>(A.mul + base, mm);
+      tile.load(A.mul + base, mm);
 #pragma unroll
       for (int m = 0; m < V; ++m) res[m] *= mm[m];
     }
@@ -1233,11 +1306,11 @@ __global__ void __launch_bounds__(256) xwave_kernel(const LineArgs<T> A, int nli
     }
     if (EPI && acc) {
       T aa[V];
-      load_run<T, V>(acc + base, aa);
+      tile.load(acc + base, aa);
 #pragma unroll
       for (int m = 0; m < V; ++m) res[m] = A.ac * aa[m] + res[m];
     }
-    store_run<T, V>(t + base, res);
+    tile.store(t + base, res);
   }
 }
 

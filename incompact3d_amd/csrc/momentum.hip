@@ -203,44 +203,44 @@ __global__ void __launch_bounds__(256) mom_x_kernel(const MomArgs<T> A, int nlin
   const int wave = (blockIdx.x * blockDim.x + threadIdx.x) >> 6;
   const int nwaves = (gridDim.x * blockDim.x) >> 6;
   const int n = A.n;
-  const int e0 = lane * V;
   LineCoef<T, V> C;
   C.load(A, lane);
   // the next velocities (u_x of the next line last) are loaded before this
   // component is solved, so that their latency overlaps the solves (each wave
   // loops over several lines)
-  T ud[V], uc[V], nx[V], nd[V];
+  // memory order in 16 bytes of the widest type; FP32 keeps run order, 16 or 32
+  // bytes a lane (512^3: 2050 us against 2300)
+  constexpr int PER = sizeof(T) == 4 && !GEN ? V : (V == 1 ? 1 : 2);
+  using Tile = LineTile<T, V, PER>;
+  __shared__ __align__(16) T lines[4 * Tile::WORDS];
+  const Tile tile(lines);
+  T ud[V], uc[V], um[V], nx[V], nd[V];   // run order; um (u_c), nx, nd: memory order
   const int c0 = ALL ? 0 : (int)blockIdx.z, c1 = ALL ? 3 : c0 + 1;
   if (wave < nlines) {
-    load_run<T, V>(A.ud + (long long)wave * n + e0, nd);
-    if constexpr (!ALL) load_run<T, V>(A.uc[c0] + (long long)wave * n + e0, nx);
+    tile.load(A.ud + (long long)wave * n, nd);
+    if constexpr (!ALL) tile.load(A.uc[c0] + (long long)wave * n, nx);
   }
   for (int ln = wave; ln < nlines; ln += nwaves) {
-    const long long base = (long long)ln * n + e0;
-#pragma unroll
-    for (int m = 0; m < V; ++m) ud[m] = nd[m];
+    const long long base = (long long)ln * n;
+    tile.to_run(nd, ud);
 #pragma unroll 1
     for (int comp = c0; comp < c1; ++comp) {
       const T *const acc_in = A.acc[comp], *const f2_in = A.f2[comp], *const f3_in = A.f3[comp];
       const bool more = ln + nwaves < nlines;
       if constexpr (ALL) {
-        if (comp == 0) {
 #pragma unroll
-          for (int m = 0; m < V; ++m) uc[m] = ud[m];
-        } else {
-#pragma unroll
-          for (int m = 0; m < V; ++m) uc[m] = nx[m];
-        }
-        if (comp < 2) load_run<T, V>(A.uc[comp + 1] + base, nx);
-        else if (more) load_run<T, V>(A.ud + base + (long long)nwaves * n, nd);
+        for (int m = 0; m < V; ++m) um[m] = comp == 0 ? nd[m] : nx[m];
+        if (comp < 2) tile.load(A.uc[comp + 1] + base, nx);
+        else if (more) tile.load(A.ud + base + (long long)nwaves * n, nd);
       } else {
 #pragma unroll
-        for (int m = 0; m < V; ++m) uc[m] = nx[m];
+        for (int m = 0; m < V; ++m) um[m] = nx[m];
         if (more) {
-          load_run<T, V>(A.ud + base + (long long)nwaves * n, nd);
-          load_run<T, V>(A.uc[comp] + base + (long long)nwaves * n, nx);
+          tile.load(A.ud + base + (long long)nwaves * n, nd);
+          tile.load(A.uc[comp] + base + (long long)nwaves * n, nx);
         }
       }
+      tile.to_run(um, uc);
       // every epilogue input is read before the first store (the compiler
       // cannot move loads above stores to possibly aliasing arrays), and ahead
       // of the solves where there are registers for it
@@ -250,19 +250,21 @@ __global__ void __launch_bounds__(256) mom_x_kernel(const MomArgs<T> A, int nlin
       auto inputs = [&] {
         if constexpr (GEN) {
           const MomUpdate<T> &U = A.up;
-          load_run<T, V>(acc_in + base, acc);
-          if (U.nterms >= 2) load_run<T, V>(U.f2[comp] + base, f2);
-          if (U.nterms >= 3) load_run<T, V>(U.f3[comp] + base, f3);
-          if (U.rot[comp]) load_run<T, V>(U.rot[comp] + base, rot);
-          if constexpr (sizeof(T) == 4) load_run<double, V>(U.u64[comp] + base, un);
+          tile.load(acc_in + base, acc);
+          if (U.nterms >= 2) tile.load(U.f2[comp] + base, f2);
+          if (U.nterms >= 3) tile.load(U.f3[comp] + base, f3);
+          if (U.rot[comp]) tile.load(U.rot[comp] + base, rot);
+          if constexpr (sizeof(T) == 4) tile.load(U.u64[comp] + base, un);
         } else {
-          if (acc_in) load_run<T, V>(acc_in + base, acc);
-          if (A.nterms >= 2) load_run<T, V>(f2_in + base, f2);
-          if (A.nterms >= 3) load_run<T, V>(f3_in + base, f3);
+          if (acc_in) tile.load(acc_in + base, acc);
+          if (A.nterms >= 2) tile.load(f2_in + base, f2);
+          if (A.nterms >= 3) tile.load(f3_in + base, f3);
         }
       };
       if constexpr (EARLY) inputs();
-      mom_line<T, V>(A, C, ud, uc, r, lane);
+      T run[V];
+      mom_line<T, V>(A, C, ud, uc, run, lane);
+      tile.to_memory(run, r);
       if constexpr (!EARLY) inputs();
       if constexpr (GEN) {
         const MomUpdate<T> &U = A.up;
@@ -270,16 +272,16 @@ __global__ void __launch_bounds__(256) mom_x_kernel(const MomArgs<T> A, int nlin
 #pragma unroll
         for (int m = 0; m < V; ++m) {
           r[m] = mom_forced(U, comp, acc[m] + r[m], rot[m]);
-          const double uo = sizeof(T) == 8 ? (double)uc[m] : un[m];
-          un[m] = pre_correc_point(U, comp, e0 + m, j, k, mom_increment(U, r[m], f2[m], f3[m]) + uo);
+          const double uo = sizeof(T) == 8 ? (double)um[m] : un[m];
+          un[m] = pre_correc_point(U, comp, tile.point(m), j, k, mom_increment(U, r[m], f2[m], f3[m]) + uo);
         }
-        store_run<T, V>(A.out[comp] + base, r);
-        store_run<double, V>(U.u64[comp] + base, un);
+        tile.store(A.out[comp] + base, r);
+        tile.store(U.u64[comp] + base, un);
         if constexpr (sizeof(T) == 4) {
           float sh[V];
 #pragma unroll
           for (int m = 0; m < V; ++m) sh[m] = (float)un[m];
-          store_run<float, V>(U.u32[comp] + base, sh);
+          tile.store(U.u32[comp] + base, sh);
         }
         continue;
       }
@@ -287,7 +289,7 @@ __global__ void __launch_bounds__(256) mom_x_kernel(const MomArgs<T> A, int nlin
 #pragma unroll
         for (int m = 0; m < V; ++m) r[m] = acc[m] + r[m];
       }
-      store_run<T, V>(A.out[comp] + base, r);
+      tile.store(A.out[comp] + base, r);
       if (A.nterms) {
         // AB3 with FP64 accumulation: du = a f1 + b f2 + c f3, u_new = du + u_old
         double du[V];
@@ -301,17 +303,17 @@ __global__ void __launch_bounds__(256) mom_x_kernel(const MomArgs<T> A, int nlin
           // u_c is the FP64 velocity itself
           double un[V];
 #pragma unroll
-          for (int m = 0; m < V; ++m) un[m] = du[m] + (double)uc[m];
-          store_run<double, V>(A.u_new[comp] + base, un);
+          for (int m = 0; m < V; ++m) un[m] = du[m] + (double)um[m];
+          tile.store(A.u_new[comp] + base, un);
         } else {
           float d[V], sh[V];
 #pragma unroll
           for (int m = 0; m < V; ++m) {
             d[m] = (float)du[m];
-            sh[m] = (float)(du[m] + (double)uc[m]);
+            sh[m] = (float)(du[m] + (double)um[m]);
           }
-          store_run<float, V>(A.delta[comp] + base, d);
-          store_run<float, V>(A.shadow[comp] + base, sh);
+          tile.store(A.delta[comp] + base, d);
+          tile.store(A.shadow[comp] + base, sh);
         }
       }
     }

@@ -141,27 +141,28 @@ __global__ void __launch_bounds__(1024) proj_yz_kernel(const ProjArgs<T> A) {
 }
 
 // ---------------------------------------------------------------- x sweeps (one wavefront per line)
-// cor_vel (navier.f90:206-249) on one run of V points: u -= g in FP64, and
+// cor_vel (navier.f90:206-249) on a line in memory order: u -= g in FP64, and
 // for FP32-bulk compute first u += the step's AB3 increment, then the FP32
 // copy refreshed.  The FP64 velocity is read from and written to either a
 // plain FP64 array or its split form (hold/res in, u32/res out).
-template <int V, typename T>
-__device__ __forceinline__ void correct(const ProjArgs<T> &A, const int c, const long long base, const T (&g)[V]) {
+template <int V, typename T, int PER>
+__device__ __forceinline__ void correct(const ProjArgs<T> &A, const int c, const LineTile<T, V, PER> &tile,
+                                        const long long base, const T (&g)[V]) {
   double u[V];
   const bool split = sizeof(T) == 4 && A.res[c];
   if (split) {
     float h[V];
     int32_t r[V];
-    load_run<float, V>(A.hold[c] + base, h);
-    load_run<int32_t, V>(A.res[c] + base, r);
+    tile.load(A.hold[c] + base, h);
+    tile.load(A.res[c] + base, r);
 #pragma unroll
     for (int m = 0; m < V; ++m) u[m] = join_split(h[m], r[m]);
   } else {
-    load_run<double, V>(A.u64[c] + base, u);
+    tile.load(A.u64[c] + base, u);
   }
   if (sizeof(T) == 4 && A.du[c]) {
     float d[V];
-    load_run<float, V>(A.du[c] + base, d);
+    tile.load(A.du[c] + base, d);
 #pragma unroll
     for (int m = 0; m < V; ++m) u[m] = u[m] + (double)d[m];
   }
@@ -175,37 +176,37 @@ __device__ __forceinline__ void correct(const ProjArgs<T> &A, const int c, const
       f[m] = (float)u[m];
       r[m] = split_residual(u[m], f[m]);
     }
-    store_run<float, V>(A.u32[c] + base, f);
-    store_run<int32_t, V>(A.res[c] + base, r);
+    tile.store(A.u32[c] + base, f);
+    tile.store(A.res[c] + base, r);
     return;
   }
-  store_run<double, V>(A.u64[c] + base, u);
+  tile.store(A.u64[c] + base, u);
   if (sizeof(T) == 4 && A.u32[c]) {
     float f[V];
 #pragma unroll
     for (int m = 0; m < V; ++m) f[m] = (float)u[m];
-    store_run<float, V>(A.u32[c] + base, f);
+    tile.store(A.u32[c] + base, f);
   }
 }
 
 // The same in the general step (no split state, no increment), with the wall
-// planes stored; base is the first of V points of line (j, k).
-template <int V, typename T>
-__device__ __forceinline__ void correct_general(const CorVel &A, const int c, const long long base, const int i0,
-                                                const int j, const int k, const T (&g)[V]) {
+// planes stored; base is the first point of line (j, k).
+template <int V, typename T, int PER>
+__device__ __forceinline__ void correct_general(const CorVel &A, const int c, const LineTile<T, V, PER> &tile,
+                                                const long long base, const int j, const int k, const T (&g)[V]) {
 #pragma unroll
-  for (int m = 0; m < V; ++m) store_wall(A, c, i0 + m, j, k, g[m]);
+  for (int m = 0; m < V; ++m) store_wall(A, c, tile.point(m), j, k, g[m]);
   if (!A.apply) return;
   double u[V];
-  load_run<double, V>(A.u64[c] + base, u);
+  tile.load(A.u64[c] + base, u);
 #pragma unroll
   for (int m = 0; m < V; ++m) u[m] = u[m] - (double)g[m];
-  store_run<double, V>(A.u64[c] + base, u);
+  tile.store(A.u64[c] + base, u);
   if constexpr (sizeof(T) == 4) {
     float f[V];
 #pragma unroll
     for (int m = 0; m < V; ++m) f[m] = (float)u[m];
-    store_run<float, V>(A.u32[c] + base, f);
+    tile.store(A.u32[c] + base, f);
   }
 }
 
@@ -233,21 +234,29 @@ __global__ void __launch_bounds__(256, (projx_wpe<T, V, SW>())) proj_x_kernel(co
   }
   // the next line's inputs are loaded before this line is solved, so that
   // their latency overlaps the solves (each wave loops over several lines)
-  T pre[R::NIN][V];
+  // memory order in 16 bytes of the widest type; FP32 keeps run order, 16 or 32
+  // bytes a lane (512^3: 650 and 1930 us against 813 and 2250), where it does
+  // not meet the FP64 velocity
+  constexpr int PER = sizeof(T) == 4 || V == 1 ? V : 2;
+  constexpr int PERO = GEN && sizeof(T) == 4 && V > 2 ? 2 : PER;
+  using TileIn = LineTile<T, V, PER>;
+  using TileOut = LineTile<T, V, PERO>;
+  __shared__ __align__(16) T lines[4 * (TileIn::WORDS > TileOut::WORDS ? TileIn::WORDS : TileOut::WORDS)];
+  const TileIn tin(lines);
+  const TileOut tout(lines);
+  T pre[R::NIN][V];             // memory order
   if (wave < nlines) {
 #pragma unroll
-    for (int i = 0; i < R::NIN; ++i) load_run<T, V>(A.in[i] + (long long)wave * n + e0, pre[i]);
+    for (int i = 0; i < R::NIN; ++i) tin.load(A.in[i] + (long long)wave * n, pre[i]);
   }
   for (int ln = wave; ln < nlines; ln += nwaves) {
-    const long long base = (long long)ln * n + e0;
+    const long long base = (long long)ln * n;
     T cur[R::NIN][V];
 #pragma unroll
-    for (int i = 0; i < R::NIN; ++i)
-#pragma unroll
-      for (int m = 0; m < V; ++m) cur[i][m] = pre[i][m];
+    for (int i = 0; i < R::NIN; ++i) tin.to_run(pre[i], cur[i]);
     if (ln + nwaves < nlines) {
 #pragma unroll
-      for (int i = 0; i < R::NIN; ++i) load_run<T, V>(A.in[i] + (long long)(ln + nwaves) * n + e0, pre[i]);
+      for (int i = 0; i < R::NIN; ++i) tin.load(A.in[i] + (long long)(ln + nwaves) * n, pre[i]);
     }
     T wI[2][V], wD[V];
 #pragma unroll
@@ -271,19 +280,20 @@ __global__ void __launch_bounds__(256, (projx_wpe<T, V, SW>())) proj_x_kernel(co
     wave_solve<T, V>(wI[0], fsI, fwI, ffwI, smI, A.alfaI, A.rdenI, lane);
     wave_solve<T, V>(wI[1], fsI, fwI, ffwI, smI, A.alfaI, A.rdenI, lane);
     wave_solve<T, V>(wD, fsD, fwD, ffwD, smD, A.alfaD, A.rdenD, lane);
+    T r[3][V];
+    tout.to_memory(wD, r[0]);
+    tout.to_memory(wI[0], r[1]);
+    tout.to_memory(wI[1], r[2]);
     if constexpr (SW == SW_DIV_X) {
-      store_run<T, V>(A.out[0] + base, wD);
-      store_run<T, V>(A.out[1] + base, wI[0]);
-      store_run<T, V>(A.out[2] + base, wI[1]);
+#pragma unroll
+      for (int i = 0; i < 3; ++i) tout.store(A.out[i] + base, r[i]);
     } else if constexpr (GEN) {
       const int lu = __builtin_amdgcn_readfirstlane(ln), k = lu / A.cv.ny, j = lu - k * A.cv.ny;
-      correct_general<V>(A.cv, 0, base, e0, j, k, wD);
-      correct_general<V>(A.cv, 1, base, e0, j, k, wI[0]);
-      correct_general<V>(A.cv, 2, base, e0, j, k, wI[1]);
+#pragma unroll
+      for (int i = 0; i < 3; ++i) correct_general<V>(A.cv, i, tout, base, j, k, r[i]);
     } else {   // SW_GRAD_X: u_c -= grad_c p with the FP64 velocity (cor_vel)
-      correct<V>(A, 0, base, wD);
-      correct<V>(A, 1, base, wI[0]);
-      correct<V>(A, 2, base, wI[1]);
+#pragma unroll
+      for (int i = 0; i < 3; ++i) correct<V>(A, i, tout, base, r[i]);
     }
   }
 }
