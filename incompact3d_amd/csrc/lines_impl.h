@@ -49,7 +49,8 @@ struct LineArgs {
   long long sa_out, sb_out, se_out;   // output strides
   int row;                            // LDS row stride (x mode)
   // blockIdx.z > 0: further operands of a batch (seg_line_kernel and
-  // xwave_kernel; same operator, same coefficients)
+  // xwave_kernel; same operator, same coefficients).  BATCH kernels choose
+  // among them, a load behind a load that single calls do without.
   const T *ub[2], *accb[2];
   T *tb[2];
 };
@@ -865,7 +866,7 @@ __global__ void __launch_bounds__(LB) line_kernel(const LineArgs<T> A) {
 // a window, the solve of seg_solve with the set's truncated carry chain, and
 // the epilogue's inputs read before the first store (acc may be t).  Byte
 // offsets are 32-bit (the host checks the field size).
-template <typename T, int OP, int L, bool EPI>
+template <typename T, int OP, int L, bool EPI, bool BATCH = false>
 __global__ void __launch_bounds__(1024) seg_line_kernel(const LineArgs<T> A, const T rden, const int kdepth) {
   extern __shared__ __align__(16) unsigned char smem_raw[];
   T *smem = reinterpret_cast<T *>(smem_raw);
@@ -873,7 +874,7 @@ __global__ void __launch_bounds__(1024) seg_line_kernel(const LineArgs<T> A, con
   const int line = threadIdx.x, seg = threadIdx.y;
   const int tid = seg * TL + line, nthr = TL * P;
   const int n = A.n_out;
-  const int item = (int)blockIdx.z;
+  const int item = BATCH ? (int)blockIdx.z : 0;
   const T *const u = item == 0 ? A.u : A.ub[item - 1];
   const T *const acc = item == 0 ? A.acc : A.accb[item - 1];
   T *const t = item == 0 ? A.t : A.tb[item - 1];
@@ -941,6 +942,15 @@ static int launch_seg_line(const LineArgs<T> &a, T rden, const YzShape<T> &Y, bo
   const dim3 grid((a.na + Y.TL - 1) / Y.TL, a.nb, batch), block(Y.TL, Y.P);
   const size_t shmem = Y.shmem;
   constexpr int L = YzShape<T>::L;
+  if constexpr (OP == OP_DER1) {   // the only operator that comes in batches
+    if (batch > 1) {
+      if (epi) hipLaunchKernelGGL((seg_line_kernel<T, OP, L, true, true>), grid, block, shmem, st, a, rden, kdepth);
+      else hipLaunchKernelGGL((seg_line_kernel<T, OP, L, false, true>), grid, block, shmem, st, a, rden, kdepth);
+      hipError_t e = hipGetLastError();
+      if (e != hipSuccess) return fail(X3D_ERR_HIP, std::string("segmented line launch: ") + hipGetErrorString(e));
+      return X3D_OK;
+    }
+  }
   if (epi) hipLaunchKernelGGL((seg_line_kernel<T, OP, L, true>), grid, block, shmem, st, a, rden, kdepth);
   else hipLaunchKernelGGL((seg_line_kernel<T, OP, L, false>), grid, block, shmem, st, a, rden, kdepth);
   hipError_t e = hipGetLastError();
@@ -1215,7 +1225,7 @@ struct LineTile {
   }
 };
 
-template <typename T, int OP, int V, bool EPI>
+template <typename T, int OP, int V, bool EPI, bool BATCH = false>
 __global__ void __launch_bounds__(256) xwave_kernel(const LineArgs<T> A, int nlines) {
   constexpr int HL = Halo<OP>::L, HR = Halo<OP>::R, W = V + HL + HR;
   const int lane = threadIdx.x & 63;
@@ -1223,7 +1233,7 @@ __global__ void __launch_bounds__(256) xwave_kernel(const LineArgs<T> A, int nli
   const int nwaves = (gridDim.x * blockDim.x) >> 6;
   const int n = A.n_out;   // == n_in == 64*V
   const int e0 = lane * V;
-  const int item = (int)blockIdx.z;
+  const int item = BATCH ? (int)blockIdx.z : 0;
   const T *const u = item == 0 ? A.u : A.ub[item - 1];
   const T *const acc = item == 0 ? A.acc : A.accb[item - 1];
   T *const t = item == 0 ? A.t : A.tb[item - 1];
@@ -1316,6 +1326,13 @@ __global__ void __launch_bounds__(256) xwave_kernel(const LineArgs<T> A, int nli
 
 template <typename T, int OP, int V>
 static void launch_xv(const LineArgs<T> &a, bool epi, int nlines, dim3 grid, dim3 block, hipStream_t st) {
+  if constexpr (OP == OP_DER1) {
+    if (grid.z > 1) {
+      if (epi) hipLaunchKernelGGL((xwave_kernel<T, OP, V, true, true>), grid, block, 0, st, a, nlines);
+      else hipLaunchKernelGGL((xwave_kernel<T, OP, V, false, true>), grid, block, 0, st, a, nlines);
+      return;
+    }
+  }
   if (epi) hipLaunchKernelGGL((xwave_kernel<T, OP, V, true>), grid, block, 0, st, a, nlines);
   else hipLaunchKernelGGL((xwave_kernel<T, OP, V, false>), grid, block, 0, st, a, nlines);
 }
