@@ -97,7 +97,7 @@ def roofline_momentum_yz(X, p, stream, reps=10):
     HIP events on that stream.  Algorithmic bytes per launch: the fields each
     launch must move once (u_d if it differs from u_c, u_c, the accumulator
     when present, the output), N*8 bytes each, averaged over the six launch
-    configurations (19 fields per step / 6)."""
+    configurations (19 fields per step / 6; three components to a launch)."""
     import torch
     s = X.Solver(p, 0)
     s.init_tgv()
@@ -254,7 +254,7 @@ def channel_step_bench(X, stream, warmup=20, steps=200):
     from incompact3d_amd import channel
     p = channel.params()
     npts = p.nx * p.ny * p.nz
-    out = {"workload": "channel Re_tau 180, 256x129x128, istret 2, RK3 dt 0.005, per-operator step"}
+    out = {"workload": "channel Re_tau 180, 256x129x128, istret 2, RK3 dt 0.005"}
     X.init(p)
     X.set_stream(stream.cuda_stream)
     try:

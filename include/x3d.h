@@ -315,11 +315,13 @@ int x3d_host_transpose_y_to_x_f32(const float *src, float *dst, const int *n1, c
  * precision: 0 = FP64 everywhere; 1 = FP32 bulk (FP32 derivatives, FFTs,
  * convective products) with FP64 velocity accumulation, FP64 Poisson divide
  * and FP64 diagnostics reductions.
- * For nx in {64,128,256,512} and ny, nz multiples of 16 up to 512 the
- * momentum right-hand side and AB3 run as nine fused sweeps and the
- * divergence / gradient + cor_vel as six; other grids (or the environment
- * variable X3D_UNFUSED_MOMENTUM set at create time) use one launch per
- * derivative.  Both paths compute the same quantities.
+ * Where every direction is periodic with nx in {64,128,256,512} or ny, nz
+ * multiples of 16 up to 512, or bounded with lines that the bounded sweeps
+ * cover (two segments of 8 FP64 / 16 FP32 points up to what fits in LDS), the
+ * momentum right-hand side with the velocity update runs as three fused
+ * sweeps and the divergence / gradient + cor_vel as six; other grids (or the
+ * environment variable X3D_UNFUSED_MOMENTUM set at create time) use one launch
+ * per derivative.  Both paths compute the same quantities.
  * Boundaries: periodic or free-slip (ncl=1 at both ends) per direction, and
  * in y also no-slip walls (ncl=2, either or both faces), with the Poisson
  * solver of the grid (poisson_000, poisson_010 with its stretched branch,
@@ -330,8 +332,7 @@ int x3d_host_transpose_y_to_x_f32(const float *src, float *dst, const int *n1, c
  * ppyi and forms the y viscous term as pp2y deryy - pp4y dery
  * (transeq.f90:337-370).
  * Time schemes: AB3 (itimescheme=3) and the low-storage RK3 (itimescheme=5,
- * time_integrators.f90:151-157, three projected sub-steps per step); the
- * fused sweeps run AB3 on periodic boxes. */
+ * time_integrators.f90:151-157, three projected sub-steps per step). */
 typedef struct x3d_solver x3d_solver;
 int x3d_solver_create(int precision, x3d_solver **out);
 int x3d_solver_destroy(x3d_solver *s);
@@ -377,7 +378,7 @@ int x3d_solver_set_forcing(x3d_solver *s, int mode, double value);
  * namelist): while the step index (1 at the first step, as itime with
  * ifirst = 1) is below spinup_time, every (sub-)step adds -wrotation * uy
  * to the x and +wrotation * ux to the y right-hand side.  spinup_time 0
- * turns it off.  Per-operator step only (bounded y, or RK3). */
+ * turns it off.  For bounded y or RK3. */
 int x3d_solver_set_rotation(x3d_solver *s, double wrotation, int spinup_time);
 /* Bulk velocity ub = dy / (yly nx nz) sum ux / ppy of channel_cfr
  * (Case-Channel.f90:234-246), FP64. */

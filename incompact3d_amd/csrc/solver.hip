@@ -8,16 +8,14 @@
 //   solve_poisson          navier.f90:27-141    (divergence, poisson, gradp)
 //   cor_vel                navier.f90:206-249
 // as in the time loop of xcompact3d.f90:29-102.  On grids the fused sweeps
-// cover, each direction of the momentum right-hand side is one launch per
-// velocity component (AB3 fused into the x sweep) and each direction of the
-// divergence and of the gradient + cor_vel is one launch; elsewhere every
-// derivative and staggered operator is one line-solve launch whose epilogue
-// does the reference's array arithmetic.  precision 0 computes in FP64;
+// cover, periodic or bounded, each direction of the momentum right-hand side
+// (forcing, AB3 or RK3 and pre_correc in the x sweep), of the divergence and of
+// the gradient + cor_vel is one launch; elsewhere every derivative and
+// staggered operator is one line-solve launch whose epilogue does the
+// reference's array arithmetic.  precision 0 computes in FP64;
 // precision 1 keeps an FP32 copy of the velocity for every derivative, FFT
 // and product, while the velocity itself is accumulated in FP64 (AB3 and
-// cor_vel) and the Poisson divide and reductions run in FP64.  RK3
-// (itimescheme=5), free-slip faces, y walls and stretched y meshes run on
-// the per-operator path.
+// cor_vel) and the Poisson divide and reductions run in FP64.
 #include <sys/stat.h>
 
 #include <cerrno>
@@ -1089,7 +1087,7 @@ int x3d_solver_set_rotation(x3d_solver *S, double wrotation, int spinup_time) {
   if (!S) return fail(X3D_ERR_ARG, "null solver");
   if (!std::isfinite(wrotation) || spinup_time < 0) return fail(X3D_ERR_ARG, "bad rotation arguments");
   if (S->plain && spinup_time > 0)
-    return fail(X3D_ERR_UNSUPPORTED, "the spin-up rotation runs on the per-operator step (bounded y, or RK3)");
+    return fail(X3D_ERR_UNSUPPORTED, "the spin-up rotation needs bounded y or RK3");
   S->wrotation = wrotation;
   S->spinup_time = spinup_time;
   return X3D_OK;
