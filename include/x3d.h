@@ -359,6 +359,9 @@ int x3d_solver_divergence_stats(x3d_solver *s, double out2[2]);
  * X3D_ERR_STATE before the first step. */
 int x3d_solver_divu_stats(x3d_solver *s, double out2[2]);
 int x3d_solver_itime(x3d_solver *s, int *itime);
+/* Which path the solver's steps take, decided when it was created: 1 the fused
+ * sweeps, 0 one launch per derivative. */
+int x3d_solver_fused(x3d_solver *s, int *fused);
 /* Channel initial condition of init_channel (Case-Channel.f90:96-128, iin=1,
  * idir_stream=1): u = init_noise um (2r-1) + 1 - y^2, v, w = init_noise um
  * (2r-1), um = exp(-0.2 y^2), y the wall-normal coordinate (yp on a

@@ -282,6 +282,13 @@ class Solver:
         check(_lib.lib().x3d_solver_itime(self._h, C.byref(v)), "itime")
         return v.value
 
+    @property
+    def fused(self):
+        """Whether the steps run as fused sweeps (else one launch per derivative)."""
+        v = C.c_int(0)
+        check(_lib.lib().x3d_solver_fused(self._h, C.byref(v)), "fused")
+        return bool(v.value)
+
     def set_les(self, model: int, cs: float = 0.15, iconserv: int = 0, beta: float = 0.0, mlp=None,
                 gscale: float = 1.0, delta0: float = 1.0):
         """x3d_solver_set_les: 0 none, 1 Smagorinsky (jles=1, smagcst=cs,

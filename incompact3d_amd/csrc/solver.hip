@@ -1119,6 +1119,12 @@ int x3d_solver_itime(x3d_solver *S, int *itime) {
   return X3D_OK;
 }
 
+int x3d_solver_fused(x3d_solver *S, int *fused) {
+  if (!S || !fused) return fail(X3D_ERR_ARG, "null pointer");
+  *fused = S->fused ? 1 : 0;
+  return X3D_OK;
+}
+
 // ---------------------------------------------------------------- checkpoint / restart
 // restart() of tools.f90:205-514 for this solver's state: the checkpoint
 // directory <rundir>/checkpoint holds one file per variable the reference
