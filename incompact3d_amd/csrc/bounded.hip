@@ -259,19 +259,11 @@ __global__ void __launch_bounds__(MAXT) bmom_yz_kernel(const BMomArgs<T> A) {
     for (int m = 0; m < L; ++m) dd[m] = wd[m + 2];
     bmom_rhs<T, L>(A, wc, wd, w, along, seg, rows);
   }
-  // (a block has at least n threads)
-  T mt[3];
-  if (A.m1 && tid < n) {
-    mt[0] = A.m1[tid];
-    mt[1] = A.m2[tid];
-    mt[2] = A.m4[tid];
-  }
+  const T *const msrc[3] = {A.m1, A.m2, A.m4};
+  BoundCopy<T, 3, 1> mc;
+  if (A.m1) mc.load(msrc, tid, nthr, n);
   tc.store(cs, src, tid, nthr, CW);
-  if (A.m1 && tid < n) {
-    met[tid] = mt[0];
-    met[n + tid] = mt[1];
-    met[2 * n + tid] = mt[2];
-  }
+  if (A.m1) mc.store(met, msrc, tid, nthr, n);
   __syncthreads();
   bound_solve<T, L, 3, NT>(w, cs, cf, cb, gf, gb, line, seg, TL, P, A.K);
   if (!active) return;

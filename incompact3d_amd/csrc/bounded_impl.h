@@ -262,20 +262,22 @@ __device__ __forceinline__ void bound_solve(T (&v)[N][L], const T *cs, T *cf, T 
   }
 }
 
-// Copy of NT device tables into LDS split around the caller's window loads, as
-// TableCopy does for two.
-template <typename T, int NT>
+// Copy of NT device tables of cnt words into LDS split around the caller's
+// window loads, as TableCopy does for two: R words a thread through registers,
+// what is left of larger tables (a block may have fewer threads than words)
+// straight in store().
+template <typename T, int NT, int R = 2>
 struct BoundCopy {
-  static constexpr int R = 2;
   T v[NT][R];
-  __device__ __forceinline__ void load(const T *const (&src)[NT], int tid, int nthr, int cnt) {
+  __host__ __device__ __forceinline__ void load(const T *const (&src)[NT], int tid, int nthr, int cnt) {
 #pragma unroll
     for (int t = 0; t < NT; ++t)
 #pragma unroll
       for (int r = 0; r < R; ++r)
         if (tid + r * nthr < cnt) v[t][r] = src[t][tid + r * nthr];
   }
-  __device__ __forceinline__ void store(T *cs, const T *const (&src)[NT], int tid, int nthr, int cnt) const {
+  __host__ __device__ __forceinline__ void store(T *cs, const T *const (&src)[NT], int tid, int nthr,
+                                                 int cnt) const {
 #pragma unroll
     for (int t = 0; t < NT; ++t) {
 #pragma unroll
