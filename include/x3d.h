@@ -316,12 +316,15 @@ int x3d_host_transpose_y_to_x_f32(const float *src, float *dst, const int *n1, c
  * convective products) with FP64 velocity accumulation, FP64 Poisson divide
  * and FP64 diagnostics reductions.
  * Where every direction is periodic with nx in {64,128,256,512} or ny, nz
- * multiples of 16 up to 512, or bounded with lines that the bounded sweeps
- * cover (two segments of 8 FP64 / 16 FP32 points up to what fits in LDS), the
- * momentum right-hand side with the velocity update runs as three fused
- * sweeps and the divergence / gradient + cor_vel as six; other grids (or the
- * environment variable X3D_UNFUSED_MOMENTUM set at create time) use one launch
- * per derivative.  Both paths compute the same quantities.
+ * multiples of 16 up to 512, or bounded with lines that the bounded sweeps of
+ * the solver's precision cover, the momentum right-hand side with the velocity
+ * update runs as three fused sweeps and the divergence / gradient + cor_vel as
+ * six; other grids (or the environment variable X3D_UNFUSED_MOMENTUM set at
+ * create time) use one launch per derivative.  Both paths compute the same
+ * quantities; x3d_solver_fused tells which one a solver takes.  Bounded lines
+ * are covered from two segments (16 rows in FP64, 32 in FP32) up to what 64 KB
+ * of LDS hold, of the sizes the pressure solve has: in FP64 17 to 129 points in
+ * x, to 257 in y and z, to 513 between uniform no-slip walls; in FP32 33 to 513.
  * Boundaries: periodic or free-slip (ncl=1 at both ends) per direction, and
  * in y also no-slip walls (ncl=2, either or both faces), with the Poisson
  * solver of the grid (poisson_000, poisson_010 with its stretched branch,

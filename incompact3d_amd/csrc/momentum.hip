@@ -325,20 +325,27 @@ __global__ void __launch_bounds__(256) mom_x_kernel(const MomArgs<T> A, int nlin
 
 // ---------------------------------------------------------------- host side
 
-// The fused sweeps cover bounded lines that have tables (bounded.hip) and
-// periodic lines with nx = 64, 128, 256 or 512 (one
-// wavefront per x line, 1..8 points per lane) and ny, nz that YzShape can
-// plan (a multiple of 16 whose block fits; 16..512 for both precisions).  The product derivative
-// uses the set of parity d==c (transeq.f90:125) and the velocity derivative
-// the opposite one; one set serves both, so they must hold the same
-// coefficients, which is the case for periodic lines (schemes.f90:583-596
-// builds ffp from ff and prepares both from the same diagonals when
-// ncl1 = ncln = 0).
+// The fused sweeps of precision T cover bounded lines that have a plan in that
+// precision (bounded.hip; up to 1024 points, where the operators that the
+// solver's other calls use end) and periodic lines with nx = 64, 128, 256 or
+// 512 (one wavefront per x line, 1..8 points per lane) and ny, nz that YzShape
+// can plan (a multiple of 16 whose block fits; 16..512 for both precisions).
+// An FP32 solver does not ask for the FP64 plan, whose tables are twice the
+// size in LDS: on free-slip lines of 257 points in x or 513 in y or z and on
+// stretched walls of 513 points only FP32 fits (RK3 step, per operator and
+// fused: 257^3 10727 and 7598, 256x513x128 stretched 8967 and 4759 us), on 17
+// points only FP64 has its two segments (17^3 901 and 249 us).
+// The product derivative uses the set of parity d==c (transeq.f90:125) and the
+// velocity derivative the opposite one; one set serves both on periodic lines,
+// so they must hold the same coefficients, which is the case there
+// (schemes.f90:583-596 builds ffp from ff and prepares both from the same
+// diagonals when ncl1 = ncln = 0).
+template <typename T>
 bool momentum_fusable(const Context &c) {
   for (int d = 0; d < 3; ++d) {
     const DirCoef &D = c.dir[d];
     if (D.bc1 != 0 && D.bcn != 0) {
-      if (!bounded_momentum_ok<double>(c, d) || !bounded_momentum_ok<float>(c, d)) return false;
+      if (D.n > 1024 || !bounded_momentum_ok<T>(c, d)) return false;
       continue;
     }
     if (D.bc1 != 0 || D.bcn != 0) return false;
@@ -353,6 +360,8 @@ bool momentum_fusable(const Context &c) {
   }
   return true;
 }
+template bool momentum_fusable<double>(const Context &);
+template bool momentum_fusable<float>(const Context &);
 
 template <typename T, bool GEN, bool ALL>
 static void launch_mom_x(const MomArgs<T> &A, int V, int nlines, dim3 grid, dim3 block, hipStream_t st) {

@@ -301,12 +301,13 @@ __global__ void __launch_bounds__(256, (projx_wpe<T, V, SW>())) proj_x_kernel(co
 // ---------------------------------------------------------------- host side
 // The fused projection covers the grids of the fused momentum sweeps: periodic
 // lines with nx = 64..512 (x wavefronts) and ny, nz planned by YzShape, and
-// bounded lines that have tables (bounded.hip).
+// bounded lines that have a plan in precision T (bounded.hip).
+template <typename T>
 bool projection_fusable(const Context &c) {
   for (int d = 0; d < 3; ++d) {
     const DirCoef &D = c.dir[d];
     if (D.bc1 != 0 && D.bcn != 0) {
-      if (!bounded_projection_ok<double>(c, d) || !bounded_projection_ok<float>(c, d)) return false;
+      if (!bounded_projection_ok<T>(c, d)) return false;
       continue;
     }
     if (D.bc1 != 0 || D.bcn != 0 || D.nm != D.n) return false;
@@ -319,6 +320,8 @@ bool projection_fusable(const Context &c) {
   }
   return true;
 }
+template bool projection_fusable<double>(const Context &);
+template bool projection_fusable<float>(const Context &);
 
 template <typename T, int SW>
 static void launch_yz(const ProjArgs<T> &A, const YzShape<T> &Y, hipStream_t st) {

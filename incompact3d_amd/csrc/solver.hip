@@ -875,7 +875,9 @@ int x3d_solver_create(int precision, x3d_solver **out) {
   S->n = (size_t)S->nx * S->ny * S->nz;
   S->wall1 = c->dir[1].bc1 == 2;
   S->walln = c->dir[1].bcn == 2;
-  S->fused = momentum_fusable(*c) && projection_fusable(*c) && getenv("X3D_UNFUSED_MOMENTUM") == nullptr;
+  S->fused = (precision == 0 ? momentum_fusable<double>(*c) && projection_fusable<double>(*c)
+                             : momentum_fusable<float>(*c) && projection_fusable<float>(*c)) &&
+             getenv("X3D_UNFUSED_MOMENTUM") == nullptr;
   S->plain = S->fused && c->p.itimescheme == 3 && c->dir[0].bc1 == 0 && c->dir[1].bc1 == 0 && c->dir[2].bc1 == 0;
   S->split = S->plain && precision == 1;
   int r = alloc_solver(*c, S);

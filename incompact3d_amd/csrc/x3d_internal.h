@@ -266,6 +266,7 @@ struct MomIO {
   const double *wallg = nullptr;
   double gdt = 0;
 };
+template <typename T>
 bool momentum_fusable(const Context &c);
 template <typename T>
 int launch_momentum(const Context &c, int dir, const MomIO<T> &io, int nx, int ny, int nz, hipStream_t st);
@@ -297,6 +298,7 @@ struct ProjIO {
   double *wallg = nullptr;
   double gdt = 0;
 };
+template <typename T>
 bool projection_fusable(const Context &c);
 template <typename T>
 int launch_projection(const Context &c, int sw, const ProjIO<T> &io, hipStream_t st);
