@@ -199,6 +199,14 @@ struct BMomArgs {
 // (L = 8, NT = 3, x) of them: 65^3 FP64 16.6 -> 14.4 us a y or z sweep, the
 // channel's y sweep 96 -> 84.  (Blocks of x lines are smaller: their LDS.)
 constexpr int BMOM_FEW = 512;
+// Larger blocks of y and z lines.  A solver's bounded lines have 2^k + 1 points
+// (the pressure solve's sizes), and only 513 of them need such blocks: in FP64
+// 65 x 8 threads with segments of 8 rows and two tables (three do not fit in
+// LDS), in FP32 31 x 32 with segments of 17.  Others are not compiled.
+template <typename T>
+constexpr bool bmom_many(bool longer, int nt) {
+  return sizeof(T) == 8 ? !longer && nt == 2 : longer;
+}
 
 // -1/2 D1(u_d u_c) - 1/2 u_d D1(u_c) + nu D2(u_c) of the rows of a segment:
 // the right-hand sides from the windows.
@@ -414,7 +422,7 @@ static bool bmom_plan(const Context &c, int dir, BoundPick<T> *Y, int *nt) {
   const bool stretched = dir == 1 && c.p.istret != 0;
   return Y->plan(n, *nt, 3, [&](int TL) {
     return dir == 0 ? 2 * (size_t)TL * row : (stretched ? 3 * (size_t)n : (size_t)0);
-  }) && (dir != 0 || Y->TL * Y->P <= BMOM_FEW);
+  }) && (Y->TL * Y->P <= BMOM_FEW || (dir != 0 && bmom_many<T>(Y->longer, *nt)));
 }
 
 template <typename T>
@@ -432,13 +440,21 @@ static void launch_bmom_x(const BMomArgs<T> &A, int nt, dim3 grid, dim3 block, s
   else hipLaunchKernelGGL((bmom_x_kernel<T, L, 3>), grid, block, sh, st, A);
 }
 
+template <typename T, int L, int NT>
+static void launch_bmom_nt(const BMomArgs<T> &A, dim3 grid, dim3 block, size_t sh, hipStream_t st) {
+  if constexpr (bmom_many<T>(L != BoundShape<T>::L, NT)) {
+    if (block.x * block.y > BMOM_FEW) {
+      hipLaunchKernelGGL((bmom_yz_kernel<T, L, NT, 1024>), grid, block, sh, st, A);
+      return;
+    }
+  }
+  hipLaunchKernelGGL((bmom_yz_kernel<T, L, NT, BMOM_FEW>), grid, block, sh, st, A);
+}
+
 template <typename T, int L>
 static void launch_bmom_yz(const BMomArgs<T> &A, int nt, dim3 grid, dim3 block, size_t sh, hipStream_t st) {
-  const bool few = block.x * block.y <= BMOM_FEW;
-  if (nt == 2 && few) hipLaunchKernelGGL((bmom_yz_kernel<T, L, 2, BMOM_FEW>), grid, block, sh, st, A);
-  else if (nt == 2) hipLaunchKernelGGL((bmom_yz_kernel<T, L, 2, 1024>), grid, block, sh, st, A);
-  else if (few) hipLaunchKernelGGL((bmom_yz_kernel<T, L, 3, BMOM_FEW>), grid, block, sh, st, A);
-  else hipLaunchKernelGGL((bmom_yz_kernel<T, L, 3, 1024>), grid, block, sh, st, A);
+  if (nt == 2) launch_bmom_nt<T, L, 2>(A, grid, block, sh, st);
+  else launch_bmom_nt<T, L, 3>(A, grid, block, sh, st);
 }
 
 template <typename T>

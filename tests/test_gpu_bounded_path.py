@@ -30,6 +30,8 @@ BLOCKS = {
     "wall-s1-513": (dict(nx=64, ny=513, nz=16, itimescheme=5, istret=1, **{**WALL, "dt": 5e-4}), (False, True)),
     "free-y1-wall-yn-513": (dict(nx=64, ny=513, nz=16, itimescheme=5, **{**WALL, "dt": 5e-4, "ncly1": 1}),
                             (False, True)),
+    "free-y-257": (dict(nx=64, ny=257, nz=16, ncly1=1, nclyn=1, yly=math.pi, itimescheme=5), (True, True)),
+    "wall-s2-257": (dict(nx=64, ny=257, nz=16, itimescheme=5, istret=2, **{**WALL, "dt": 5e-4}), (True, True)),
     "free-x-257": (dict(nx=257, ny=32, nz=16, nclx1=1, nclxn=1, xlx=math.pi, itimescheme=5), (False, True)),
     "free-x-513": (dict(nx=513, ny=16, nz=32, nclx1=1, nclxn=1, xlx=math.pi, itimescheme=3), (False, True)),
     "free-z-513": (dict(nx=33, ny=33, nz=513, itimescheme=5, **FREE), (False, True)),
