@@ -107,6 +107,7 @@ struct DirCoef {
 template <typename T>
 struct AnchorTab {
   T *pk = nullptr;
+  size_t off = 0;               // where it begins in Context::btab_mem
   int P = 0, K = 0;
 };
 struct BoundTab {
@@ -123,6 +124,7 @@ struct Context {
   DirCoef dir[3];
   std::vector<TriSet> sets;
   BoundTab btab[3][6][2];       // [direction][LineOpKind][parity]
+  void *btab_mem = nullptr;     // the allocation that holds their tables
   hipStream_t stream = nullptr;
   int device = 0;
   // stretched y mesh (istret != 0): the metrics of stretching.f90 on the
