@@ -21,7 +21,7 @@
 //   3 c2c forward along z, divide by -K (FP64), c2c inverse along z
 //   4 c2c inverse along y            (DCT-III for a non-periodic y)
 //   5 c2r along x
-// Line FFTs run in registers: each thread holds E = 16 points of a line in
+// Line FFTs run in registers: each thread holds E = 16 (8: LineShape) points of a line in
 // cyclic order (point t + m*NT for thread t of NT), does radix-16 (then
 // radix-2/4/8) Stockham butterflies on them and exchanges through LDS only
 // between stages -- one exchange for lines of up to 256 points.  The
@@ -546,7 +546,7 @@ __global__ void __launch_bounds__((SShape<T, N>::threads()))
     lk[2] = tb.kx2[a];
     lk[3] = tb.tx[a];
   }
-  // the z pass reads tz and kz2 at its 16 points per thread: staged in LDS
+  // the z pass reads tz and kz2 at each of a thread's points: staged in LDS
   // with the twiddles instead of read from global memory after the FFT
   constexpr bool ZT = MODE == FFT_Z_SOLVE && !COS && SShape<T, N>::ZTAB;
   double *ztab = reinterpret_cast<double *>(dct + N);

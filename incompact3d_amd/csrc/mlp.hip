@@ -419,7 +419,7 @@ __global__ void __launch_bounds__(WG_WAVES * 64) mlp_wgrad_kernel(const bf16x4 *
 // ADAM_P parameters with ADAM_G threads each, every thread a strided set of
 // the partials and four sums in flight, so the reduction is spread over the
 // chip (one thread a parameter walked 256 partials one after the other: 60 us
-// of a training step on 8192 points; now 6 us with the packing and the loss,
+// of a training step on 8192 points; now 4 us with the packing and the loss,
 // which were kernels of 6 us each).
 constexpr int ADAM_P = 32, ADAM_G = 8;
 
@@ -523,9 +523,9 @@ struct ClosureArgs {
 //
 // Bound by the issue of vector instructions: a tile of 16 points takes about
 // 880, of them 48 GELUs a lane with an exp2 and a reciprocal each at a quarter
-// rate, 17 of the 30 us at 64^3 FP32; its MFMAs run beside them.  Weights in
-// LDS: held in registers (80 of them) they left one wave a SIMD and moved
-// through accumulation registers, 33.2 us.
+// rate, 17 of the 30 us at 64^3 FP32; its MFMAs run beside them.  The weights
+// stay in LDS, four waves a SIMD in FP32: held in registers (80, half of them
+// moved out of accumulation registers for every tile) they left two, 33.2 us.
 template <typename T>
 __global__ void __launch_bounds__(256) closure_kernel(const bf16x4 *__restrict__ tiles, const float *__restrict__ bias,
                                                      const ClosureArgs<T> A, int *__restrict__ nfallback) {
@@ -538,8 +538,6 @@ __global__ void __launch_bounds__(256) closure_kernel(const bf16x4 *__restrict__
   if (threadIdx.x == 0) cnt = 0;
   __syncthreads();
   const int lane = threadIdx.x & 63, kb = lane >> 4, r16 = lane & 15;
-  // the weights stay in LDS: held in registers (80, half of them moved out of
-  // accumulation registers for every tile) they left two waves a SIMD
   const LdsTiles At{sw, lane};
   const long long wave = (blockIdx.x * (long long)blockDim.x + threadIdx.x) >> 6;
   const long long nwaves = (gridDim.x * (long long)blockDim.x) >> 6;

@@ -54,9 +54,11 @@ struct MomArgs {
 };
 
 // ---------------------------------------------------------------- y / z sweeps
-// Three components to a launch.  256^3 FP64: 312 (y) and 282 us (z); without
-// the solves 315 and 260, loads alone 135 and 165, stores alone 75: bound by
-// strided reads and writes in turn, 3.8 to 4.7 TB/s of the fields it moves.
+// Three components to a launch.  256^3 FP64: 292 (y) and 278 us (z), 5.1 and 3.9
+// TB/s of the fields it moves; with the fields end to end (solver.hip) 312 and
+// 282, without the solves then 315 and 260, loads alone 135 and 165, stores
+// alone 75: bound by strided reads and writes in turn.  FP32 150 and 128 us, the
+// vector ALU busy for 69 and 83 % of them.
 template <typename T, int L>
 __global__ void __launch_bounds__(1024) mom_yz_kernel(const MomArgs<T> A) {
   extern __shared__ __align__(16) unsigned char smem_raw[];

@@ -753,9 +753,9 @@ int alloc_solver(Context &c, x3d_solver *S) {
   // further than whole fields would put it: a sweep reads and writes the same
   // point of up to nine fields at once, and with fields of 2^k bytes end to end
   // these met on one channel.  256^3 step, without and with the 256 bytes: FP64
-  // 2173 and 2095 us, FP32 1187 and 1168; 128^3 299 and 292, 197 and 194 (512
-  // bytes to 3 MB apart: the same if an odd number of 256 bytes is in it, no
-  // gain from 64 KB alone).
+  // 2173 and 2095 us, FP32 1187 and 1168; 128^3 299 and 292, 197 and 194 (other
+  // distances up to 10 MB with an odd number of 256 bytes in them: within 1.5 %;
+  // whole multiples of 1 KB: no gain in FP64).
   constexpr size_t STAGGER = 256;
   struct Part {
     void **p;
