@@ -407,12 +407,13 @@ int x3d_solver_checkpoint(x3d_solver *s, const char *rundir, double t);
  * file or one whose size does not match the grid. */
 int x3d_solver_restart(x3d_solver *s, const char *rundir, double *t);
 /* Instrumentation, no counterpart in the reference: enqueue nrep times the
- * six fused y/z momentum sweeps of one step (z then y for each component,
- * on the current velocity, into the solver's work buffer; the velocity and
- * the AB3 history are not touched) on the library stream, without
- * synchronizing.  *bytes_per_launch receives the HBM bytes one launch moves
- * on average (u_d when it differs from u_c, u_c, the accumulator when
- * present, the output).  Fused solvers only. */
+ * six fused y/z momentum sweeps of one step (z, then y, the three components
+ * of each in one launch, on the current velocity, into the solver's work
+ * buffers; the velocity and the AB3 history are not touched, the kept pressure
+ * is) on the library stream, without synchronizing.  *bytes_per_launch receives
+ * the HBM bytes one component's sweep moves on average (u_d when it differs
+ * from u_c, u_c, the accumulator when present, the output).  Fused AB3 solvers
+ * of periodic boxes only. */
 int x3d_solver_momentum_yz(x3d_solver *s, int nrep, double *bytes_per_launch);
 
 /* ---- LES subgrid stress (les_models.f90) ----------------------------------
